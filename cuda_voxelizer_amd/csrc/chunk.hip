@@ -8,17 +8,16 @@
 // and, at the x that passed ZX, the plane and XY edges) and ORs the passing
 // bits into an LDS hash table keyed by table word, so bits that several
 // triangles of the chunk set in one word are merged before memory is
-// touched.  Triangles with a large voxel box (or one far larger than the
-// rest of their wave's) are queued; afterwards their owners publish test
-// records to LDS (up to kRecs per round) and the workgroup deals the rounds'
-// (row, 32-voxel x chunk) items evenly over its lanes, testing only the x
-// range that the plane band leaves open.  The table is then updated with one
-// non-returning global atomicOr per distinct word; words that do not fit in
-// the hash go straight to global atomics.  The table is zero-filled
+// touched.  Triangles with a large voxel box (or one far larger than the rest
+// of their wave's) are queued; afterwards their wave deals their rows over its
+// lanes and ORs each row's interval (rows.h).  The table is then updated with
+// one non-returning global atomicOr per distinct word; words that do not fit
+// in the hash go straight to global atomics.  The table is zero-filled
 // beforehand (unless accumulating).
 #include "jobs.h"
 #include "raster.h"
 #include "region.h"
+#include "rows.h"
 #include "vox_kernels.h"
 
 #pragma clang fp contract(off)
@@ -44,17 +43,16 @@ constexpr int kBigVox = 256;    // voxel boxes above this (or wider than 32 in x
 // the rule after one ballot.
 constexpr int kRowsFloor = 16;
 constexpr int kRowsRatio = 3;
-constexpr int kRecs = 48;       // queued triangles whose records are in LDS at once
+constexpr int kRecs = 5;        // queued triangles whose records are in LDS at once, per wave (26 KB of LDS in
+                                // all: six workgroups per CU)
 
 struct ChunkShared {
     uint32_t keys[kHashCap];
     uint32_t vals[kHashCap];
     union {
-        SurfRec recs[kRecs];      // records of the queued triangles of one round
-        RegionFlushShared flush;  // last: grouping of the region algorithm's pairs
+        WaveRows<kRecs> rows[kChunk / 64];  // each wave's queued triangles
+        RegionFlushShared flush;            // last: grouping of the region algorithm's pairs
     };
-    unsigned long long incl[kRecs];  // inclusive prefix of the round's item counts
-    unsigned wq[kChunk / 64];        // queued triangles per wave
 };
 
 // ident: the slot is the key modulo kHashCap.  Used when the whole table has
@@ -211,11 +209,11 @@ __device__ __forceinline__ void lane_raster(ChunkShared& S, uint32_t* __restrict
 }
 
 // Work unit: `span` consecutive chunks of kChunk triangles of one job, merged
-// in one LDS table and flushed once -- or, with `parts` > 1, one chunk whose
-// queued items are shared by `parts` workgroups (each does the setup, takes
-// every parts-th slice of the items, and part 0 also the lane rasters; queue
-// slots follow lane order, so every part sees the same items).  MULTI: the job
-// comes from the launch's job map; otherwise it is `one` (kernel arguments).
+// in one LDS table and flushed once -- or one chunk of it.per triangles.  With
+// `parts` > 1 the row windows of a chunk's queued triangles are shared: the
+// first units (part 0) take every parts-th window and the lane rasters, further
+// units of it.hper triangles each one part's windows.  MULTI: the job comes
+// from the launch's job map; otherwise it is `one` (kernel arguments).
 // LOOP: some job has span > 1 (otherwise the chunk loop is compiled out, which
 // keeps the register count of the one-chunk form down).  REG: the merged
 // words are staged as region pairs (RA) instead of ORed into the table.
@@ -244,22 +242,40 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE ? 6 : 5))
     const uint64_t n = info.n_triangles;
     const uint32_t parts = it.parts > 1u ? it.parts : 1u;
     const uint32_t span = (!LOOP || parts > 1u) ? 1u : (it.span > 1u ? it.span : 1u);
-    const uint32_t part = local % parts;
-    const uint64_t begin = (uint64_t)(local / parts) * span * kChunk;
+    // the first units take `per` triangles each (part 0); then, for each further
+    // part, units of `hper` triangles
+    uint32_t part = 0, per = LOOP || it.per == 0u ? (uint32_t)kChunk : it.per, unit = local;
+    if (!LOOP && parts > 1u) {
+        const uint32_t first_units = (uint32_t)((n + per - 1) / per);
+        if (unit >= first_units) {
+            per = it.hper ? it.hper : per;
+            const uint32_t nh = (uint32_t)((n + per - 1) / per);
+            part = 1u + (unit - first_units) / nh;
+            unit = (unit - first_units) % nh;
+        }
+    }
+    const uint64_t begin = (uint64_t)unit * span * per;
     if (begin >= n) return;
-    const uint64_t end = n - begin > (uint64_t)span * kChunk ? begin + (uint64_t)span * kChunk : n;
+    const uint64_t end = n - begin > (uint64_t)span * per ? begin + (uint64_t)span * per : n;
     const uint32_t G = info.gridsize[0];
     const uint64_t words = ((uint64_t)G * G * G + 31) / 32;
     const bool dense = !REG && words <= (uint64_t)kHashCap;  // region keys are not table words
     const bool ident = dense || layout == VOX_LAYOUT_MORTON;
-    for (int i = threadIdx.x; i < kHashCap; i += kChunk) {
-        S.keys[i] = dense && (uint64_t)i < words ? (uint32_t)i : kEmpty;
-        S.vals[i] = 0u;
-    }
-    __syncthreads();  // every slot is set before any lane inserts into the table
+    const int wave = (int)(threadIdx.x >> 6);
+    // a wave takes per / 4 consecutive triangles, one per lane
+    const uint32_t mine = (threadIdx.x >> 6) * (per >> 2) + (uint32_t)__lane_id();
+    const bool taken = (uint32_t)__lane_id() < (per >> 2);
+    const auto clear = [&]() {
+        for (int i = threadIdx.x; i < kHashCap; i += kChunk) {
+            S.keys[i] = dense && (uint64_t)i < words ? (uint32_t)i : kEmpty;
+            S.vals[i] = 0u;
+        }
+    };
+    if (LOOP || parts == 1u) clear();
     uint64_t first = begin;
     do {
-        const int count = (int)(end - first < (uint64_t)kChunk ? end - first : (uint64_t)kChunk);
+        const uint64_t left = end - first;
+        const bool live = taken && mine < left;
         // each lane loads its own triangle: the nine loads of a lane are in
         // flight together and a wave's 2304 bytes are contiguous, so they are
         // served by the cache after the first; staging the chunk through LDS
@@ -268,8 +284,8 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE ? 6 : 5))
         int rows = 0;  // rows of a lane-path box
         SurfTri T;
         float v[3][3];
-        if ((int)threadIdx.x < count) {
-            load_tri(it.tris, first + threadIdx.x, info, v);
+        if (live) {
+            load_tri(it.tris, first + mine, info, v);
             surface_box(v, info, T.lo, T.hi);
             const int nx = T.hi[0] - T.lo[0] + 1;
             const int ny = T.hi[1] - T.lo[1] + 1, nz = T.hi[2] - T.lo[2] + 1;
@@ -283,96 +299,35 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE ? 6 : 5))
             int sum = rows;
 #pragma unroll
             for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-            const int live = (int)__popcll(__ballot((int)threadIdx.x < count));
-            if (rows > kRowsFloor && rows * live > kRowsRatio * sum) big = true;
+            const int nlive = (int)__popcll(__ballot(live));
+            if (rows > kRowsFloor && rows * nlive > kRowsRatio * sum) big = true;
         }
-        const unsigned long long bal = __ballot(big);
-        const int wave = (int)(threadIdx.x >> 6);
-        if (__lane_id() == 0) S.wq[wave] = (unsigned)__popcll(bal);
-        if (part == 0 && (int)threadIdx.x < count && !big) {
+        if (first == begin) {
+            if (!LOOP && parts > 1u && !__syncthreads_or(big) && part) return;  // nothing to share
+            if (!LOOP && parts > 1u) clear();
+            __syncthreads();  // every slot is set before any lane inserts into the table
+        }
+        if (part == 0 && live && !big) {
             surface_setup_tests(v, info, T);  // the box is T's already
             lane_raster<REG, SPEC>(S, table, ident, T, info, layout, RA);  // nx <= 32 here
         }
-        __syncthreads();  // S.wq is complete
-        int myq = -1, nq = 0;  // this lane's queue slot (lane order), queue length
-#pragma unroll
-        for (int w = 0; w < kChunk / 64; w++) {
-            if (w == wave) myq = nq + (int)__popcll(bal & ((1ull << __lane_id()) - 1ull));
-            nq += (int)S.wq[w];
-        }
-        if (!big) myq = -1;
-        const float ux = info.unit[0], uy = info.unit[1], uz = info.unit[2];
-        for (int r0 = 0; r0 < nq; r0 += kRecs) {
-            const int nr = nq - r0 < kRecs ? nq - r0 : kRecs;
-            if (myq >= r0 && myq < r0 + nr) {
-                // the setup again, from memory (cheaper than keeping it in registers through the lane rasters)
-                float v[3][3];
-                load_tri(it.tris, first + threadIdx.x, info, v);
-                SurfTri T;
-                surface_setup(v, info, T);
-                const int xa = T.lo[0], xb = T.hi[0], ya = T.lo[1], yb = T.hi[1], za = T.lo[2], zb = T.hi[2];
-                int nk = 1, band = 0;
-                float sx = 0.0f;
-                band_chunks(T, info, xa, xb, yb, zb, nk, band, sx);
-                publish(S.recs[myq - r0], T, xa, xb, ya, yb, za, zb, nk, band, sx);
-                S.incl[myq - r0] = (xa > xb || ya > yb || za > zb)
-                                       ? 0ull
-                                       : (unsigned long long)(yb - ya + 1) * (unsigned long long)(zb - za + 1) *
-                                             (unsigned long long)nk;
+        const auto setup = [&](SurfTri& Q) {
+            // again from memory: cheaper than keeping it in registers through the lane rasters
+            float p[3][3];
+            load_tri(it.tris, first + mine, info, p);
+            surface_setup(p, info, Q);
+        };
+        wave_rows(S.rows[wave], info, big, part, parts, setup, [&](int xa, int xb, int y, int z) {
+            for (int c = xa & ~31; c <= xb; c += 32) {
+                uint32_t m = 0xFFFFFFFFu;
+                if (c < xa) m &= 0xFFFFFFFFu << (xa - c);
+                if (c + 31 > xb) m &= 0xFFFFFFFFu >> (31 - (xb - c));
+                emit_mask<REG, SPEC>(S, table, ident, info, layout, c, y, z, m, RA);
             }
-            __syncthreads();
-            if (threadIdx.x < 64) {  // inclusive scan of the round's counts (nr <= 64)
-                const int lane = (int)threadIdx.x;
-                unsigned long long c = lane < nr ? S.incl[lane] : 0ull;
-#pragma unroll
-                for (int d = 1; d < 64; d <<= 1) {
-                    const unsigned long long o = __shfl_up(c, d);
-                    if (lane >= d) c += o;
-                }
-                if (lane < nr) S.incl[lane] = c;
-            }
-            __syncthreads();
-            const unsigned long long total = S.incl[nr - 1];
-            for (unsigned long long j = threadIdx.x + (unsigned long long)part * kChunk; j < total;
-                 j += (unsigned long long)kChunk * parts) {
-                int lo = 0, hi = nr - 1;  // record: first whose inclusive prefix exceeds j
-                while (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
-                    if (S.incl[mid] > j) hi = mid; else lo = mid + 1;
-                }
-                const SurfRec& R = S.recs[lo];
-                const unsigned long long q = j - (lo ? S.incl[lo - 1] : 0ull);
-                const unsigned nk = (unsigned)R.nk, ny = (unsigned)(R.yb - R.ya + 1);
-                int k, y, z;
-                if (q < 0x100000000ull) {  // 32-bit division whenever it suffices
-                    const unsigned row = (unsigned)q / nk;
-                    k = (int)((unsigned)q - row * nk);
-                    y = R.ya + (int)(row % ny);
-                    z = R.za + (int)(row / ny);
-                } else {
-                    const unsigned long long row = q / nk;
-                    k = (int)(q - row * nk);
-                    y = R.ya + (int)(row % ny);
-                    z = R.za + (int)(row / ny);
-                }
-                const float py = (float)y * uy, pz = (float)z * uz;
-                if (!pass3(R.yz, py, pz)) continue;
-                int bx0 = R.xa, bx1 = R.xb;
-                if (R.band) {
-                    plane_band(R, ux, py, pz, bx0, bx1);
-                    if (bx0 > bx1) continue;
-                }
-                const int cx = ((bx0 >> 5) + k) << 5;
-                if (cx > bx1) continue;
-                const int x0 = cx > bx0 ? cx : bx0, x1 = (cx + 31) < bx1 ? (cx + 31) : bx1;
-                emit_mask<REG, SPEC>(S, table, ident, info, layout, cx, y, z,
-                               row_mask(R.n, R.d1, R.d2, R.xy, R.zx, ux, py, pz, x0, x1, cx), RA);
-            }
-            __syncthreads();  // the records are rewritten by the next round
-        }
-        __syncthreads();  // S.wq is read above and rewritten by the next chunk
-        first += kChunk;
+        });
+        first += per;
     } while (LOOP && first < end);
+    __syncthreads();
     // every slot read before the first atomic (one LDS wait, not one per slot)
     static_assert(kHashCap % kChunk == 0, "whole slots per thread");
     constexpr int kPer = kHashCap / kChunk;
@@ -434,9 +389,10 @@ uint32_t chunk_span(uint32_t G, uint64_t n_triangles) {
     return s < 1 ? 1u : (s > 16 ? 16u : (uint32_t)s);
 }
 
-// Workgroups per chunk.  A coarse mesh (fewer than G^2/4 triangles) has few
-// chunks of large triangles: its queued items are split over up to 32
-// workgroups per chunk, aiming at 256 workgroups per job.
+// Parts per chunk of a batch's job, whose other jobs fill the device as well
+// (a lone call: chunk_shape).  A coarse mesh (fewer than G^2/4 triangles) has few
+// chunks of large triangles: their row windows are shared by up to 32 parts,
+// aiming at 256 workgroups per job.
 uint32_t chunk_parts(uint32_t G, uint64_t n_triangles) {
     if (!coarse_mesh(n_triangles, G)) return 1u;
     const uint64_t chunks = (n_triangles + kChunk - 1) / kChunk;
@@ -444,9 +400,11 @@ uint32_t chunk_parts(uint32_t G, uint64_t n_triangles) {
     return p < 1 ? 1u : (p > 32 ? 32u : (uint32_t)p);
 }
 
-uint32_t chunk_units(uint64_t n_triangles, uint32_t span, uint32_t parts) {
-    const uint64_t chunks = (n_triangles + kChunk - 1) / kChunk;
-    if (parts > 1u) return (uint32_t)(chunks * parts);
+uint32_t chunk_units(uint64_t n_triangles, uint32_t span, uint32_t parts, uint32_t per, uint32_t hper) {
+    if (!per) per = kChunk;
+    if (!hper) hper = per;
+    const uint64_t chunks = (n_triangles + per - 1) / per;
+    if (parts > 1u) return (uint32_t)(chunks + (parts - 1u) * ((n_triangles + hper - 1) / hper));
     const uint64_t sp = span > 1u ? span : 1u;
     return (uint32_t)((chunks + sp - 1) / sp);
 }
@@ -507,8 +465,39 @@ static ItemDev single_job(const vox_info& info, const float* tris, uint32_t* tab
     one.table = table;
     one.layout = layout;
     one.span = chunk_span(info.gridsize[0], info.n_triangles);
-    one.parts = chunk_parts(info.gridsize[0], info.n_triangles);
+    one.parts = 1;
     return one;
+}
+
+// The work shape of a lone call: a mesh of few triangles must still give every
+// CU several waves, so its workgroups take fewer triangles and share their
+// queued ones with further parts.  Boxes above 16 voxels are queued where the
+// mesh is coarse (about 2.5 voxels a triangle's edge and more): the wave's
+// row windows then have less divergence than its lanes' own boxes.  Measured
+// (us per call, 256 triangles a workgroup and one part -> this rule):
+// icosphere 1,280 at 256^3 258 -> 21, 5,120 at 64^3 21.1 -> 19.3; displaced
+// sphere 20,480 at 256^3 52 -> 31; torus 26,896 at 200^3 32.4 -> 28.6; soups
+// at 256^3 5,003 194 -> 29, 30,003 174 -> 70, 100,003 146 -> 117, 200,003
+// 196 -> 189.  A torus of 59,780 at 256^3 (21.0) and a displaced sphere of
+// 327,680 at 512^3 (96.9) have nothing to share and measure the same.
+static void chunk_shape(ItemDev& one) {
+    const uint64_t n = one.info.n_triangles, G = one.info.gridsize[0];
+    const bool coarse = 8ull * n < 5ull * G * G;
+    if (one.span > 1u) return;
+    if (n <= 32768u) {
+        if (coarse) {
+            const uint64_t p = n ? (16384u + n - 1) / n : 2u;
+            one.per = one.hper = 32u;
+            one.parts = p < 2u ? 2u : (p > 16u ? 16u : (uint32_t)p);
+            if (!one.big) one.big = 16u;
+        } else {
+            one.per = one.hper = 64u;
+            one.parts = 4u;
+        }
+    } else {
+        one.per = one.hper = (uint32_t)kChunk;
+        one.parts = n <= 131072u ? 4u : (n <= 262144u ? 2u : 1u);
+    }
 }
 
 hipError_t launch_fill_zero(const vox_info& info, uint32_t* table, hipStream_t stream) {
@@ -541,7 +530,8 @@ hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_
     const ItemMap none{nullptr, nullptr, 1, 0};
     ItemDev one = single_job(info, tris, table, layout);
     one.big = big;
-    return launch_chunk_jobs(one, none, chunk_units(info.n_triangles, one.span, one.parts),
+    chunk_shape(one);
+    return launch_chunk_jobs(one, none, chunk_units(info.n_triangles, one.span, one.parts, one.per, one.hper),
                              one.span > 1u && one.parts <= 1u, stream, waves);
 }
 

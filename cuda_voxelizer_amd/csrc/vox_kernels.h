@@ -85,11 +85,8 @@ bool chunk_supported(uint32_t G);
 // coarse mesh, which spreads its columns over the whole device (1,280
 // triangles at 256^3: tile 0.09 ms vs marker 0.36 ms), the marker algorithm
 // otherwise (1,310,720 at 1024^3: marker 0.14 ms vs tile 0.41 ms).  Surface
-// default: chunk for every mesh; a coarse mesh's chunk splits its queued
-// items over up to 32 workgroups (chunk_parts), which measured faster than
-// tile from 6 to 1,310,720 triangles at 64^3 to 2048^3 (1,280 at 256^3: 0.057
-// vs 0.112 ms; a 12-triangle cube at 2048^3: 2.8 vs 8.4 ms), except for a few
-// hundred triangles at 128^3 to 512^3 (at most 1.5x slower).
+// default: chunk for every mesh (chunk.hip says how it shares the large
+// triangles of small or coarse meshes).
 inline bool coarse_mesh(uint64_t n_triangles, uint32_t G) {
     return n_triangles < (uint64_t)G * G / 4u;
 }
@@ -106,7 +103,8 @@ hipError_t launch_fill_zero(const vox_info& info, uint32_t* table, hipStream_t s
 uint32_t fill_units(uint32_t G);
 uint32_t chunk_span(uint32_t G, uint64_t n_triangles);
 uint32_t chunk_parts(uint32_t G, uint64_t n_triangles);
-uint32_t chunk_units(uint64_t n_triangles, uint32_t span, uint32_t parts);
+uint32_t chunk_units(uint64_t n_triangles, uint32_t span, uint32_t parts, uint32_t per = 0,
+                     uint32_t hper = 0);
 hipError_t launch_fill_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, hipStream_t stream);
 // What a chunk kernel instantiation knows of its jobs' layout: nothing, linear
 // with G a multiple of 32 (whole words per row), or Morton with G <= 1024
