@@ -2,8 +2,8 @@
 
 A voxelization job's best algorithm (chunk / marker / tile / direct, all
 bit-identical) depends on its grid, layout, mode and size: chunk wins on most
-surfaces, coarse ones included (it splits their large triangles over several
-workgroups), marker on fine solid meshes and tile on coarse ones, direct on
+surfaces and marker on most solids, coarse ones included (both split their
+large triangles over several workgroups), direct on
 fine solid meshes at small grids.  ``Tuner.choose`` times
 every applicable algorithm once per class (grid, layout, surface/solid, log2
 size bucket) on the job it is asked about, keeps the fastest, and remembers it

@@ -223,7 +223,7 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
         else if (algo & VOX_FLAG_ALGO_CHUNK) a = chunk_supported(G) ? CHUNK : DIRECT;
         else if (algo & VOX_FLAG_ALGO_MARKER) a = have_marker ? MARKER : (have_plan ? TILE : DIRECT);
         else if (solid && prefer_direct_solid(it.info.n_triangles, G)) a = DIRECT;
-        else if (solid && have_marker && !(have_plan && coarse_mesh(it.info.n_triangles, G))) a = MARKER;
+        else if (solid && have_marker) a = MARKER;
         else if (solid) a = have_plan ? TILE : DIRECT;
         else a = chunk_supported(G) ? CHUNK : (have_plan ? TILE : DIRECT);
         ItemDev d{};
@@ -244,8 +244,9 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
         if (a == MARKER) {
             if ((uint64_t)b->marker.total_c + n > 0xFFFFFFFFull)
                 return fail(VOX_ERR_UNSUPPORTED, "more than 2^32-1 triangles in one marker batch class");
+            const uint32_t units = marker_block_units(d);
             b->marker.items.push_back(d);
-            add_prefix(b->marker.base_a, b->marker.total_a, marker_block_units(n));
+            add_prefix(b->marker.base_a, b->marker.total_a, units);
             add_prefix(b->marker.base_b, b->marker.total_b, marker_row_units(G));
             add_prefix(b->marker.base_c, b->marker.total_c, n);  // triangles (spill overflow pass)
         } else if (a == CHUNK) {

@@ -9,8 +9,8 @@
 //   1. fill      zero the marker table: the output table itself (linear
 //                layout, no accumulate) or a linear scratch table
 //   2. markers   per triangle (one lane each; triangles with many columns
-//                are split over the workgroup): solid setup, column tests,
-//                xmax, one non-returning atomicXor per hit column
+//                have them dealt over the workgroup, columns.h): solid setup,
+//                column tests, xmax, one non-returning atomicXor per hit column
 //   3. suffix    per row (G/32 words, lanes = words): in-word prefix XOR from
 //                bit 0 up (larger x = lower bit) plus the parity of the words
 //                of larger x (a ballot).  In place for the linear layout;
@@ -26,6 +26,7 @@
 // G % 32 == 0 (rows are whole words); Morton: power-of-two G up to 4096.
 // Per-column arithmetic: vox_device.h (the reference CPU path bit for bit).
 #include "bricks.h"
+#include "columns.h"
 #include "jobs.h"
 #include "region.h"
 #include "vox_device.h"
@@ -41,9 +42,9 @@
 namespace voxamd {
 
 constexpr int kMBlock = 256;
-constexpr int kMQueue = kMBlock;   // triangles with many columns, split over the workgroup
-constexpr int kMBigCols = 32;      // columns above which a triangle is queued (the bunny at 64^3:
-                                   // 0.0325 vs 0.0349 ms at 64; the benchmark spheres unchanged)
+constexpr int kMBigCols = 32;      // columns above which a triangle's are dealt over the workgroup (the bunny at
+                                   // 64^3: 0.0325 vs 0.0349 ms at 64; the benchmark spheres unchanged)
+constexpr uint32_t kMBigColsCoarse = 8;
 constexpr uint32_t kSpillCap = 1u << 16;
 constexpr int kJobShift = 42;  // spill records: job index above the bit index (G^3 <= 2^42)
 constexpr unsigned long long kBitMask = (1ull << kJobShift) - 1ull;
@@ -116,15 +117,16 @@ __device__ __forceinline__ void column_run(uint32_t* __restrict__ table, int64_t
     }
 }
 
-// Work unit: kMBlock consecutive triangles of one job; the markers go to the
-// job's table.  MULTI: the job comes from the launch's job map (block
-// prefix); otherwise it is `one`.  REG: the markers are staged as region
-// pairs (RA) instead (phase 1 of the region algorithm).
+// Work unit: it.per (0: kMBlock) consecutive triangles of one job, or with
+// it.parts > 1 one part of their shared columns; the markers go to the job's
+// table.  MULTI: the job comes from the launch's job map (block prefix);
+// otherwise it is `one`.  REG: the markers are staged as region pairs (RA)
+// instead (phase 1 of the region algorithm).
 template <bool MULTI, bool REG>
 __global__ void __launch_bounds__(kMBlock)
     solid_marker_kernel(ItemDev one, ItemMap M, MarkerWs ws, int spills, RegionArgs RA) {
-    __shared__ unsigned queue[kMQueue];
-    __shared__ unsigned qn;
+    __shared__ ColRec recs[kColRecs];
+    __shared__ uint32_t nbig[kMBlock / 64];
     __shared__ BlockJob J;
     __shared__ MarkerLds<REG> H;
     uint32_t local = blockIdx.x;
@@ -142,79 +144,61 @@ __global__ void __launch_bounds__(kMBlock)
     unsigned long long* __restrict__ offrow_out = it.offrow;
     const unsigned long long jobtag = (unsigned long long)job << kJobShift;
     const uint64_t n = info.n_triangles;
-    const uint64_t first = (uint64_t)local * kMBlock;
-    if (first >= n) return;
-    const int count = (int)((n - first) < (uint64_t)kMBlock ? (n - first) : (uint64_t)kMBlock);
+    const uint32_t per = it.per ? it.per : (uint32_t)kMBlock, parts = it.parts > 1u ? it.parts : 1u;
+    // the parts of a unit are a grid's width apart, so part 0, which has the lanes' own columns too, comes first
+    const uint32_t units = (uint32_t)((n + per - 1) / per);
+    const uint32_t part = parts > 1u ? local / units : 0u;
+    const uint64_t first = (uint64_t)(local - part * units) * per;
+    if (first >= n || part >= parts) return;
     const int G = (int)info.gridsize[0];
     const uint64_t total_bits = (uint64_t)G * G * G;
-    if (threadIdx.x == 0) qn = 0;
     if constexpr (REG) {
         for (int i = threadIdx.x; i < kMHash; i += kMBlock) {
             H.keys[i] = kRegionEmpty;
             H.vals[i] = 0u;
         }
+        __syncthreads();  // the LDS hash is set
     }
-    __syncthreads();  // qn (and the LDS hash) set
     unsigned long long offrow = 0;
-    if ((int)threadIdx.x < count) {
+    const auto run = [&](const SolidTri& S, int y, int z, float py, float pz) {
+        column_run<REG>(table, column_xmax(S, info, py, pz), y, z, (uint32_t)G, total_bits, ws, offrow, spills != 0,
+                        jobtag, H, RA);
+    };
+    // a wave takes per / 4 consecutive triangles, one per lane
+    const uint64_t mine = first + (threadIdx.x >> 6) * (per >> 2) + (uint32_t)__lane_id();
+    SolidTri S;
+    ColBox B{0, 0, 0, 0};
+    bool big = false;
+    if ((uint32_t)__lane_id() < (per >> 2) && mine < n) {
         float v[3][3];
-        load_tri(tris, first + threadIdx.x, info, v);
-        SolidTri S;
+        load_tri(tris, mine, info, v);
         solid_setup(v, info, S);
         if (S.valid) {
-            // column range, clamped to the grid, and its out-of-grid events
-            // (as the reference loops from the unclamped bounds)
-            int ylo = (int)S.ymin, zlo = (int)S.zmin;
-            if (ylo < 0) { offrow++; ylo = 0; }
-            if (zlo < 0) { offrow++; zlo = 0; }
-            if (S.ymax > (float)(G - 1)) offrow++;
-            if (S.zmax > (float)(G - 1)) offrow++;
-            const int yhi = S.ymax >= (float)(G - 1) ? G - 1 : (S.ymax >= 0.0f ? (int)S.ymax : -1);
-            const int zhi = S.zmax >= (float)(G - 1) ? G - 1 : (S.zmax >= 0.0f ? (int)S.zmax : -1);
-            const int64_t cols = (yhi >= ylo && zhi >= zlo) ? (int64_t)(yhi - ylo + 1) * (zhi - zlo + 1) : 0;
-            bool queued = false;
-            if (cols > (it.big ? (int64_t)it.big : (int64_t)kMBigCols)) {
-                const unsigned q = atomicAdd(&qn, 1u);
-                if (q < (unsigned)kMQueue) {
-                    queue[q] = threadIdx.x;
-                    queued = true;
-                }
+            B = column_box(S, G);
+            if (part == 0) {
+                // out-of-grid events of the column range (as the reference loops from the unclamped bounds)
+                if ((int)S.ymin < 0) offrow++;
+                if ((int)S.zmin < 0) offrow++;
+                if (S.ymax > (float)(G - 1)) offrow++;
+                if (S.zmax > (float)(G - 1)) offrow++;
             }
-            if (!queued) {
-                for (int y = ylo; y <= yhi; y++) {
+            const bool any = B.ny > 0 && B.nz > 0;
+            big = any && (int64_t)B.ny * B.nz > (it.big ? (int64_t)it.big : (int64_t)kMBigCols);
+            if (any && !big && part == 0) {
+                for (int y = B.ylo; y < B.ylo + B.ny; y++) {
                     const float py = ((float)y + 0.5f) * info.unit[1];
-                    for (int z = zlo; z <= zhi; z++) {
+                    for (int z = B.zlo; z < B.zlo + B.nz; z++) {
                         const float pz = ((float)z + 0.5f) * info.unit[2];
-                        if (!column_hit(S, py, pz)) continue;
-                        column_run<REG>(table, column_xmax(S, info, py, pz), y, z, (uint32_t)G, total_bits, ws,
-                                        offrow, spills != 0, jobtag, H, RA);
+                        if (column_hit(S, py, pz)) run(S, y, z, py, pz);
                     }
                 }
             }
         }
     }
+    const unsigned long long queued = __ballot(big);
+    if (__lane_id() == 0) nbig[threadIdx.x >> 6] = (uint32_t)__popcll(queued);
     __syncthreads();
-    const unsigned nq = qn < (unsigned)kMQueue ? qn : (unsigned)kMQueue;
-    for (unsigned q = 0; q < nq; q++) {
-        const int lt = (int)queue[q];
-        float v[3][3];
-        load_tri(tris, first + (uint64_t)lt, info, v);  // the same triangle in every lane
-        SolidTri S;
-        solid_setup(v, info, S);
-        const int ylo = (int)S.ymin < 0 ? 0 : (int)S.ymin, zlo = (int)S.zmin < 0 ? 0 : (int)S.zmin;
-        const int yhi = S.ymax >= (float)(G - 1) ? G - 1 : (S.ymax >= 0.0f ? (int)S.ymax : -1);
-        const int zhi = S.zmax >= (float)(G - 1) ? G - 1 : (S.zmax >= 0.0f ? (int)S.zmax : -1);
-        const int ny = yhi - ylo + 1, nz = zhi - zlo + 1;
-        const int64_t cols = (int64_t)ny * nz;
-        for (int64_t c = threadIdx.x; c < cols; c += kMBlock) {
-            const int y = ylo + (int)(c / nz), z = zlo + (int)(c % nz);
-            const float py = ((float)y + 0.5f) * info.unit[1];
-            const float pz = ((float)z + 0.5f) * info.unit[2];
-            if (!column_hit(S, py, pz)) continue;
-            column_run<REG>(table, column_xmax(S, info, py, pz), y, z, (uint32_t)G, total_bits, ws, offrow,
-                            spills != 0, jobtag, H, RA);
-        }
-    }
+    block_columns<kMBlock / 64>(recs, nbig, S, B, big, info, part, parts, run);
     if (offrow_out && offrow) atomicAdd(offrow_out, offrow);
     if constexpr (REG) {
         __syncthreads();  // every marker of the workgroup is in the hash
@@ -659,6 +643,30 @@ bool marker_supported(uint32_t G, int layout, bool accumulate) {
     return true;
 }
 
+// How a job's triangles are split over workgroups.  A coarse mesh (fewer than
+// G^2/4 triangles) has few workgroups of 256 and triangles of many columns, so
+// its units take 32, deal boxes of more than 8 columns (kMBigCols) and share
+// them with further parts, up to about 1024 workgroups.  Measured (us per
+// call; the triangles one after the other over a workgroup of 256 -> this):
+// icosphere 1,280 at 256^3 360 -> 19, 5,120 at 256^3 300 -> 19, 20,480 at
+// 576^3 349 -> 62; displaced sphere 20,480 at 512^3 277 -> 33, 81,920 at
+// 1024^3 346 -> 124 (the row pass takes 58 of it).  From G^2/4 on a limit of 8
+// loses: displaced sphere 20,480 at 256^3 20 with 32 columns, 26 with 8.
+static void marker_shape(ItemDev& it) {
+    const uint64_t n = it.info.n_triangles;
+    if (!coarse_mesh(n, it.info.gridsize[0]) || n == 0) return;
+    if (!it.big) it.big = kMBigColsCoarse;
+    it.per = n <= 65536u ? 32u : (uint32_t)kMBlock;
+    const uint64_t units = (n + it.per - 1) / it.per;
+    const uint64_t p = 1024u / units;
+    it.parts = p < 1u ? 1u : (p > 256u ? 256u : (uint32_t)p);
+}
+
+static uint32_t marker_units(const ItemDev& it) {
+    const uint64_t per = it.per ? it.per : (uint64_t)kMBlock;
+    return (uint32_t)((it.info.n_triangles + per - 1) / per) * (it.parts > 1u ? it.parts : 1u);
+}
+
 hipError_t launch_marker_in_place(const vox_info& info, const float* tris, uint32_t* table,
                                   unsigned long long* offrow, const MarkerWs& ws, hipStream_t stream, uint32_t big);
 
@@ -731,11 +739,10 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     one.solid = 1;
     ItemDev fin = one;  // spills: into the final table
     fin.table = table;
-    if (info.n_triangles) {
-        const uint64_t blocks = (info.n_triangles + kMBlock - 1) / kMBlock;
-        solid_marker_kernel<false, false><<<(unsigned)blocks, kMBlock, 0, stream>>>(one, none, ws, linear ? 1 : 0,
+    marker_shape(one);
+    if (info.n_triangles)
+        solid_marker_kernel<false, false><<<marker_units(one), kMBlock, 0, stream>>>(one, none, ws, linear ? 1 : 0,
                                                                                     RegionArgs{});
-    }
     if (stream_rows) {
         const uint64_t nrows = (uint64_t)G * G;
         const uint64_t per = 64 / (G >> 7);
@@ -827,10 +834,9 @@ hipError_t launch_marker_in_place(const vox_info& info, const float* tris, uint3
     one.offrow = offrow;
     one.layout = VOX_LAYOUT_LINEAR;
     one.solid = 1;
-    if (info.n_triangles) {
-        const uint64_t blocks = (info.n_triangles + kMBlock - 1) / kMBlock;
-        solid_marker_kernel<false, false><<<(unsigned)blocks, kMBlock, 0, stream>>>(one, none, ws, 1, RegionArgs{});
-    }
+    marker_shape(one);
+    if (info.n_triangles)
+        solid_marker_kernel<false, false><<<marker_units(one), kMBlock, 0, stream>>>(one, none, ws, 1, RegionArgs{});
     if (rows4_ok(G, table)) {
         const uint64_t nrows = (uint64_t)G * G;
         const uint64_t per = 64 / (G >> 7);
@@ -902,7 +908,10 @@ hipError_t launch_solid_marker_static(const vox_info& info, const float* tris, u
 
 // ---- batched form (linear layout, no accumulation: in place) -------------------
 uint64_t marker_ws_bytes() { return 256 + 16ull * kSpillCap; }
-uint32_t marker_block_units(uint64_t n_triangles) { return (uint32_t)((n_triangles + kMBlock - 1) / kMBlock); }
+uint32_t marker_block_units(ItemDev& it) {
+    marker_shape(it);
+    return marker_units(it);
+}
 uint32_t marker_row_units(uint32_t G) { return (uint32_t)(((uint64_t)G * G + kSuffixRows - 1) / kSuffixRows); }
 bool marker_batch_supported(uint32_t G, int layout, bool accumulate) {
     return layout == VOX_LAYOUT_LINEAR && !accumulate && marker_supported(G, layout, accumulate);

@@ -32,7 +32,7 @@ bool marker_batch_supported(uint32_t G, int layout, bool accumulate);
 bool layout_convert_fast(uint32_t G);
 hipError_t launch_layout_convert(const uint32_t* src, uint32_t* dst, uint32_t G, bool to_morton, hipStream_t stream);
 uint64_t marker_ws_bytes();
-uint32_t marker_block_units(uint64_t n_triangles);
+uint32_t marker_block_units(ItemDev& it);  // sets the job's work shape
 uint32_t marker_row_units(uint32_t G);
 hipError_t launch_marker_jobs(const ItemMap& m_blocks, const ItemMap& m_rows, const ItemMap& m_tris,
                               uint32_t blocks, uint32_t row_units, void* mws, hipStream_t stream);
@@ -81,12 +81,9 @@ inline RegionKnobs region_knobs(unsigned flags) {
 
 bool chunk_supported(uint32_t G);
 // A coarse mesh has few triangles for its grid, so each covers a large voxel
-// box and many columns.  Solid default: the output-tiled algorithm for a
-// coarse mesh, which spreads its columns over the whole device (1,280
-// triangles at 256^3: tile 0.09 ms vs marker 0.36 ms), the marker algorithm
-// otherwise (1,310,720 at 1024^3: marker 0.14 ms vs tile 0.41 ms).  Surface
-// default: chunk for every mesh (chunk.hip says how it shares the large
-// triangles of small or coarse meshes).
+// box and many columns.  The defaults are chunk for surfaces and marker for
+// solids at every size; both give a coarse mesh smaller workgroups that share
+// its large triangles (chunk.hip, marker.hip: marker_shape).
 inline bool coarse_mesh(uint64_t n_triangles, uint32_t G) {
     return n_triangles < (uint64_t)G * G / 4u;
 }
