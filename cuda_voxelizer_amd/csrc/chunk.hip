@@ -9,8 +9,8 @@
 // bits into an LDS hash table keyed by table word, so bits that several
 // triangles of the chunk set in one word are merged before memory is
 // touched.  Triangles with a large voxel box (or one far larger than the rest
-// of their wave's) are queued; afterwards their wave deals their rows over its
-// lanes and ORs each row's interval (rows.h).  The table is then updated with
+// of their wave's) are queued; afterwards the workgroup deals their rows over
+// its lanes and ORs each row's interval (rows.h).  The table is then updated with
 // one non-returning global atomicOr per distinct word; words that do not fit
 // in the hash go straight to global atomics.  The table is zero-filled
 // beforehand (unless accumulating).
@@ -43,15 +43,16 @@ constexpr int kBigVox = 256;    // voxel boxes above this (or wider than 32 in x
 // the rule after one ballot.
 constexpr int kRowsFloor = 16;
 constexpr int kRowsRatio = 3;
-constexpr int kRecs = 5;        // queued triangles whose records are in LDS at once, per wave (26 KB of LDS in
-                                // all: six workgroups per CU)
+constexpr int kRecs = 20;       // queued triangles whose records are in LDS at once (26 KB of LDS in all: six
+                                // workgroups per CU)
 
 struct ChunkShared {
     uint32_t keys[kHashCap];
     uint32_t vals[kHashCap];
+    uint32_t nbig[2][kChunk / 64];  // queued triangles per wave, of an even and an odd chunk
     union {
-        WaveRows<kRecs> rows[kChunk / 64];  // each wave's queued triangles
-        RegionFlushShared flush;            // last: grouping of the region algorithm's pairs
+        BlockRows<kRecs, kChunk / 64> rows;  // queued triangles
+        RegionFlushShared flush;             // last: grouping of the region algorithm's pairs
     };
 };
 
@@ -133,10 +134,11 @@ __device__ __forceinline__ void emit_mask(ChunkShared& S, uint32_t* __restrict__
 // a row then tests the XY edges and the plane only at the x that passed ZX.
 // Every test is the same binary32 expression as in vox_device.h, evaluated
 // for a subset of the voxels: the resulting bits are unchanged.
-template <bool REG, int SPEC>
+// SPLIT: 2^lg lanes share the box; lane `sub` of them takes every 2^lg-th row.
+template <bool REG, int SPEC, bool SPLIT>
 __device__ __forceinline__ void lane_raster(ChunkShared& S, uint32_t* __restrict__ table, bool ident,
                                             const SurfTri& T, const vox_info& info, int layout,
-                                            const RegionArgs& RA) {
+                                            const RegionArgs& RA, int sub, int lg) {
     const float ux = info.unit[0], uy = info.unit[1], uz = info.unit[2];
     const int xa = T.lo[0], xb = T.hi[0];
     const int c0 = xa & ~31, sh = xa - c0;
@@ -146,7 +148,15 @@ __device__ __forceinline__ void lane_raster(ChunkShared& S, uint32_t* __restrict
                      (SPEC == kSpecAny && layout == VOX_LAYOUT_MORTON && info.gridsize[0] <= 1024u);
     const uint32_t sc0 = m32 ? spread10((uint32_t)c0) : 0u, sc1 = m32 ? spread10((uint32_t)c0 + 32u) : 0u;
     const auto put = [&](uint64_t w, uint32_t bits) { word_or<REG>(S, table, ident, (uint32_t)w, bits, RA); };
+    const int step = SPLIT ? 1 << lg : 1;
+    int ynext = T.lo[1] + (SPLIT ? sub : 0);  // the lane's next row in y
     for (int z = T.lo[2]; z <= T.hi[2]; z++) {
+        if (SPLIT && ynext > T.hi[1]) {  // no row of this slice is the lane's
+            ynext -= T.hi[1] - T.lo[1] + 1;
+            continue;
+        }
+        const int ybeg = ynext;
+        if (SPLIT) ynext += ((T.hi[1] - ybeg) >> lg) * step + step - (T.hi[1] - T.lo[1] + 1);
         const float pz = (float)z * uz;
         float azx[3];
 #pragma unroll
@@ -166,7 +176,7 @@ __device__ __forceinline__ void lane_raster(ChunkShared& S, uint32_t* __restrict
         }
         if (!zxm) continue;
         const float nzpz = T.n[2] * pz;
-        for (int y = T.lo[1]; y <= T.hi[1]; y++) {
+        for (int y = SPLIT ? ybeg : T.lo[1]; y <= T.hi[1]; y += step) {
             const float py = (float)y * uy;
             if (!edges_pass(T.yz, py, pz)) continue;
             const float nypy = T.n[1] * py;
@@ -209,22 +219,22 @@ __device__ __forceinline__ void lane_raster(ChunkShared& S, uint32_t* __restrict
 }
 
 // Work unit: `span` consecutive chunks of kChunk triangles of one job, merged
-// in one LDS table and flushed once -- or one chunk of it.per triangles.  With
-// `parts` > 1 the row windows of a chunk's queued triangles are shared: the
-// first units (part 0) take every parts-th window and the lane rasters, further
-// units of it.hper triangles each one part's windows.  MULTI: the job comes
-// from the launch's job map; otherwise it is `one` (kernel arguments).
+// in one LDS table and flushed once -- or one chunk of it.per triangles, each
+// shared by 2^it.lg_split lanes (SPLIT).  With `parts` > 1 the row windows of
+// a chunk's queued triangles are shared: the first units (part 0) take every
+// parts-th window and the lane rasters, further units one part's windows each.
+// MULTI: the job comes from the launch's job map; otherwise it is `one` (kernel
+// arguments).
 // LOOP: some job has span > 1 (otherwise the chunk loop is compiled out, which
 // keeps the register count of the one-chunk form down).  REG: the merged
 // words are staged as region pairs (RA) instead of ORed into the table.
 // Workgroups per CU: the LDS allows six.  The bound holds the registers at
-// five waves per SIMD, or six with WIDE (a few spilled registers: it pays for
-// the linear layout, whose chunks touch more words and so wait longer on the
-// LDS table, not for the Morton layout), or four for the chunk loop.  SPEC:
+// five waves per SIMD, or six with WIDE and in a single job's specialised form
+// (no spills there), or four for the chunk loop.  SPEC:
 // the layout when it is known at compile time, so the other layout's word
 // paths are compiled out (at six waves this removes the spills).
-template <bool MULTI, bool LOOP, bool WIDE, bool REG, int SPEC = kSpecAny>
-__global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE ? 6 : 5))
+template <bool MULTI, bool LOOP, bool WIDE, bool REG, int SPEC = kSpecAny, bool SPLIT = false>
+__global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE || (SPEC != kSpecAny && !MULTI) ? 6 : 5))
     surface_chunk_kernel(ItemDev one, ItemMap M, RegionArgs RA) {
     __shared__ ChunkShared S;
     __shared__ BlockJob J;
@@ -242,17 +252,14 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE ? 6 : 5))
     const uint64_t n = info.n_triangles;
     const uint32_t parts = it.parts > 1u ? it.parts : 1u;
     const uint32_t span = (!LOOP || parts > 1u) ? 1u : (it.span > 1u ? it.span : 1u);
-    // the first units take `per` triangles each (part 0); then, for each further
-    // part, units of `hper` triangles
-    uint32_t part = 0, per = LOOP || it.per == 0u ? (uint32_t)kChunk : it.per, unit = local;
+    // lg: each triangle is shared by 2^lg lanes of a wave
+    const int lg = SPLIT ? (int)it.lg_split : 0;
+    const uint32_t per = (uint32_t)kChunk >> lg;
+    uint32_t part = 0, unit = local;
     if (!LOOP && parts > 1u) {
-        const uint32_t first_units = (uint32_t)((n + per - 1) / per);
-        if (unit >= first_units) {
-            per = it.hper ? it.hper : per;
-            const uint32_t nh = (uint32_t)((n + per - 1) / per);
-            part = 1u + (unit - first_units) / nh;
-            unit = (unit - first_units) % nh;
-        }
+        const uint32_t units = (uint32_t)((n + per - 1) / per);
+        part = unit / units;
+        unit -= part * units;
     }
     const uint64_t begin = (uint64_t)unit * span * per;
     if (begin >= n) return;
@@ -262,9 +269,8 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE ? 6 : 5))
     const bool dense = !REG && words <= (uint64_t)kHashCap;  // region keys are not table words
     const bool ident = dense || layout == VOX_LAYOUT_MORTON;
     const int wave = (int)(threadIdx.x >> 6);
-    // a wave takes per / 4 consecutive triangles, one per lane
-    const uint32_t mine = (threadIdx.x >> 6) * (per >> 2) + (uint32_t)__lane_id();
-    const bool taken = (uint32_t)__lane_id() < (per >> 2);
+    const uint32_t mine = threadIdx.x >> lg;  // the lane's triangle in the chunk
+    const int sub = (int)(threadIdx.x & ((1u << lg) - 1u));
     const auto clear = [&]() {
         for (int i = threadIdx.x; i < kHashCap; i += kChunk) {
             S.keys[i] = dense && (uint64_t)i < words ? (uint32_t)i : kEmpty;
@@ -273,9 +279,10 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE ? 6 : 5))
     };
     if (LOOP || parts == 1u) clear();
     uint64_t first = begin;
+    int odd = 0;
     do {
         const uint64_t left = end - first;
-        const bool live = taken && mine < left;
+        const bool live = mine < left;
         // each lane loads its own triangle: the nine loads of a lane are in
         // flight together and a wave's 2304 bytes are contiguous, so they are
         // served by the cache after the first; staging the chunk through LDS
@@ -291,7 +298,8 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE ? 6 : 5))
             const int ny = T.hi[1] - T.lo[1] + 1, nz = T.hi[2] - T.lo[2] + 1;
             const int64_t vol = (int64_t)nx * ny * nz;
             big = vol > (it.big ? (int64_t)it.big : (int64_t)kBigVox) || nx > 32;
-            rows = big ? 0 : ny * nz;  // at most the queue threshold here (<= 2^15): no overflow
+            // the lane's rows; at most the queue threshold here (<= 2^15): no overflow
+            rows = big ? 0 : (ny * nz + (1 << lg) - 1) >> lg;
         }
         if (!it.big && __ballot(rows > kRowsFloor)) {
             // sum over the wave (dead and queued lanes add 0); the mean is
@@ -305,19 +313,21 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE ? 6 : 5))
         if (first == begin) {
             if (!LOOP && parts > 1u && !__syncthreads_or(big) && part) return;  // nothing to share
             if (!LOOP && parts > 1u) clear();
-            __syncthreads();  // every slot is set before any lane inserts into the table
         }
+        const bool queue = big && (!SPLIT || sub == 0);  // once, whatever lanes share it
+        const unsigned long long queued = __ballot(queue);
+        if (__lane_id() == 0) S.nbig[odd][wave] = (uint32_t)__popcll(queued);
+        __syncthreads();  // every slot is set before any lane inserts into the table; the counts are there
         if (part == 0 && live && !big) {
             surface_setup_tests(v, info, T);  // the box is T's already
-            lane_raster<REG, SPEC>(S, table, ident, T, info, layout, RA);  // nx <= 32 here
+            lane_raster<REG, SPEC, SPLIT>(S, table, ident, T, info, layout, RA, sub, lg);  // nx <= 32 here
         }
-        const auto setup = [&](SurfTri& Q) {
-            // again from memory: cheaper than keeping it in registers through the lane rasters
+        const auto setup = [&](uint32_t thread, SurfTri& Q) {
             float p[3][3];
-            load_tri(it.tris, first + mine, info, p);
+            load_tri(it.tris, first + (thread >> lg), info, p);
             surface_setup(p, info, Q);
         };
-        wave_rows(S.rows[wave], info, big, part, parts, setup, [&](int xa, int xb, int y, int z) {
+        block_rows(S.rows, S.nbig[odd], info, queue, part, parts, setup, [&](int xa, int xb, int y, int z) {
             for (int c = xa & ~31; c <= xb; c += 32) {
                 uint32_t m = 0xFFFFFFFFu;
                 if (c < xa) m &= 0xFFFFFFFFu << (xa - c);
@@ -326,6 +336,7 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE ? 6 : 5))
             }
         });
         first += per;
+        odd ^= 1;
     } while (LOOP && first < end);
     __syncthreads();
     // every slot read before the first atomic (one LDS wait, not one per slot)
@@ -400,11 +411,10 @@ uint32_t chunk_parts(uint32_t G, uint64_t n_triangles) {
     return p < 1 ? 1u : (p > 32 ? 32u : (uint32_t)p);
 }
 
-uint32_t chunk_units(uint64_t n_triangles, uint32_t span, uint32_t parts, uint32_t per, uint32_t hper) {
-    if (!per) per = kChunk;
-    if (!hper) hper = per;
+uint32_t chunk_units(uint64_t n_triangles, uint32_t span, uint32_t parts, uint32_t lg_split) {
+    const uint64_t per = (uint32_t)kChunk >> lg_split;
     const uint64_t chunks = (n_triangles + per - 1) / per;
-    if (parts > 1u) return (uint32_t)(chunks + (parts - 1u) * ((n_triangles + hper - 1) / hper));
+    if (parts > 1u) return (uint32_t)(chunks * parts);
     const uint64_t sp = span > 1u ? span : 1u;
     return (uint32_t)((chunks + sp - 1) / sp);
 }
@@ -421,15 +431,15 @@ int chunk_spec(int layout, uint32_t G) {
     return kSpecAny;
 }
 
-template <bool MULTI, bool WIDE>
+template <bool MULTI, bool WIDE, bool SPLIT = false>
 static void launch_chunk_spec(int spec, uint32_t units, hipStream_t stream, const ItemDev& one, const ItemMap& M) {
     const RegionArgs none{};
     if (spec == kSpecLinear)
-        surface_chunk_kernel<MULTI, false, WIDE, false, kSpecLinear><<<units, kChunk, 0, stream>>>(one, M, none);
+        surface_chunk_kernel<MULTI, false, WIDE, false, kSpecLinear, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
     else if (spec == kSpecMorton)
-        surface_chunk_kernel<MULTI, false, WIDE, false, kSpecMorton><<<units, kChunk, 0, stream>>>(one, M, none);
+        surface_chunk_kernel<MULTI, false, WIDE, false, kSpecMorton, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
     else
-        surface_chunk_kernel<MULTI, false, WIDE, false, kSpecAny><<<units, kChunk, 0, stream>>>(one, M, none);
+        surface_chunk_kernel<MULTI, false, WIDE, false, kSpecAny, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
 }
 
 // waves: 5 or 6 waves per SIMD for the one-chunk form (0: 6 for the linear
@@ -451,6 +461,8 @@ hipError_t launch_chunk_jobs(const ItemDev& one, const ItemMap& M, uint32_t unit
         launch_chunk_spec<true, true>(spec, units, stream, one, M);
     else if (M.items)
         launch_chunk_spec<true, false>(spec, units, stream, one, M);
+    else if (one.lg_split)
+        launch_chunk_spec<false, false, true>(spec, units, stream, one, M);
     else if (wide)
         launch_chunk_spec<false, true>(spec, units, stream, one, M);
     else
@@ -469,34 +481,37 @@ static ItemDev single_job(const vox_info& info, const float* tris, uint32_t* tab
     return one;
 }
 
-// The work shape of a lone call: a mesh of few triangles must still give every
-// CU several waves, so its workgroups take fewer triangles and share their
-// queued ones with further parts.  Boxes above 16 voxels are queued where the
-// mesh is coarse (about 2.5 voxels a triangle's edge and more): the wave's
-// row windows then have less divergence than its lanes' own boxes.  Measured
-// (us per call, 256 triangles a workgroup and one part -> this rule):
-// icosphere 1,280 at 256^3 258 -> 21, 5,120 at 64^3 21.1 -> 19.3; displaced
-// sphere 20,480 at 256^3 52 -> 31; torus 26,896 at 200^3 32.4 -> 28.6; soups
-// at 256^3 5,003 194 -> 29, 30,003 174 -> 70, 100,003 146 -> 117, 200,003
-// 196 -> 189.  A torus of 59,780 at 256^3 (21.0) and a displaced sphere of
-// 327,680 at 512^3 (96.9) have nothing to share and measure the same.
+// The work shape of a lone call.  A mesh of few triangles must still give every
+// CU several waves, so its triangles are shared by up to 16 lanes each, as long
+// as the call has at most 1280 workgroups (five per CU) by that; more lanes
+// only repeat the setup, and Morton chunks of under 32 triangles merge too few
+// of their words.  A coarse mesh (about 2.5 voxels a triangle's edge and more)
+// queues smaller boxes and shares its few workgroups' queued rows with further
+// parts, the more the coarser it is.  A finer one of up to 262,144 triangles
+// takes two parts, for the large triangles that it may have among them.
+// Measured (us per call, 256 triangles a workgroup and one part -> this rule; a
+// loop of calls does not go below about 15): icosphere 5,120 at 64^3 21.7 ->
+// 15, 1,280 at 256^3 277 -> 18; torus 26,896 at 200^3 32.7 -> 17, 5,000 at
+// 128^3 76 -> 16; displaced sphere 20,480 at 256^3 90 -> 25, 81,920 at 256^3
+// 39 -> 34; slivers of 150,000 at 512^3 Morton 39 -> 33; soups at 256^3 2,003
+// 119 -> 20, 20,003 114 -> 40, 100,003 123 -> 90.
 static void chunk_shape(ItemDev& one) {
     const uint64_t n = one.info.n_triangles, G = one.info.gridsize[0];
-    const bool coarse = 8ull * n < 5ull * G * G;
-    if (one.span > 1u) return;
-    if (n <= 32768u) {
-        if (coarse) {
-            const uint64_t p = n ? (16384u + n - 1) / n : 2u;
-            one.per = one.hper = 32u;
-            one.parts = p < 2u ? 2u : (p > 16u ? 16u : (uint32_t)p);
-            if (!one.big) one.big = 16u;
-        } else {
-            one.per = one.hper = 64u;
-            one.parts = 4u;
-        }
+    if (one.span > 1u || n == 0) return;
+    const uint32_t top = one.layout == VOX_LAYOUT_MORTON ? 3u : 4u;
+    one.lg_split = 0;
+    while (one.lg_split < top && n << (one.lg_split + 1u) <= 327680u) one.lg_split++;
+    if (8ull * n < 5ull * G * G) {
+        const uint64_t units = ((n << one.lg_split) + kChunk - 1) / kChunk;
+        uint64_t p = 2048u / units;
+        if (p > G * G / (2u * n)) p = G * G / (2u * n);
+        one.parts = p < 1u ? 1u : (p > 16u ? 16u : (uint32_t)p);
+        if (!one.big && n <= 32768u)
+            one.big = 16u;
+        else if (!one.big && 8u * n < G * G)
+            one.big = 64u;  // 81,920 at 1024^3: 165 us at 256 voxels, 150 at 64; at 512^3 66 and 80
     } else {
-        one.per = one.hper = (uint32_t)kChunk;
-        one.parts = n <= 131072u ? 4u : (n <= 262144u ? 2u : 1u);
+        one.parts = one.lg_split <= 1u && n <= 262144u ? 2u : 1u;
     }
 }
 
@@ -531,7 +546,7 @@ hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_
     ItemDev one = single_job(info, tris, table, layout);
     one.big = big;
     chunk_shape(one);
-    return launch_chunk_jobs(one, none, chunk_units(info.n_triangles, one.span, one.parts, one.per, one.hper),
+    return launch_chunk_jobs(one, none, chunk_units(info.n_triangles, one.span, one.parts, one.lg_split),
                              one.span > 1u && one.parts <= 1u, stream, waves);
 }
 

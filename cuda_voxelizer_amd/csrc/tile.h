@@ -46,8 +46,8 @@ struct ItemDev {
     uint32_t parts;      // chunk algorithm: workgroups per chunk (0 or 1: one)
     uint32_t big;        // chunk: voxel boxes above this are shared by the workgroup; marker: columns
                          // above this (0: the built-in threshold)
-    uint32_t per;        // chunk algorithm: triangles per workgroup (0: 256)
-    uint32_t hper;       // chunk algorithm: and per workgroup of the parts after the first (0: as per)
+    uint32_t per;        // marker algorithm: triangles per workgroup (0: 256)
+    uint32_t lg_split;   // chunk algorithm: 2^lg_split lanes share a triangle, so a workgroup takes 256 >> lg_split
     uint32_t pad2;
 };
 

@@ -66,3 +66,13 @@ def test_chunk_shapes(oracle, gpu, n):
     for grid in (64, 224):
         got, exp = _surface(oracle, gpu, tris, grid)
         assert (got == exp).all(), grid
+
+
+@pytest.mark.parametrize("n", [7, 20480, 20481, 40961, 81921, 163841])
+@pytest.mark.parametrize("grid,morton", [(64, True), (100, False), (160, False)])
+def test_shared_lanes(oracle, gpu, n, grid, morton):
+    """Boxes of one to some hundred rows, shared by one to sixteen lanes."""
+    from cuda_voxelizer_amd import meshgen
+    tris = meshgen.triangle_soup(n, seed=n + grid, mu=-4.0, sigma=0.7)
+    got, exp = _surface(oracle, gpu, tris, grid, morton)
+    assert (got == exp).all()
