@@ -117,9 +117,9 @@ __device__ __forceinline__ void column_run(uint32_t* __restrict__ table, int64_t
     }
 }
 
-// Work unit: it.per (0: kMBlock) consecutive triangles of one job, or with
-// it.parts > 1 one part of their shared columns; the markers go to the job's
-// table.  MULTI: the job comes from the launch's job map (block prefix);
+// Work unit: kMBlock >> it.lg_split consecutive triangles of one job, each
+// shared by 2^it.lg_split lanes, or with it.parts > 1 one part of their dealt
+// columns; the markers go to the job's table.  MULTI: the job comes from the launch's job map (block prefix);
 // otherwise it is `one`.  REG: the markers are staged as region pairs (RA)
 // instead (phase 1 of the region algorithm).
 template <bool MULTI, bool REG>
@@ -144,7 +144,8 @@ __global__ void __launch_bounds__(kMBlock)
     unsigned long long* __restrict__ offrow_out = it.offrow;
     const unsigned long long jobtag = (unsigned long long)job << kJobShift;
     const uint64_t n = info.n_triangles;
-    const uint32_t per = it.per ? it.per : (uint32_t)kMBlock, parts = it.parts > 1u ? it.parts : 1u;
+    const int lg = (int)it.lg_split;
+    const uint32_t per = (uint32_t)kMBlock >> lg, parts = it.parts > 1u ? it.parts : 1u;
     // the parts of a unit are a grid's width apart, so part 0, which has the lanes' own columns too, comes first
     const uint32_t units = (uint32_t)((n + per - 1) / per);
     const uint32_t part = parts > 1u ? local / units : 0u;
@@ -164,18 +165,18 @@ __global__ void __launch_bounds__(kMBlock)
         column_run<REG>(table, column_xmax(S, info, py, pz), y, z, (uint32_t)G, total_bits, ws, offrow, spills != 0,
                         jobtag, H, RA);
     };
-    // a wave takes per / 4 consecutive triangles, one per lane
-    const uint64_t mine = first + (threadIdx.x >> 6) * (per >> 2) + (uint32_t)__lane_id();
+    const uint64_t mine = first + (threadIdx.x >> lg);
+    const int sub = (int)(threadIdx.x & ((1u << lg) - 1u)), step = 1 << lg;
     SolidTri S;
     ColBox B{0, 0, 0, 0};
     bool big = false;
-    if ((uint32_t)__lane_id() < (per >> 2) && mine < n) {
+    if (mine < n) {
         float v[3][3];
         load_tri(tris, mine, info, v);
         solid_setup(v, info, S);
         if (S.valid) {
             B = column_box(S, G);
-            if (part == 0) {
+            if (part == 0 && sub == 0) {
                 // out-of-grid events of the column range (as the reference loops from the unclamped bounds)
                 if ((int)S.ymin < 0) offrow++;
                 if ((int)S.zmin < 0) offrow++;
@@ -185,14 +186,18 @@ __global__ void __launch_bounds__(kMBlock)
             const bool any = B.ny > 0 && B.nz > 0;
             big = any && (int64_t)B.ny * B.nz > (it.big ? (int64_t)it.big : (int64_t)kMBigCols);
             if (any && !big && part == 0) {
+                int znext = sub;  // the lane's next column in z: every 2^lg-th of the box
                 for (int y = B.ylo; y < B.ylo + B.ny; y++) {
                     const float py = ((float)y + 0.5f) * info.unit[1];
-                    for (int z = B.zlo; z < B.zlo + B.nz; z++) {
+                    for (; znext < B.nz; znext += step) {
+                        const int z = B.zlo + znext;
                         const float pz = ((float)z + 0.5f) * info.unit[2];
                         if (column_hit(S, py, pz)) run(S, y, z, py, pz);
                     }
+                    znext -= B.nz;
                 }
             }
+            big = big && sub == 0;  // queued once, whatever lanes share it
         }
     }
     const unsigned long long queued = __ballot(big);
@@ -643,27 +648,29 @@ bool marker_supported(uint32_t G, int layout, bool accumulate) {
     return true;
 }
 
-// How a job's triangles are split over workgroups.  A coarse mesh (fewer than
-// G^2/4 triangles) has few workgroups of 256 and triangles of many columns, so
-// its units take 32, deal boxes of more than 8 columns (kMBigCols) and share
-// them with further parts, up to about 1024 workgroups.  Measured (us per
-// call; the triangles one after the other over a workgroup of 256 -> this):
-// icosphere 1,280 at 256^3 360 -> 19, 5,120 at 256^3 300 -> 19, 20,480 at
+// How a job's triangles are split over workgroups.  Those of a small mesh are
+// shared by up to 16 lanes each, as long as the job has at most 1280 workgroups
+// by that.  A coarse mesh (fewer than G^2/4 triangles) has triangles of many
+// columns: boxes of more than 8 (kMBigCols) are dealt, and further parts take
+// their share of them, up to about 1024 workgroups.  Measured (us per call;
+// the triangles one after the other over a workgroup of 256 -> this):
+// icosphere 1,280 at 256^3 360 -> 17, 5,120 at 256^3 300 -> 18, 20,480 at
 // 576^3 349 -> 62; displaced sphere 20,480 at 512^3 277 -> 33, 81,920 at
 // 1024^3 346 -> 124 (the row pass takes 58 of it).  From G^2/4 on a limit of 8
 // loses: displaced sphere 20,480 at 256^3 20 with 32 columns, 26 with 8.
 static void marker_shape(ItemDev& it) {
     const uint64_t n = it.info.n_triangles;
-    if (!coarse_mesh(n, it.info.gridsize[0]) || n == 0) return;
+    if (n == 0) return;
+    while (it.lg_split < 4u && n << (it.lg_split + 1u) <= 327680u) it.lg_split++;
+    if (!coarse_mesh(n, it.info.gridsize[0])) return;
     if (!it.big) it.big = kMBigColsCoarse;
-    it.per = n <= 65536u ? 32u : (uint32_t)kMBlock;
-    const uint64_t units = (n + it.per - 1) / it.per;
+    const uint64_t units = ((n << it.lg_split) + kMBlock - 1) / kMBlock;
     const uint64_t p = 1024u / units;
     it.parts = p < 1u ? 1u : (p > 256u ? 256u : (uint32_t)p);
 }
 
 static uint32_t marker_units(const ItemDev& it) {
-    const uint64_t per = it.per ? it.per : (uint64_t)kMBlock;
+    const uint64_t per = (uint64_t)kMBlock >> it.lg_split;
     return (uint32_t)((it.info.n_triangles + per - 1) / per) * (it.parts > 1u ? it.parts : 1u);
 }
 

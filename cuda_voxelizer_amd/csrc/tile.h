@@ -43,11 +43,10 @@ struct ItemDev {
     uint32_t tile_base;  // first global tile id of this job (tile algorithm)
     uint64_t tri_base;   // first global triangle id of this job
     uint32_t span;       // chunk algorithm: chunks per workgroup (0 or 1: one)
-    uint32_t parts;      // chunk algorithm: workgroups per chunk (0 or 1: one)
+    uint32_t parts;      // chunk, marker: workgroups that share a unit's large triangles (0 or 1: one)
     uint32_t big;        // chunk: voxel boxes above this are shared by the workgroup; marker: columns
                          // above this (0: the built-in threshold)
-    uint32_t per;        // marker algorithm: triangles per workgroup (0: 256)
-    uint32_t lg_split;   // chunk algorithm: 2^lg_split lanes share a triangle, so a workgroup takes 256 >> lg_split
+    uint32_t lg_split;   // chunk, marker: 2^lg_split lanes share a triangle, so a workgroup takes 256 >> lg_split
     uint32_t pad2;
 };
 
