@@ -219,6 +219,29 @@ def _info_checked(info: VoxInfo, tris, table, grid_words_needed=True):
             raise ValueError(f"vtable holds {table.numel()} words, need {table_words(info.grid)}")
 
 
+def _plain_call(info: VoxInfo, tris, table, stream):
+    """(table, stream pointer) of a call on the current stream with plain, valid
+    tensors; None for every other call, which takes the general path below and
+    is refused there if it must be.  The general path's stream objects and
+    repeated checks took more of the host's time than a small call's kernels."""
+    torch = _torch()
+    if (stream is not None or type(tris) is not torch.Tensor or not tris.is_cuda or tris.dtype is not torch.float32
+            or not tris.is_contiguous()):
+        return None
+    c = info._c
+    g = c.gridsize[0]
+    words = (g * g * g + 31) // 32
+    if tris.numel() < 9 * c.n_triangles:
+        return None
+    device = tris.device
+    if table is None:
+        table = torch.empty(words, dtype=torch.int32, device=device)
+    elif (type(table) is not torch.Tensor or not table.is_cuda or table.dtype is not torch.int32
+          or not table.is_contiguous() or table.numel() < words):
+        return None
+    return table, torch._C._cuda_getCurrentRawStream(device.index) or None
+
+
 def voxelize_surface(info: VoxInfo, tris, morton: bool = False, table=None, accumulate: bool = False,
                      algo: str = "auto", stream=None, tune: int = 0):
     """Surface voxelization (stream-ordered).  Returns the int32 table tensor.
@@ -227,13 +250,19 @@ def voxelize_surface(info: VoxInfo, tris, morton: bool = False, table=None, accu
     bits are OR-ed into the existing contents (reference semantics).
     ``tune``: VOX_TUNE_* bits (``_capi.tune_*``) and the algorithm's VOX_SLAB_* / VOX_REGION_*
     bits (``_capi.region_*``); every setting gives the same table."""
+    flags = (VOX_FLAG_ACCUMULATE if accumulate else 0) | _algo_flag(algo) | (int(tune) & _capi.KNOB_MASK)
+    lib = _capi.load()
+    plain = _plain_call(info, tris, table, stream)
+    if plain is not None:
+        table, ptr = plain
+        check(lib.vox_surface(info._c, tris.data_ptr(), table.data_ptr(),
+                              VOX_LAYOUT_MORTON if morton else VOX_LAYOUT_LINEAR, flags, ptr))
+        return table
     torch = _torch()
     with _OnStream(stream, tris.device) as on:
         if table is None:
             table = torch.empty(table_words(info.grid), dtype=torch.int32, device=tris.device)
         _info_checked(info, tris, table)
-        flags = (VOX_FLAG_ACCUMULATE if accumulate else 0) | _algo_flag(algo) | (int(tune) & _capi.KNOB_MASK)
-        lib = _capi.load()
         check(lib.vox_surface(ctypes.byref(info._c), tris.data_ptr(), table.data_ptr(),
                               VOX_LAYOUT_MORTON if morton else VOX_LAYOUT_LINEAR, flags, on.ptr))
     return table
@@ -248,17 +277,23 @@ def voxelize_solid_table(info: VoxInfo, tris, morton: bool = False, table=None, 
     it).  Such runs spill into the next rows (linear layout) or are cut at
     the table end exactly as the reference indexes them; runs with a
     negative end are empty."""
+    flags = (VOX_FLAG_ACCUMULATE if accumulate else 0) | _algo_flag(algo) | (int(tune) & _capi.KNOB_MASK)
+    lib = _capi.load()
+    plain = _plain_call(info, tris, table, stream) if offrow is None else None
+    if plain is not None:
+        table, ptr = plain
+        check(lib.vox_solid(info._c, tris.data_ptr(), table.data_ptr(),
+                            VOX_LAYOUT_MORTON if morton else VOX_LAYOUT_LINEAR, flags, None, ptr))
+        return table
     torch = _torch()
     with _OnStream(stream, tris.device) as on:
         if table is None:
             table = torch.empty(table_words(info.grid), dtype=torch.int32, device=tris.device)
         _info_checked(info, tris, table)
-        flags = (VOX_FLAG_ACCUMULATE if accumulate else 0) | _algo_flag(algo) | (int(tune) & _capi.KNOB_MASK)
         cl_ptr = None
         if offrow is not None:
             _check_tensor(offrow, "torch.int64", "offrow")
             cl_ptr = offrow.data_ptr()
-        lib = _capi.load()
         check(lib.vox_solid(ctypes.byref(info._c), tris.data_ptr(), table.data_ptr(),
                             VOX_LAYOUT_MORTON if morton else VOX_LAYOUT_LINEAR, flags, cl_ptr, on.ptr))
     return table
@@ -399,12 +434,20 @@ def sort_triangles(info: VoxInfo, tris, stream=None, with_perm: bool = False):
     return (out, perm) if with_perm else out
 
 
-def upload(host_array: np.ndarray, device="cuda:0", stream=None):
-    """Host array -> new device tensor through pinned double-buffered staging."""
+def _upload_queued(host_array: np.ndarray, device, stream):
+    """Host array -> new device tensor; the array has been read when this returns,
+    the copy to the device is in `stream`'s (None: the current stream's) order."""
     torch = _torch()
     a = np.ascontiguousarray(host_array)
     out = torch.empty(a.shape, dtype=getattr(torch, str(a.dtype)), device=device)
     check(_capi.load().vox_upload_async(a.ctypes.data, a.nbytes, out.data_ptr(), _stream_ptr(stream)))
+    return out
+
+
+def upload(host_array: np.ndarray, device="cuda:0", stream=None):
+    """Host array -> new device tensor through pinned double-buffered staging."""
+    torch = _torch()
+    out = _upload_queued(host_array, device, stream)
     torch.cuda.current_stream().synchronize() if stream is None else stream.synchronize()
     return out
 
@@ -414,11 +457,25 @@ def prepare_mesh(vertices: np.ndarray, faces: np.ndarray, grid: int, device="cud
     AoS packing.  Returns (VoxInfo, triangle tensor).  With `spatial_order`
     the triangles are then put in spatial order (sort_triangles), for a mesh
     that is voxelized many times."""
-    v = upload(np.asarray(vertices, np.float32).reshape(-1), device)
-    f = upload(np.asarray(faces, np.int32).reshape(-1), device)
-    box = mesh_bbox_device(v)
-    info = VoxInfo(create_mesh_bbox_cube(box), (grid, grid, grid), f.numel() // 3)
-    tris = pack_triangles(v, f)
+    torch = _torch()
+    # one stream orders the uploads, the box and the packing, so the host waits
+    # once, for the box and the count of bad indices together (32 bytes)
+    with torch.cuda.device(device):
+        v = _upload_queued(np.asarray(vertices, np.float32).reshape(-1), device, None)
+        f = _upload_queued(np.asarray(faces, np.int32).reshape(-1), device, None)
+        n = f.numel() // 3
+        lib = _capi.load()
+        ptr = _stream_ptr(None)
+        tris = torch.empty(n * 9, dtype=torch.float32, device=device)
+        found = torch.zeros(4, dtype=torch.int64, device=device)  # six floats, and the count
+        check(lib.vox_mesh_bbox(v.data_ptr(), v.numel() // 3, found.data_ptr(), ptr))
+        check(lib.vox_pack_triangles(v.data_ptr(), v.numel() // 3, f.data_ptr(), n, tris.data_ptr(),
+                                     found.data_ptr() + 24, ptr))
+        h = found.cpu().numpy()
+    box = h[:3].view(np.float32)
+    info = VoxInfo(create_mesh_bbox_cube(AABox(box[:3], box[3:])), (grid, grid, grid), n)
+    if int(h[3]):
+        raise ValueError(f"{int(h[3])} face indices out of range")
     return info, (sort_triangles(info, tris) if spatial_order else tris)
 
 
