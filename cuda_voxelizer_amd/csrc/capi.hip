@@ -234,13 +234,16 @@ vox_status run(const vox_info* info, const float* d_tris, uint32_t* d_table, int
         if (e != hipSuccess) return hip_fail(e, "tile kernels launch");
         return VOX_OK;
     }
+    if (algo == CHUNK) {
+        e = launch_surface_chunk(*info, d_tris, d_table, layout, accumulate, st, tune_big(flags), tune_waves(flags));
+        if (e != hipSuccess) return hip_fail(e, "chunk kernels launch");
+        return VOX_OK;
+    }
     if (!accumulate) {
         e = launch_fill_zero(*info, d_table, st);
         if (e != hipSuccess) return hip_fail(e, "table zero-fill");
     }
-    if (algo == CHUNK)
-        e = launch_surface_chunk(*info, d_tris, d_table, layout, st, tune_big(flags), tune_waves(flags));
-    else if (solid)
+    if (solid)
         e = launch_solid_direct(*info, d_tris, d_table, layout, (unsigned long long*)d_offrow, st);
     else
         e = launch_surface_direct(*info, d_tris, d_table, layout, st);

@@ -13,12 +13,24 @@
 // its lanes and ORs each row's interval (rows.h).  The table is then updated with
 // one non-returning global atomicOr per distinct word; words that do not fit
 // in the hash go straight to global atomics.  The table is zero-filled
-// beforehand (unless accumulating).
+// beforehand (unless accumulating), or the words go to a zeroed scratch table in
+// blocked order, from which the table is then written.
+//
+// Blocked order: a memory atomic costs the same whatever it hits (26 G/s on
+// scattered words, in 256 KB as in 1 GB; plain stores do 70 to 190 G/s), but
+// neighbouring lanes with words of one 64-byte line are one request.  In a
+// linear table such a line is 512 voxels of one row, of which a surface has one
+// or two; a blocked line is a word of 4 x 4 rows (32 x 4 x 4 voxels), so a
+// triangle's rows share two or three lines.
 #include "jobs.h"
 #include "raster.h"
 #include "region.h"
 #include "rows.h"
 #include "vox_kernels.h"
+
+#include <map>
+#include <mutex>
+#include <utility>
 
 #pragma clang fp contract(off)
 
@@ -56,6 +68,14 @@ struct ChunkShared {
     };
 };
 
+// A word's bits into the table; kSpecFlagged: the flags that say which 256 bytes
+// of the scratch table hold any come before it.
+template <int SPEC>
+__device__ __forceinline__ void memory_or(uint32_t* __restrict__ table, uint32_t key, uint32_t mask) {
+    if (SPEC == kSpecFlagged) *((uint8_t*)table - 1 - (key >> 6)) = 1;
+    atomicOr(table + key, mask);
+}
+
 // ident: the slot is the key modulo kHashCap.  Used when the whole table has
 // at most kHashCap words (its slots are preset to their keys, so every word is
 // found at its first probe) and for Morton keys (a chunk's words are a compact
@@ -63,10 +83,16 @@ struct ChunkShared {
 // stride, so they are hashed multiplicatively.
 // REG (region algorithm): more slots are tried, and a word that finds none is
 // staged as a fallback pair instead of going to the table.
-template <bool REG>
+// BLK (blocked keys): the 16 words of a key's line take the slots of one group of
+// 16, in order, so that the flush finds them in neighbouring lanes; a word
+// whose slot another line's word has moves on by whole groups.
+template <bool REG, int SPEC>
 __device__ __forceinline__ void word_or(ChunkShared& S, uint32_t* __restrict__ table, bool ident, uint32_t key,
                                         uint32_t mask, const RegionArgs& RA) {
-    uint32_t h = ident ? (key & (kHashCap - 1)) : (key * 2654435761u) >> (32 - kHashBits);
+    constexpr bool BLK = SPEC >= kSpecBlocked;
+    uint32_t h = BLK     ? ((((key >> 4) * 2654435761u) >> (32 - (kHashBits - 4))) << 4) | (key & 15u)
+                 : ident ? (key & (kHashCap - 1))
+                         : (key * 2654435761u) >> (32 - kHashBits);
 #pragma unroll 1
     for (int probe = 0; probe < (REG ? kRegionProbes : kProbes); probe++) {
         // one round trip: the CAS claims an empty slot or returns the key
@@ -77,12 +103,12 @@ __device__ __forceinline__ void word_or(ChunkShared& S, uint32_t* __restrict__ t
             atomicOr(&S.vals[h], mask);
             return;
         }
-        h = (h + 1) & (kHashCap - 1);
+        h = (h + (BLK ? 16u : 1u)) & (kHashCap - 1);
     }
     if (REG)
         region_fallback(RA.P, RA.W, key, mask);
     else
-        atomicOr(table + key, mask);  // hash table crowded: go to memory directly
+        memory_or<SPEC>(table, key, mask);  // hash table crowded: go to memory directly
 }
 
 // Passing voxels of row (y, z) as a mask (bit k = voxel cx + k, cx a multiple
@@ -101,14 +127,17 @@ __device__ __forceinline__ void emit_mask(ChunkShared& S, uint32_t* __restrict__
                                          : morton3((uint32_t)cx, (uint32_t)y, (uint32_t)z);
         const uint32_t yz_low = ((uint32_t)(y & 1) << 1) | ((uint32_t)(z & 1) << 2) | ((uint32_t)((y >> 1) & 1) << 4);
         morton_chunk_words(base, yz_low, mask,
-                           [&](uint64_t w, uint32_t bits) { word_or<REG>(S, table, ident, (uint32_t)w, bits, RA); });
+                           [&](uint64_t w, uint32_t bits) { word_or<REG, SPEC>(S, table, ident, (uint32_t)w, bits, RA); });
     } else if (REG) {
-        word_or<REG>(S, table, ident, region_row_key(RA.P, (uint32_t)cx >> 5, (uint32_t)y, (uint32_t)z),
+        word_or<REG, SPEC>(S, table, ident, region_row_key(RA.P, (uint32_t)cx >> 5, (uint32_t)y, (uint32_t)z),
                      __brev(mask), RA);
+    } else if (SPEC >= kSpecBlocked) {
+        word_or<REG, SPEC>(S, table, ident, blocked_word(G, (uint32_t)cx >> 5, (uint32_t)y, (uint32_t)z), __brev(mask),
+                           RA);
     } else if (SPEC == kSpecLinear || (G & 31u) == 0) {
         // (z G + y) G/32 + cx/32 < G^3/32 < 2^32 (chunk_supported), so 32-bit arithmetic is exact
         const uint32_t w = ((uint32_t)z * G + (uint32_t)y) * (G >> 5) + ((uint32_t)cx >> 5);
-        word_or<REG>(S, table, ident, w, __brev(mask), RA);
+        word_or<REG, SPEC>(S, table, ident, w, __brev(mask), RA);
     } else {
         // linear rows not aligned to words: per voxel
         const uint64_t row = (uint64_t)y * G + (uint64_t)z * G * G;
@@ -119,13 +148,13 @@ __device__ __forceinline__ void emit_mask(ChunkShared& S, uint32_t* __restrict__
             const uint64_t idx = row + (uint64_t)(cx + k);
             const uint32_t w = (uint32_t)(idx >> 5);
             if (w != cur) {
-                if (bits) word_or<REG>(S, table, ident, cur, bits, RA);
+                if (bits) word_or<REG, SPEC>(S, table, ident, cur, bits, RA);
                 cur = w;
                 bits = 0;
             }
             bits |= bit_mask(idx);
         }
-        if (bits) word_or<REG>(S, table, ident, cur, bits, RA);
+        if (bits) word_or<REG, SPEC>(S, table, ident, cur, bits, RA);
     }
 }
 
@@ -147,7 +176,7 @@ __device__ __forceinline__ void lane_raster(ChunkShared& S, uint32_t* __restrict
     const bool m32 = SPEC == kSpecMorton ||
                      (SPEC == kSpecAny && layout == VOX_LAYOUT_MORTON && info.gridsize[0] <= 1024u);
     const uint32_t sc0 = m32 ? spread10((uint32_t)c0) : 0u, sc1 = m32 ? spread10((uint32_t)c0 + 32u) : 0u;
-    const auto put = [&](uint64_t w, uint32_t bits) { word_or<REG>(S, table, ident, (uint32_t)w, bits, RA); };
+    const auto put = [&](uint64_t w, uint32_t bits) { word_or<REG, SPEC>(S, table, ident, (uint32_t)w, bits, RA); };
     const int step = SPLIT ? 1 << lg : 1;
     int ynext = T.lo[1] + (SPLIT ? sub : 0);  // the lane's next row in y
     for (int z = T.lo[2]; z <= T.hi[2]; z++) {
@@ -246,8 +275,8 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE || (SPEC != kSpecAny 
     }
     const ItemDev& it = MULTI ? J.it : one;
     const vox_info& info = it.info;
-    uint32_t* __restrict__ table = it.table;
-    const int layout = SPEC == kSpecLinear ? (int)VOX_LAYOUT_LINEAR
+    uint32_t* __restrict__ table = SPEC >= kSpecBlocked ? it.scratch : it.table;
+    const int layout = SPEC == kSpecLinear || SPEC >= kSpecBlocked ? (int)VOX_LAYOUT_LINEAR
                        : SPEC == kSpecMorton ? (int)VOX_LAYOUT_MORTON : it.layout;
     const uint64_t n = info.n_triangles;
     const uint32_t parts = it.parts > 1u ? it.parts : 1u;
@@ -353,7 +382,7 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE || (SPEC != kSpecAny 
     } else {
 #pragma unroll
         for (int u = 0; u < kPer; u++)
-            if (kk[u] != kEmpty && vv[u] != 0u) atomicOr(table + kk[u], vv[u]);
+            if (kk[u] != kEmpty && vv[u] != 0u) memory_or<SPEC>(table, kk[u], vv[u]);
     }
 }
 
@@ -379,6 +408,178 @@ __global__ void __launch_bounds__(256) fill_zero_kernel(ItemDev one, ItemMap M) 
     } else {
         for (uint64_t i = w0 + threadIdx.x; i < w1; i += 256) table[i] = 0u;
     }
+}
+
+// Blocked scratch table -> rows of the linear table (G a multiple of 32); the
+// scratch words that held bits return to zero.  A thread takes 4 words in x of
+// the 4 rows in y of one z: four 16-byte loads, a transpose in registers, four
+// 16-byte stores (VEC: rows of whole 16-byte groups, aligned tables), or else
+// one word in x of those 4 rows.  Work unit: 256 threads.
+// accumulate: bits are ORed into the table, only where there are any.
+// FLAGS: groups of 256 bytes whose flag is not set are zero and not read.
+template <bool FLAGS>
+__device__ __forceinline__ void unblock_quad(const ItemDev& it, uint32_t t, bool vec) {
+    const uint32_t G = it.info.gridsize[0], rw = G >> 5;
+    uint4* __restrict__ s4 = (uint4*)it.scratch;
+    const uint32_t zl = t & 3u;
+    uint32_t r = t >> 2;
+    if (vec) {
+        const uint32_t wq = r % (rw >> 2);
+        r /= rw >> 2;
+        const uint32_t by = r % (G >> 2), bz = r / (G >> 2);
+        if (bz >= G >> 2) return;
+        const uint64_t base = ((uint64_t)(bz * (G >> 2) + by) * rw + 4u * wq) * 4u + zl;
+        uint4 v[4];
+        // the four lanes of a 256-byte group read its flag in one instruction, before it is cleared
+        uint8_t* flag = (uint8_t*)it.scratch - 1 - (base >> 4);
+        const bool any = !FLAGS || *flag != 0;
+        if (FLAGS && any && zl == 0u) *flag = 0;
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = any ? s4[base + 4u * (uint32_t)u] : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (v[u].x | v[u].y | v[u].z | v[u].w) s4[base + 4u * (uint32_t)u] = make_uint4(0u, 0u, 0u, 0u);
+        const uint4 o[4] = {make_uint4(v[0].x, v[1].x, v[2].x, v[3].x), make_uint4(v[0].y, v[1].y, v[2].y, v[3].y),
+                            make_uint4(v[0].z, v[1].z, v[2].z, v[3].z), make_uint4(v[0].w, v[1].w, v[2].w, v[3].w)};
+        uint4* __restrict__ d4 = (uint4*)it.table;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint64_t d = (((uint64_t)(4u * bz + zl) * G + 4u * by + (uint32_t)u) * rw >> 2) + wq;
+            if (!it.accumulate) {
+                d4[d] = o[u];
+            } else if (o[u].x | o[u].y | o[u].z | o[u].w) {
+                const uint4 p = d4[d];
+                d4[d] = make_uint4(p.x | o[u].x, p.y | o[u].y, p.z | o[u].z, p.w | o[u].w);
+            }
+        }
+        return;
+    }
+    const uint32_t w = r % rw;
+    r /= rw;
+    const uint32_t by = r % (G >> 2), bz = r / (G >> 2);
+    if (bz >= G >> 2) return;
+    const uint64_t i = ((uint64_t)(bz * (G >> 2) + by) * rw + w) * 4u + zl;
+    const uint4 v = s4[i];
+    if (v.x | v.y | v.z | v.w) s4[i] = make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t o[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const uint64_t d = ((uint64_t)(4u * bz + zl) * G + 4u * by + (uint32_t)u) * rw + w;
+        if (!it.accumulate)
+            it.table[d] = o[u];
+        else if (o[u])
+            it.table[d] |= o[u];
+    }
+}
+
+__host__ __device__ inline bool unblock_vec(uint32_t G, const uint32_t* table) {
+    return (G & 127u) == 0 && (((uintptr_t)table) & 15u) == 0;
+}
+
+template <bool FLAGS>
+__global__ void __launch_bounds__(256) unblock_kernel(ItemDev one, ItemMap M) {
+    __shared__ BlockJob J;
+    if (M.items) {
+        resolve_job(one, M, blockIdx.x, J);
+        if (J.local == ~0u) return;
+    }
+    const ItemDev& it = M.items ? J.it : one;
+    const uint32_t local = M.items ? J.local : blockIdx.x;
+    unblock_quad<FLAGS>(it, local * 256u + threadIdx.x, FLAGS || unblock_vec(it.info.gridsize[0], it.table));
+}
+
+uint32_t unblock_units(uint32_t G, const uint32_t* table) {
+    const uint64_t words = (uint64_t)G * G * G / 32u;
+    return (uint32_t)((words / (unblock_vec(G, table) ? 16u : 4u) + 255u) / 256u);
+}
+
+hipError_t launch_unblock_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, hipStream_t stream) {
+    if (units == 0) return hipSuccess;
+    if (!M.items && one.flagged)
+        unblock_kernel<true><<<units, 256, 0, stream>>>(one, M);
+    else
+        unblock_kernel<false><<<units, 256, 0, stream>>>(one, M);
+    return hipGetLastError();
+}
+
+// A stream's blocked scratch table of at least `bytes` bytes, all zero between
+// calls: grow-only, at most the table's size
+// and its flags (1 GB + 4 MB, kBlockedGrid).  It is the holder's until the
+// lease ends, so that two threads' calls on one stream do not mix their
+// launches.  words is null when there is none: while the stream is being
+// captured (a later call may replace the buffer that the graph would hold), or
+// without memory.  clean() says that all launches are queued that leave it zero;
+// without it the next holder zero-fills it.
+struct SurfaceScratch {
+    void* ptr = nullptr;
+    uint64_t bytes = 0;
+    bool dirty = true;
+    std::mutex use;
+};
+static std::mutex g_scratch_mutex;
+static std::map<std::pair<int, hipStream_t>, SurfaceScratch> g_scratch;
+
+struct ScratchLease {
+    uint32_t* words = nullptr;
+    SurfaceScratch* b = nullptr;
+
+    ScratchLease(uint64_t bytes, hipStream_t stream) {
+        int dev = 0;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &cap) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
+            (void)hipGetLastError();
+            return;
+        }
+        if (cap != hipStreamCaptureStatusNone) return;
+        {
+            std::lock_guard<std::mutex> lock(g_scratch_mutex);
+            b = &g_scratch[{dev, stream}];
+        }
+        b->use.lock();
+        hipError_t e = hipSuccess;
+        if (b->bytes < bytes) {
+            if (b->ptr) {
+                e = hipStreamSynchronize(stream);  // a previous call on this stream may still use it
+                if (e == hipSuccess) e = hipFree(b->ptr);
+            }
+            b->ptr = nullptr;
+            b->bytes = 0;
+            if (e == hipSuccess) e = hipMalloc(&b->ptr, bytes);
+            if (e == hipSuccess) b->bytes = bytes;
+            b->dirty = true;
+        }
+        if (e == hipSuccess && b->dirty) e = hipMemsetAsync(b->ptr, 0, b->bytes, stream);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            return;
+        }
+        words = (uint32_t*)b->ptr;
+        b->dirty = true;
+    }
+    void clean() { b->dirty = false; }
+    ~ScratchLease() {
+        if (b) b->use.unlock();
+    }
+    ScratchLease(const ScratchLease&) = delete;
+    ScratchLease& operator=(const ScratchLease&) = delete;
+};
+
+// Where words go through a blocked scratch table: linear rows of whole words, in
+// tables beyond the dense LDS merge; a call of few triangles at G <= 80 has too
+// few atomics for it (displaced sphere of 1,280 at 64^3 12.3 us, 13.3 blocked; a
+// soup of 100,003 at 64^3 76.6 and 27.9).  Measured with the rows of a linear
+// table as keys -> blocked (us per call): soup of 300,003 at 128^3 160 -> 45,
+// 100,003 at 256^3 88 -> 67; displaced sphere of 81,920 at 256^3 31 -> 21, at
+// 512^3 65 -> 37, 327,680 at 512^3 92 -> 60; torus of 200,000 at 256^3 19 -> 14;
+// with flags: 81,920 at 1024^3 149 -> 86, at 2048^3 728 -> 485; torus of
+// 1,048,576 at 1024^3 105 -> 76.  The flags save the row pass most of the
+// scratch table at 1024^3 and above (81,920 at 1024^3 103 -> 86, at 2048^3 529 ->
+// 485); at 512^3 and below setting them costs more than that (327,680 at 256^3
+// 41 without, 46 with).
+bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles) {
+    const uint64_t words = (uint64_t)G * G * G / 32u;
+    return layout == VOX_LAYOUT_LINEAR && (G & 31u) == 0 && G <= kBlockedGrid &&
+           words > (n_triangles < 16384u ? 16384u : (uint64_t)kHashCap);
 }
 
 bool chunk_supported(uint32_t G) { return (uint64_t)G * G * G / 32 < 0xFFFFFFFFull; }
@@ -436,6 +637,10 @@ static void launch_chunk_spec(int spec, uint32_t units, hipStream_t stream, cons
     const RegionArgs none{};
     if (spec == kSpecLinear)
         surface_chunk_kernel<MULTI, false, WIDE, false, kSpecLinear, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
+    else if (spec == kSpecBlocked)
+        surface_chunk_kernel<MULTI, false, WIDE, false, kSpecBlocked, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
+    else if (!MULTI && spec == kSpecFlagged)
+        surface_chunk_kernel<false, false, WIDE, false, kSpecFlagged, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
     else if (spec == kSpecMorton)
         surface_chunk_kernel<MULTI, false, WIDE, false, kSpecMorton, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
     else
@@ -451,7 +656,7 @@ hipError_t launch_chunk_jobs(const ItemDev& one, const ItemMap& M, uint32_t unit
                              int waves, int spec) {
     if (units == 0) return hipSuccess;
     const bool wide = waves == 6 || (waves == 0 && !M.items && one.layout == VOX_LAYOUT_LINEAR);
-    if (!M.items) spec = chunk_spec(one.layout, one.info.gridsize[0]);
+    if (!M.items) spec = one.scratch ? (int)(one.flagged ? kSpecFlagged : kSpecBlocked) : chunk_spec(one.layout, one.info.gridsize[0]);
     const RegionArgs none{};
     if (loop && M.items)
         surface_chunk_kernel<true, true, false, false><<<units, kChunk, 0, stream>>>(one, M, none);
@@ -539,13 +744,34 @@ hipError_t launch_surface_region_chunks(const vox_info& info, const float* tris,
     return hipGetLastError();
 }
 
-hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_t* table, int layout,
+hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_t* table, int layout, bool accumulate,
                                 hipStream_t stream, uint32_t big, int waves) {
-    if (info.n_triangles == 0) return hipSuccess;
     const ItemMap none{nullptr, nullptr, 1, 0};
     ItemDev one = single_job(info, tris, table, layout);
     one.big = big;
+    one.accumulate = accumulate ? 1 : 0;
     chunk_shape(one);
+    const uint32_t G = info.gridsize[0];
+    if (info.n_triangles && chunk_blocked(layout, G, info.n_triangles)) {
+        hipError_t e = hipSuccess;
+        const uint64_t bytes = (uint64_t)G * G * G / 8u;
+        one.flagged = G > kUnflaggedGrid && unblock_vec(G, table) ? 1u : 0u;
+        const uint64_t flags = one.flagged ? bytes / 256u : 0u;
+        ScratchLease S(bytes + flags, stream);
+        if (S.words) {
+            one.scratch = S.words + flags / 4u;
+            e = launch_chunk_jobs(one, none, chunk_units(info.n_triangles, one.span, one.parts, one.lg_split), false,
+                                  stream, waves);
+            if (e == hipSuccess) e = launch_unblock_jobs(one, none, unblock_units(G, table), stream);
+            if (e == hipSuccess) S.clean();
+            return e;
+        }
+    }
+    if (!accumulate) {
+        const hipError_t e = launch_fill_zero(info, table, stream);
+        if (e != hipSuccess) return e;
+    }
+    if (info.n_triangles == 0) return hipSuccess;
     return launch_chunk_jobs(one, none, chunk_units(info.n_triangles, one.span, one.parts, one.lg_split),
                              one.span > 1u && one.parts <= 1u, stream, waves);
 }

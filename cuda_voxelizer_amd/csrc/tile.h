@@ -37,6 +37,7 @@ struct ItemDev {
     vox_info info;
     const float* tris;
     uint32_t* table;
+    uint32_t* scratch;           // chunk: blocked scratch table (null: the words go to the table)
     unsigned long long* offrow;  // solid: out-of-row run counter (may be null)
     TilePlan P;
     int32_t layout, solid, accumulate;
@@ -47,7 +48,7 @@ struct ItemDev {
     uint32_t big;        // chunk: voxel boxes above this are shared by the workgroup; marker: columns
                          // above this (0: the built-in threshold)
     uint32_t lg_split;   // chunk, marker: 2^lg_split lanes share a triangle, so a workgroup takes 256 >> lg_split
-    uint32_t pad2;
+    uint32_t flagged;    // chunk: the blocked scratch table has flags before it
 };
 
 // Work mapping of one launch: a single job passed by value (items == nullptr)

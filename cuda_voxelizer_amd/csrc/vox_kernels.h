@@ -103,14 +103,23 @@ uint32_t chunk_parts(uint32_t G, uint64_t n_triangles);
 uint32_t chunk_units(uint64_t n_triangles, uint32_t span, uint32_t parts, uint32_t lg_split = 0);
 hipError_t launch_fill_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, hipStream_t stream);
 // What a chunk kernel instantiation knows of its jobs' layout: nothing, linear
-// with G a multiple of 32 (whole words per row), or Morton with G <= 1024
-// (codes fit 30 bits).
-enum ChunkSpec : int { kSpecAny = 0, kSpecLinear = 1, kSpecMorton = 2 };
+// with G a multiple of 32 (whole words per row), Morton with G <= 1024
+// (codes fit 30 bits), or blocked (ItemDev.scratch), without or with flags.
+enum ChunkSpec : int { kSpecAny = 0, kSpecLinear = 1, kSpecMorton = 2, kSpecBlocked = 3, kSpecFlagged = 4 };
 int chunk_spec(int layout, uint32_t G);
 hipError_t launch_chunk_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, bool loop, hipStream_t stream,
                              int waves = 0, int spec = kSpecAny);
-hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_t* table, int layout,
+hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_t* table, int layout, bool accumulate,
                                 hipStream_t stream, uint32_t big = 0, int waves = 0);
+// Word w of row (y, z) in a blocked table: the 4 x 4 rows of a block lie together.
+__device__ __forceinline__ uint32_t blocked_word(uint32_t G, uint32_t w, uint32_t y, uint32_t z) {
+    return ((((z >> 2) * (G >> 2) + (y >> 2)) * (G >> 5) + w) << 4) | ((z & 3u) << 2) | (y & 3u);
+}
+constexpr uint32_t kBlockedGrid = 2048;
+constexpr uint32_t kUnflaggedGrid = 512;
+bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles);
+uint32_t unblock_units(uint32_t G, const uint32_t* table);
+hipError_t launch_unblock_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, hipStream_t stream);
 // Tuning bits of the flags (VOX_TUNE_*): queue threshold, chunk waves per SIMD, tile size.
 inline uint32_t tune_big(unsigned flags) {
     const unsigned lg = (flags >> 24) & 15u;
