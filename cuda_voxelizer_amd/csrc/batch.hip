@@ -36,16 +36,18 @@ struct vox_batch {
     int device = 0;
     bool use_graph = true;
     hipStream_t cap_stream = nullptr;
-    hipStream_t side[4] = {};  // capture only: tile chain, marker chain, direct classes, generic chunk classes
+    hipStream_t side[4] = {};  // capture only: tile chain, marker chain, direct classes, fill and its chunk classes
     hipEvent_t ev[6] = {};     // capture only: fork, tables zeroed, and the four side branches' ends
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     void* dev_mem = nullptr;
     void* ws = nullptr;
     void* mws = nullptr;  // marker class: spill records and counters
+    void* sws = nullptr;  // blocked chunk class: the jobs' scratch tables, all zero between launches
     voxamd::WorkspaceLayout L{};
     // chunk / chunkw (6 waves per SIMD): one class per layout specialisation (ChunkSpec)
-    voxamd::JobClass fill, chunk[3], chunkw[3], marker, dsurf, dsolid, tsurf, tsolid;
+    voxamd::JobClass fill, chunk[voxamd::kBlockedSpecs], chunkw[voxamd::kBlockedSpecs], unblock, marker, dsurf, dsolid,
+        tsurf, tsolid;
     int count = 0;
     uint64_t total_triangles = 0;
 };
@@ -67,16 +69,16 @@ static hipError_t launch_fill_class(vox_batch* b, hipStream_t s) {
     return launch_fill_jobs(dummy, b->fill.m_a, b->fill.total_a, s);
 }
 
-// Which chunk classes a launch covers: all, the layout-generic ones (the
-// chunk loop of small dense tables among them) or the layout-specialised ones.
-enum ChunkClassSet { kAllChunkClasses, kGenericChunkClasses, kSpecialisedChunkClasses };
+// Which chunk classes a launch covers: those whose tables are zero-filled
+// before, or the blocked one, whose scratch tables are zero already and whose
+// tables the unblock pass then writes.
+enum ChunkClassSet { kFilledChunkClasses, kBlockedChunkClass };
 
-static hipError_t launch_chunk_classes(vox_batch* b, hipStream_t s, ChunkClassSet which = kAllChunkClasses) {
+static hipError_t launch_chunk_classes(vox_batch* b, hipStream_t s, ChunkClassSet which) {
     const ItemDev dummy{};
     hipError_t e = hipSuccess;
-    for (int sp = 0; sp < 3; sp++) {
-        if ((which == kGenericChunkClasses && sp != kSpecAny) || (which == kSpecialisedChunkClasses && sp == kSpecAny))
-            continue;
+    for (int sp = 0; sp < kBlockedSpecs; sp++) {
+        if ((which == kBlockedChunkClass) != (sp == kSpecBlocked)) continue;
         const JobClass& c5 = b->chunk[sp];
         const JobClass& c6 = b->chunkw[sp];
         if (c5.total_a && (e = launch_chunk_jobs(dummy, c5.m_a, c5.total_a, c5.loop, s, 5, sp)) != hipSuccess)
@@ -84,6 +86,7 @@ static hipError_t launch_chunk_classes(vox_batch* b, hipStream_t s, ChunkClassSe
         if (c6.total_a && (e = launch_chunk_jobs(dummy, c6.m_a, c6.total_a, c6.loop, s, 6, sp)) != hipSuccess)
             return e;
     }
+    if (which == kBlockedChunkClass) return launch_unblock_jobs(dummy, b->unblock.m_a, b->unblock.total_a, s);
     return hipSuccess;
 }
 
@@ -122,7 +125,8 @@ static hipError_t launch_tile_classes(vox_batch* b, hipStream_t s) {
 static hipError_t launch_all(vox_batch* b, hipStream_t s) {
     hipError_t e = hipSuccess;
     if ((e = launch_fill_class(b, s)) != hipSuccess) return e;
-    if ((e = launch_chunk_classes(b, s)) != hipSuccess) return e;
+    if ((e = launch_chunk_classes(b, s, kBlockedChunkClass)) != hipSuccess) return e;
+    if ((e = launch_chunk_classes(b, s, kFilledChunkClasses)) != hipSuccess) return e;
     if ((e = launch_marker_class(b, s)) != hipSuccess) return e;
     if ((e = launch_direct_classes(b, s)) != hipSuccess) return e;
     return launch_tile_classes(b, s);
@@ -133,21 +137,21 @@ static hipError_t launch_all(vox_batch* b, hipStream_t s) {
 // small latency-bound kernels (the tile chain's scans, the chunk loop of
 // small dense tables, the marker chain's spill pass) overlap the others
 // instead of leaving the GPU idle between kernels.  Nodes are created in the
-// order the critical path wants them dispatched: the fill, then the
-// layout-specialised chunk classes (the bulk of most batches) on `m`, then
-// the branches -- the tile chain (no fill; it forks from before the fill),
-// the marker chain, the direct classes and the layout-generic chunk classes
-// (after the fill).  `m` joins every branch at the end.  Tables of different
-// jobs do not overlap, so the branches share no data (the out-of-row
+// order the critical path wants them dispatched: the blocked chunk class (the
+// bulk of most batches; it needs no fill) on `m`, the fill, then the branches --
+// the tile chain (no fill), the marker chain, the direct classes and the other
+// chunk classes (after the fill).  `m` joins every branch at the end.  Tables of
+// different jobs do not overlap, so the branches share no data (the out-of-row
 // counters they add to are atomic).
 static hipError_t launch_forked(vox_batch* b, hipStream_t m) {
     hipError_t e = hipSuccess;
 #define VOX_TRY(x) \
     if ((e = (x)) != hipSuccess) return e
     VOX_TRY(hipEventRecord(b->ev[0], m));
-    VOX_TRY(launch_fill_class(b, m));
-    VOX_TRY(hipEventRecord(b->ev[1], m));
-    VOX_TRY(launch_chunk_classes(b, m, kSpecialisedChunkClasses));
+    VOX_TRY(launch_chunk_classes(b, m, kBlockedChunkClass));
+    VOX_TRY(hipStreamWaitEvent(b->side[3], b->ev[0], 0));
+    VOX_TRY(launch_fill_class(b, b->side[3]));
+    VOX_TRY(hipEventRecord(b->ev[1], b->side[3]));
     VOX_TRY(hipStreamWaitEvent(b->side[0], b->ev[0], 0));
     VOX_TRY(launch_tile_classes(b, b->side[0]));
     VOX_TRY(hipEventRecord(b->ev[2], b->side[0]));
@@ -157,8 +161,7 @@ static hipError_t launch_forked(vox_batch* b, hipStream_t m) {
     VOX_TRY(hipStreamWaitEvent(b->side[2], b->ev[1], 0));
     VOX_TRY(launch_direct_classes(b, b->side[2]));
     VOX_TRY(hipEventRecord(b->ev[4], b->side[2]));
-    VOX_TRY(hipStreamWaitEvent(b->side[3], b->ev[1], 0));
-    VOX_TRY(launch_chunk_classes(b, b->side[3], kGenericChunkClasses));
+    VOX_TRY(launch_chunk_classes(b, b->side[3], kFilledChunkClasses));
     VOX_TRY(hipEventRecord(b->ev[5], b->side[3]));
     for (int k = 2; k < 6; k++) VOX_TRY(hipStreamWaitEvent(m, b->ev[k], 0));
 #undef VOX_TRY
@@ -177,6 +180,7 @@ static void free_batch(vox_batch* b) {
     if (b->dev_mem) (void)hipFree(b->dev_mem);
     if (b->ws) (void)hipFree(b->ws);
     if (b->mws) (void)hipFree(b->mws);
+    if (b->sws) (void)hipFree(b->sws);
     delete b;
 }
 
@@ -186,11 +190,37 @@ struct BatchPlan {
     std::vector<char> host;
     bool ws_needed = false;
     WorkspaceLayout L{};
+    uint64_t scratch = 0;  // bytes of blocked scratch tables; the jobs hold their offsets until place_scratch
 };
 
+// A batch's scratch tables together; jobs beyond it go to their tables directly.
+constexpr uint64_t kBatchScratch = 1ull << 30;
+
+// Every chunk class and the others, in the order of the packed image.
+constexpr int kClasses = 2 * kBlockedSpecs + 7;
+struct ClassList {
+    JobClass* c[kClasses];
+    explicit ClassList(vox_batch* b) {
+        int k = 0;
+        c[k++] = &b->fill;
+        for (JobClass& j : b->chunk) c[k++] = &j;
+        for (JobClass& j : b->chunkw) c[k++] = &j;
+        for (JobClass* j : {&b->unblock, &b->marker, &b->dsurf, &b->dsolid, &b->tsurf, &b->tsolid}) c[k++] = j;
+    }
+    JobClass** begin() { return c; }
+    JobClass** end() { return c + kClasses; }
+};
+
+// The scratch offsets in the packed image become pointers.
+static void place_scratch(vox_batch* b, BatchPlan& plan) {
+    for (JobClass* c : {&b->chunk[kSpecBlocked], &b->unblock}) {
+        ItemDev* it = (ItemDev*)(plan.host.data() + c->off_items);
+        for (size_t i = 0; i < c->items.size(); i++) it[i].scratch = (uint32_t*)((char*)b->sws + (uintptr_t)it[i].scratch);
+    }
+}
+
 static void reset_classes(vox_batch* b) {
-    JobClass* classes[] = {&b->fill,      &b->chunk[0],  &b->chunk[1], &b->chunk[2], &b->chunkw[0], &b->chunkw[1],
-                           &b->chunkw[2], &b->marker,   &b->dsurf,    &b->dsolid,   &b->tsurf,     &b->tsolid};
+    ClassList classes(b);
     for (JobClass* c : classes) *c = JobClass{};
     b->count = 0;
     b->total_triangles = 0;
@@ -237,7 +267,11 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
         d.big = tune_big(it.flags);
         const uint64_t n = it.info.n_triangles;
         b->total_triangles += n;
-        if (a != TILE && !accumulate) {
+        const uint64_t table_bytes = (uint64_t)G * G * G / 8u;
+        // 48 mixed meshes, linear keys -> blocked: 740 -> 405 us a launch
+        const bool blocked = a == CHUNK && G <= kUnflaggedGrid && chunk_blocked(it.layout, G, n) &&
+                             plan.scratch + table_bytes <= kBatchScratch;
+        if (a != TILE && !accumulate && !blocked) {
             b->fill.items.push_back(d);
             add_prefix(b->fill.base_a, b->fill.total_a, fill_units(G));
         }
@@ -256,7 +290,13 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
             // a layout-specialised kernel runs at six waves per SIMD under either bound, so only
             // layout-generic jobs are split by the waves knob (each class is one more kernel)
             const bool loop = d.span > 1u && d.parts <= 1u;
-            const int sp = loop ? (int)kSpecAny : chunk_spec(it.layout, G);
+            const int sp = blocked ? (int)kSpecBlocked : (loop ? (int)kSpecAny : chunk_spec(it.layout, G));
+            if (blocked) {
+                d.scratch = (uint32_t*)(uintptr_t)plan.scratch;
+                plan.scratch += (table_bytes + 255u) & ~255ull;
+                b->unblock.items.push_back(d);
+                add_prefix(b->unblock.base_a, b->unblock.total_a, unblock_units(G, it.d_table));
+            }
             const bool wide = tune_waves(it.flags) == 6 && !loop && sp == kSpecAny;
             JobClass& c = wide ? b->chunkw[sp] : b->chunk[sp];
             if (loop) c.loop = true;
@@ -283,8 +323,7 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
         }
     }
     // one device allocation: per class the job array and its prefix arrays
-    JobClass* classes[] = {&b->fill,      &b->chunk[0],  &b->chunk[1], &b->chunk[2], &b->chunkw[0], &b->chunkw[1],
-                           &b->chunkw[2], &b->marker,   &b->dsurf,    &b->dsolid,   &b->tsurf,     &b->tsolid};
+    ClassList classes(b);
     size_t total = 0;
     auto reserve = [&](size_t bytes) {
         const size_t off = total;
@@ -317,8 +356,7 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
 // Point every class's job maps at a device copy of the packed image.
 static void bind_maps(vox_batch* b, void* dev) {
     char* dm = (char*)dev;
-    JobClass* classes[] = {&b->fill,      &b->chunk[0],  &b->chunk[1], &b->chunk[2], &b->chunkw[0], &b->chunkw[1],
-                           &b->chunkw[2], &b->marker,   &b->dsurf,    &b->dsolid,   &b->tsurf,     &b->tsolid};
+    ClassList classes(b);
     for (JobClass* c : classes) {
         const ItemDev* it = (const ItemDev*)(dm + c->off_items);
         const int ni = (int)c->items.size();
@@ -350,6 +388,15 @@ vox_status vox_batch_create(const vox_batch_item* items, int count, unsigned fla
     if (s != VOX_OK) {
         free_batch(b);
         return s;
+    }
+    if (plan.scratch) {
+        e = hipMalloc(&b->sws, plan.scratch);
+        if (e == hipSuccess) e = hipMemset(b->sws, 0, plan.scratch);
+        if (e != hipSuccess) {
+            free_batch(b);
+            return fail(VOX_ERR_OOM, std::string("batch scratch tables: ") + hipGetErrorString(e));
+        }
+        place_scratch(b, plan);
     }
     e = hipMalloc(&b->dev_mem, plan.host.size());
     if (e != hipSuccess) {
@@ -414,7 +461,7 @@ vox_status vox_batch_info(const vox_batch* b, int64_t out[8]) {
     out[0] = b->count;
     out[1] = (int64_t)b->total_triangles;
     out[2] = 0;
-    for (int sp = 0; sp < 3; sp++) out[2] += (int64_t)(b->chunk[sp].items.size() + b->chunkw[sp].items.size());
+    for (int sp = 0; sp < kBlockedSpecs; sp++) out[2] += (int64_t)(b->chunk[sp].items.size() + b->chunkw[sp].items.size());
     out[3] = (int64_t)b->tsurf.items.size();
     out[4] = (int64_t)b->tsolid.items.size();
     out[5] = (int64_t)(b->dsurf.items.size() + b->dsolid.items.size());
@@ -445,6 +492,8 @@ struct vox_runner {
     hipEvent_t ev[2] = {nullptr, nullptr};
     int slot = 0;
     uint64_t tiles_cap = 0, n_cap = 0;
+    uint64_t scratch_cap = 0;
+    bool scratch_dirty = false;  // a launch failed between the scratch tables' use and their clearing
     uint64_t launches = 0;
 };
 
@@ -480,7 +529,8 @@ vox_status vox_runner_launch(vox_runner* r, const vox_batch_item* items, int cou
     if (!r->b.tsolid.base_c.empty() && r->b.tsolid.base_c.back() > tris) tris = r->b.tsolid.base_c.back();
     const bool grow_ws = plan.ws_needed && (tiles > r->tiles_cap || tris > r->n_cap || !r->b.ws);
     const bool grow_desc = plan.host.size() > r->dev_cap;
-    if (grow_ws || grow_desc) {
+    const bool grow_scratch = plan.scratch > r->scratch_cap;
+    if (grow_ws || grow_desc || grow_scratch) {
         e = hipStreamSynchronize(r->stream);
         if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
     }
@@ -497,6 +547,25 @@ vox_status vox_runner_launch(vox_runner* r, const vox_batch_item* items, int cou
             r->tiles_cap = r->n_cap = 0;
             return fail(VOX_ERR_OOM, std::string("runner workspace: ") + hipGetErrorString(e));
         }
+    }
+    if (grow_scratch) {
+        if (r->b.sws) (void)hipFree(r->b.sws);
+        r->b.sws = nullptr;
+        r->scratch_cap = 0;
+        e = hipMalloc(&r->b.sws, plan.scratch);
+        if (e != hipSuccess) {
+            r->b.sws = nullptr;
+            return fail(VOX_ERR_OOM, std::string("runner scratch tables: ") + hipGetErrorString(e));
+        }
+        r->scratch_cap = plan.scratch;
+        r->scratch_dirty = true;
+    }
+    if (plan.scratch) {
+        if (r->scratch_dirty) {
+            e = hipMemsetAsync(r->b.sws, 0, r->scratch_cap, r->stream);
+            if (e != hipSuccess) return hip_fail(e, "runner scratch tables");
+        }
+        place_scratch(&r->b, plan);
     }
     if (!r->b.marker.items.empty() && !r->b.mws) {  // fixed size, allocated once
         e = hipMalloc(&r->b.mws, marker_ws_bytes());
@@ -537,15 +606,17 @@ vox_status vox_runner_launch(vox_runner* r, const vox_batch_item* items, int cou
     if (e == hipSuccess) e = hipEventRecord(r->ev[k], r->stream);
     if (e != hipSuccess) return hip_fail(e, "runner descriptor upload");
     bind_maps(&r->b, r->dev_desc);
+    if (plan.scratch) r->scratch_dirty = true;
     e = launch_all(&r->b, r->stream);
     if (e != hipSuccess) return hip_fail(e, "runner launch");
+    if (plan.scratch) r->scratch_dirty = false;
     r->launches++;
     return VOX_OK;
 }
 
 vox_status vox_runner_destroy(vox_runner* r) {
     if (!r) return VOX_OK;
-    if (r->stream || r->b.ws || r->b.mws || r->dev_desc) (void)hipStreamSynchronize(r->stream);
+    if (r->stream || r->b.ws || r->b.mws || r->b.sws || r->dev_desc) (void)hipStreamSynchronize(r->stream);
     for (int i = 0; i < 2; i++) {
         if (r->ev[i]) (void)hipEventDestroy(r->ev[i]);
         if (r->pinned[i]) (void)hipHostFree(r->pinned[i]);
@@ -553,8 +624,10 @@ vox_status vox_runner_destroy(vox_runner* r) {
     if (r->dev_desc) (void)hipFree(r->dev_desc);
     if (r->b.ws) (void)hipFree(r->b.ws);
     if (r->b.mws) (void)hipFree(r->b.mws);
+    if (r->b.sws) (void)hipFree(r->b.sws);
     r->b.ws = nullptr;
     r->b.mws = nullptr;
+    r->b.sws = nullptr;
     delete r;
     return VOX_OK;
 }

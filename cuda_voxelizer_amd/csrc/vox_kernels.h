@@ -115,6 +115,7 @@ hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_
 __device__ __forceinline__ uint32_t blocked_word(uint32_t G, uint32_t w, uint32_t y, uint32_t z) {
     return ((((z >> 2) * (G >> 2) + (y >> 2)) * (G >> 5) + w) << 4) | ((z & 3u) << 2) | (y & 3u);
 }
+constexpr int kBlockedSpecs = kSpecBlocked + 1;  // what a batch's classes may be
 constexpr uint32_t kBlockedGrid = 2048;
 constexpr uint32_t kUnflaggedGrid = 512;
 bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles);

@@ -109,3 +109,29 @@ def test_capture_does_not_hold_the_scratch(oracle, gpu):
         graph.replay()
         torch.cuda.synchronize()
         assert (_host(table) == exp).all()
+
+
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_blocked_batch(oracle, gpu, use_graph):
+    """Blocked jobs beside every other class, launched again and again."""
+    import cuda_voxelizer_amd as V
+    import torch
+    jobs, exp = [], []
+    for k, (n, grid) in enumerate([(3000, 96), (20000, 64), (500, 128), (800, 32), (1500, 100), (9, 160), (700, 640),
+                                   (5000, 256)]):
+        info, tris, d = _case(gpu, n, grid, 100 + k)
+        e = _expected(oracle, info, tris)
+        acc = k % 3 == 2
+        table = torch.zeros(e.size, dtype=torch.int32, device=gpu) if acc else \
+            torch.full((e.size,), -1, dtype=torch.int32, device=gpu)
+        jobs.append(V.BatchJob(info, d, table, accumulate=acc))
+        exp.append(e)
+    batch = V.Batch(jobs, use_graph=use_graph)
+    for _ in range(3):
+        batch.launch()
+        torch.cuda.synchronize()
+        for k, (j, e) in enumerate(zip(jobs, exp)):
+            assert (_host(j.table) == e).all(), k
+            if not j.accumulate:
+                j.table.fill_(0x55)
+    batch.close()
