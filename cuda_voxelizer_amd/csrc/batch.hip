@@ -267,7 +267,7 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
         d.big = tune_big(it.flags);
         const uint64_t n = it.info.n_triangles;
         b->total_triangles += n;
-        const uint64_t table_bytes = (uint64_t)G * G * G / 8u;
+        const uint64_t table_bytes = blocked_bytes(G);
         // 48 mixed meshes, linear keys -> blocked: 740 -> 405 us a launch
         const bool blocked = a == CHUNK && G <= kUnflaggedGrid && chunk_blocked(it.layout, G, n) &&
                              plan.scratch + table_bytes <= kBatchScratch;

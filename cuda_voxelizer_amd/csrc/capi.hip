@@ -153,6 +153,17 @@ vox_status get_slab_workspace(hipStream_t st, const SlabPlan& P, uint64_t n, voi
     return VOX_OK;
 }
 
+// Grids whose rows are no whole words need marker's scratch table, which a graph
+// must not hold (a later call may replace it): captured calls run direct.
+static bool ragged_marker(hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return cap == hipStreamCaptureStatusNone;
+}
+
 // One voxelization.  Algorithms: tile (binned, tile-owned writes; needs a
 // plan for this grid/layout), chunk (surface only, LDS word merging + global
 // atomics after a fill), marker (solid) and direct (one triangle per lane).
@@ -190,6 +201,7 @@ vox_status run(const vox_info* info, const float* d_tris, uint32_t* d_table, int
     else if (flags & VOX_FLAG_ALGO_CHUNK) algo = chunk_supported(G) ? CHUNK : DIRECT;
     else if (flags & VOX_FLAG_ALGO_MARKER) algo = have_marker ? MARKER : (have_plan ? TILE : DIRECT);
     else if (solid && prefer_direct_solid(info->n_triangles, G)) algo = DIRECT;
+    else if (solid && prefer_direct_ragged(info->n_triangles, G)) algo = DIRECT;
     else if (solid) algo = have_marker ? MARKER : (have_plan ? TILE : DIRECT);
     else algo = chunk_supported(G) ? CHUNK : (have_plan ? TILE : DIRECT);
     hipError_t e;
@@ -213,12 +225,16 @@ vox_status run(const vox_info* info, const float* d_tris, uint32_t* d_table, int
         if (e != hipSuccess) return hip_fail(e, "slab kernels launch");
         return VOX_OK;
     }
+    if (algo == MARKER && (G & 31u) && !ragged_marker(st)) algo = DIRECT;
     if (algo == MARKER) {
         e = launch_solid_marker(*info, d_tris, d_table, layout, accumulate, (unsigned long long*)d_offrow, st,
                                 tune_big(flags));
         if (e == hipErrorOutOfMemory && !algo_bits && have_plan && coarse_mesh(info->n_triangles, G)) {
             (void)hipGetLastError();  // tile needs no scratch table
             algo = TILE;
+        } else if (e == hipErrorOutOfMemory && (G & 31u)) {
+            (void)hipGetLastError();  // nor does direct
+            algo = DIRECT;
         } else {
             if (e != hipSuccess) return hip_fail(e, "marker kernels launch");
             return VOX_OK;
@@ -346,7 +362,7 @@ vox_status vox_solid_noalloc(const vox_info* info, const float* d_tris, uint32_t
     vox_status s = validate(info, d_tris, d_table, VOX_LAYOUT_LINEAR);
     if (s != VOX_OK) return s;
     const uint32_t G = info->gridsize[0];
-    if (!marker_supported(G, VOX_LAYOUT_LINEAR, false))
+    if (!marker_batch_supported(G, VOX_LAYOUT_LINEAR, false))
         return fail(VOX_ERR_UNSUPPORTED,
                     "vox_solid_noalloc: the grid edge must be a multiple of 32 between 32 and 16384 "
                     "(its fixed scratch holds only the spill counters and records)");

@@ -472,6 +472,31 @@ __device__ __forceinline__ void unblock_quad(const ItemDev& it, uint32_t t, bool
     }
 }
 
+// Rows that are no whole words (G not a multiple of 32; the scratch table's rows
+// are padded to words): 32 rows are G words of the linear table, from a word
+// boundary on, so a workgroup takes 32 rows into LDS, returns them to zero and
+// packs its G words.
+__device__ __forceinline__ void unblock_ragged(const ItemDev& it, uint32_t unit, uint32_t* rows) {
+    const uint32_t G = it.info.gridsize[0], rw = (G + 31u) >> 5, nrows = G * G, r0 = unit * 32u;
+    for (uint32_t i = threadIdx.x; i < 32u * rw; i += 256u) {
+        const uint32_t r = r0 + (i & 31u), w = i >> 5;  // four rows of a block are neighbours
+        uint32_t v = 0u;
+        if (r < nrows) {
+            uint32_t* p = it.scratch + blocked_word(G, w, r % G, r / G);
+            v = *p;
+            if (v) *p = 0u;
+        }
+        rows[(i & 31u) * rw + w] = v;
+    }
+    __syncthreads();
+    pack_rows(rows, rw, G, r0, it.table, [&](uint32_t* d, uint32_t v) {
+        if (!it.accumulate)
+            *d = v;
+        else if (v)
+            *d |= v;
+    });
+}
+
 __host__ __device__ inline bool unblock_vec(uint32_t G, const uint32_t* table) {
     return (G & 127u) == 0 && (((uintptr_t)table) & 15u) == 0;
 }
@@ -485,11 +510,17 @@ __global__ void __launch_bounds__(256) unblock_kernel(ItemDev one, ItemMap M) {
     }
     const ItemDev& it = M.items ? J.it : one;
     const uint32_t local = M.items ? J.local : blockIdx.x;
+    if (!FLAGS && (it.info.gridsize[0] & 31u)) {
+        __shared__ uint32_t rows[kRaggedWords];
+        unblock_ragged(it, local, rows);
+        return;
+    }
     unblock_quad<FLAGS>(it, local * 256u + threadIdx.x, FLAGS || unblock_vec(it.info.gridsize[0], it.table));
 }
 
 uint32_t unblock_units(uint32_t G, const uint32_t* table) {
     const uint64_t words = (uint64_t)G * G * G / 32u;
+    if (G & 31u) return (G * G + 31u) / 32u;
     return (uint32_t)((words / (unblock_vec(G, table) ? 16u : 4u) + 255u) / 256u);
 }
 
@@ -564,8 +595,7 @@ struct ScratchLease {
     ScratchLease& operator=(const ScratchLease&) = delete;
 };
 
-// Where words go through a blocked scratch table: linear rows of whole words, in
-// tables beyond the dense LDS merge; a call of few triangles at G <= 80 has too
+// Where words go through a blocked scratch table: the linear layout, in tables beyond the dense LDS merge; a call of few triangles at G <= 80 has too
 // few atomics for it (displaced sphere of 1,280 at 64^3 12.3 us, 13.3 blocked; a
 // soup of 100,003 at 64^3 76.6 and 27.9).  Measured with the rows of a linear
 // table as keys -> blocked (us per call): soup of 300,003 at 128^3 160 -> 45,
@@ -575,10 +605,12 @@ struct ScratchLease {
 // 1,048,576 at 1024^3 105 -> 76.  The flags save the row pass most of the
 // scratch table at 1024^3 and above (81,920 at 1024^3 103 -> 86, at 2048^3 529 ->
 // 485); at 512^3 and below setting them costs more than that (327,680 at 256^3
-// 41 without, 46 with).
+// 41 without, 46 with).  Grids whose rows are no whole words: torus of 26,866 at
+// 200^3 16.7 -> 14.2, soup of 100,000 at 201^3 89 -> 48, displaced sphere of 81,920
+// at 200^3 32 -> 18.
 bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles) {
     const uint64_t words = (uint64_t)G * G * G / 32u;
-    return layout == VOX_LAYOUT_LINEAR && (G & 31u) == 0 && G <= kBlockedGrid &&
+    return layout == VOX_LAYOUT_LINEAR && G <= ((G & 31u) ? kRaggedGrid : kBlockedGrid) &&
            words > (n_triangles < 16384u ? 16384u : (uint64_t)kHashCap);
 }
 
@@ -754,7 +786,7 @@ hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_
     const uint32_t G = info.gridsize[0];
     if (info.n_triangles && chunk_blocked(layout, G, info.n_triangles)) {
         hipError_t e = hipSuccess;
-        const uint64_t bytes = (uint64_t)G * G * G / 8u;
+        const uint64_t bytes = blocked_bytes(G);
         one.flagged = G > kUnflaggedGrid && unblock_vec(G, table) ? 1u : 0u;
         const uint64_t flags = one.flagged ? bytes / 256u : 0u;
         ScratchLease S(bytes + flags, stream);

@@ -23,7 +23,8 @@
 //                in-row part is a marker at G-1, the rest is recorded and
 //                XORed into the final table afterwards (word masks, atomics)
 //
-// G % 32 == 0 (rows are whole words); Morton: power-of-two G up to 4096.
+// Linear G % 32 == 0 (rows are whole words), other linear G up to 1024 through
+// rows padded to words; Morton: power-of-two G up to 4096.
 // Per-column arithmetic: vox_device.h (the reference CPU path bit for bit).
 #include "bricks.h"
 #include "columns.h"
@@ -101,8 +102,7 @@ __device__ __forceinline__ void column_run(uint32_t* __restrict__ table, int64_t
     if constexpr (REG) {
         marker_xor(H, region_row_key(RA.P, xm >> 5, (uint32_t)y, (uint32_t)z), 1u << (31u - (xm & 31u)), RA);
     } else {
-        const uint64_t idx = row + xm;
-        atomicXor(table + (idx >> 5), bit_mask(idx));
+        atomicXor(table + ((uint64_t)z * G + (uint32_t)y) * ((G + 31u) >> 5) + (xm >> 5), 0x80000000u >> (xm & 31u));
     }
     if (spills && xmax >= (int64_t)G && row + G < total_bits) {
         // bits row+G .. row+xmax, clipped to the table
@@ -327,6 +327,33 @@ __global__ void __launch_bounds__(256) suffix_scratch_rows4_kernel(uint32_t* __r
     const uint64_t wave = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) >> 6;
     const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) >> 6;
     suffix_rows4_range<true>(table, G, 0, nrows, wave, nwaves, markers);
+}
+
+// Rows that are no whole words (G not a multiple of 32): the markers lie in rows
+// padded to words.  32 rows are G words of the linear table, from a word
+// boundary on, so a workgroup takes 32 rows into LDS, returns them to zero,
+// takes their suffixes and packs its G words (or XORs them into the table).
+__global__ void __launch_bounds__(256) suffix_ragged_kernel(uint32_t* __restrict__ markers,
+                                                            uint32_t* __restrict__ table, uint32_t G, int accumulate) {
+    __shared__ uint32_t rows[kRaggedWords];
+    const uint32_t rw = (G + 31u) >> 5, r0 = blockIdx.x * 32u;
+    const uint64_t have = (uint64_t)G * G - r0;
+    const uint32_t n = (have < 32u ? (uint32_t)have : 32u) * rw;
+    uint32_t* __restrict__ src = markers + (uint64_t)r0 * rw;
+    for (uint32_t i = threadIdx.x; i < 32u * rw; i += 256u) {
+        const uint32_t v = i < n ? src[i] : 0u;
+        if (v) src[i] = 0u;
+        rows[i] = v;
+    }
+    __syncthreads();
+    tile_suffix(rows, rw, rw, 32u, [&](uint32_t r, uint32_t j, uint32_t fin) { rows[r * rw + j] = fin; });
+    __syncthreads();
+    pack_rows(rows, rw, G, r0, table, [&](uint32_t* d, uint32_t v) {
+        if (!accumulate)
+            *d = v;
+        else if (v)
+            *d ^= v;
+    });
 }
 
 // Batched form: work unit = kSuffixRows rows of one job's (linear, in-place)
@@ -643,6 +670,7 @@ static std::map<std::pair<int, hipStream_t>, MarkerBuffers> g_mws;
 
 bool marker_supported(uint32_t G, int layout, bool accumulate) {
     (void)accumulate;
+    if (layout == VOX_LAYOUT_LINEAR && (G & 31u)) return G > 32u && G <= kRaggedGrid;
     if (G < 32 || (G & 31u) || G > 16384u) return false;  // bit indices below 2^42 (spill records)
     if (layout == VOX_LAYOUT_MORTON) return (G & (G - 1)) == 0 && G <= 4096;
     return true;
@@ -685,8 +713,11 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     // 16-byte groups and the scratch table can be had; in place (zero-fill,
     // markers, suffix) otherwise
     bool stream_rows = layout == VOX_LAYOUT_LINEAR && !accumulate && rows4_ok(G, table);
-    bool in_place = layout == VOX_LAYOUT_LINEAR && !accumulate && !stream_rows;
-    const uint64_t table_bytes = (uint64_t)G * G * G / 8;
+    const bool ragged = (G & 31u) != 0;
+    bool in_place = layout == VOX_LAYOUT_LINEAR && !accumulate && !stream_rows && !ragged;
+    // the scratch table of the next multiple of 32, which the zero-fill covers whole (ragged rows use G^2 of its rows)
+    const uint32_t padded_g = (G + 31u) & ~31u;
+    const uint64_t table_bytes = (uint64_t)padded_g * padded_g * padded_g / 8;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
@@ -731,7 +762,9 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     }
     if (in_place) return launch_marker_in_place(info, tris, table, offrow, ws, stream, big);
     if (need_fill) {
-        e = launch_fill_zero(info, markers, stream);
+        vox_info padded = info;
+        padded.gridsize[0] = padded_g;
+        e = launch_fill_zero(padded, markers, stream);
         if (e != hipSuccess) return e;
     }
     const bool linear = layout == VOX_LAYOUT_LINEAR;
@@ -750,7 +783,9 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     if (info.n_triangles)
         solid_marker_kernel<false, false><<<marker_units(one), kMBlock, 0, stream>>>(one, none, ws, linear ? 1 : 0,
                                                                                     RegionArgs{});
-    if (stream_rows) {
+    if (ragged) {
+        suffix_ragged_kernel<<<(G * G + 31u) / 32u, 256, 0, stream>>>(markers, table, G, accumulate ? 1 : 0);
+    } else if (stream_rows) {
         const uint64_t nrows = (uint64_t)G * G;
         const uint64_t per = 64 / (G >> 7);
         uint64_t blocks = (nrows / per + 3) / 4;
@@ -921,7 +956,7 @@ uint32_t marker_block_units(ItemDev& it) {
 }
 uint32_t marker_row_units(uint32_t G) { return (uint32_t)(((uint64_t)G * G + kSuffixRows - 1) / kSuffixRows); }
 bool marker_batch_supported(uint32_t G, int layout, bool accumulate) {
-    return layout == VOX_LAYOUT_LINEAR && !accumulate && marker_supported(G, layout, accumulate);
+    return layout == VOX_LAYOUT_LINEAR && (G & 31u) == 0 && !accumulate && marker_supported(G, layout, accumulate);
 }
 
 // The tables are zero-filled beforehand (the batch's fill class).  m_blocks:

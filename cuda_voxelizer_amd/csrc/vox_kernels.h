@@ -28,7 +28,7 @@ hipError_t launch_tiled(const vox_info& info, const float* tris, uint32_t* table
                         unsigned long long* offrow, hipStream_t stream);
 
 bool marker_supported(uint32_t G, int layout, bool accumulate);
-bool marker_batch_supported(uint32_t G, int layout, bool accumulate);
+bool marker_batch_supported(uint32_t G, int layout, bool accumulate);  // the in-place form
 bool layout_convert_fast(uint32_t G);
 hipError_t launch_layout_convert(const uint32_t* src, uint32_t* dst, uint32_t G, bool to_morton, hipStream_t stream);
 uint64_t marker_ws_bytes();
@@ -96,6 +96,15 @@ inline bool coarse_mesh(uint64_t n_triangles, uint32_t G) {
 inline bool prefer_direct_solid(uint64_t n_triangles, uint32_t G) {
     return G <= 64u && n_triangles >= 4ull * G * G;
 }
+// And where rows are no whole words, on grids up to 128^3 from G^2 triangles on:
+// direct has a launch less (icosphere of 20,480 at 101^3 11.2 us, marker 13.3;
+// torus of 5,000 at 40^3 11.0 and 14.1).  Larger or coarser ones are marker's:
+// torus of 26,866 at 200^3 15.1 direct, 14.5 marker, 1,000 at 200^3 153 and 14,
+// icosphere of 1,280 at 100^3 42 and 15, displaced sphere of 327,680 at 700^3 355
+// and 72.
+inline bool prefer_direct_ragged(uint64_t n_triangles, uint32_t G) {
+    return (G & 31u) != 0 && G <= 128u && n_triangles >= (uint64_t)G * G;
+}
 hipError_t launch_fill_zero(const vox_info& info, uint32_t* table, hipStream_t stream);
 uint32_t fill_units(uint32_t G);
 uint32_t chunk_span(uint32_t G, uint64_t n_triangles);
@@ -113,7 +122,31 @@ hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_
                                 hipStream_t stream, uint32_t big = 0, int waves = 0);
 // Word w of row (y, z) in a blocked table: the 4 x 4 rows of a block lie together.
 __device__ __forceinline__ uint32_t blocked_word(uint32_t G, uint32_t w, uint32_t y, uint32_t z) {
-    return ((((z >> 2) * (G >> 2) + (y >> 2)) * (G >> 5) + w) << 4) | ((z & 3u) << 2) | (y & 3u);
+    return ((((z >> 2) * ((G + 3u) >> 2) + (y >> 2)) * ((G + 31u) >> 5) + w) << 4) | ((z & 3u) << 2) | (y & 3u);
+}
+inline uint64_t blocked_bytes(uint32_t G) {
+    const uint64_t nb = (G + 3u) >> 2;
+    return nb * nb * ((G + 31u) >> 5) * 64u;
+}
+// Grids whose rows are no whole words are packed from padded rows up to this one.
+constexpr uint32_t kRaggedGrid = 1024;
+constexpr uint32_t kRaggedWords = 32u * (kRaggedGrid / 32u);
+// 32 rows of rw words in LDS, from row r0 on -> their words of the linear table
+// (fewer at its end; bits from G on are zero in every row): put(word, value) for
+// each.  A word has bits of at most two rows (G > 32).
+template <class Put>
+__device__ __forceinline__ void pack_rows(const uint32_t* rows, uint32_t rw, uint32_t G, uint32_t r0,
+                                          uint32_t* __restrict__ table, Put&& put) {
+    const uint32_t total = (uint32_t)(((uint64_t)G * G * G + 31u) / 32u), w0 = r0 / 32u * G;
+    for (uint32_t k = threadIdx.x; k < G; k += blockDim.x) {
+        if (w0 + k >= total) return;
+        const uint32_t b = k * 32u, r = b / G, x = b - r * G;
+        const uint32_t* p = rows + r * rw + (x >> 5);
+        const uint32_t lo = p[0], hi = (x >> 5) + 1u < rw ? p[1] : 0u, s = x & 31u;
+        uint32_t v = s ? (lo << s) | (hi >> (32u - s)) : lo;
+        if (G - x < 32u && r < 31u) v |= rows[(r + 1u) * rw] >> (G - x);
+        put(table + w0 + k, v);
+    }
 }
 constexpr int kBlockedSpecs = kSpecBlocked + 1;  // what a batch's classes may be
 constexpr uint32_t kBlockedGrid = 2048;

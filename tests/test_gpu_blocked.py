@@ -135,3 +135,56 @@ def test_blocked_batch(oracle, gpu, use_graph):
             if not j.accumulate:
                 j.table.fill_(0x55)
     batch.close()
+
+
+# rows of 33 bits up to 31 words and 7 bits; 41^3 and 333^3 bits end inside a word, and
+# 41^2, 333^2 rows inside a workgroup's 32
+@pytest.mark.parametrize("grid", [33, 41, 63, 100, 127, 200, 333, 999])
+@pytest.mark.parametrize("solid", [False, True])
+def test_ragged_rows(oracle, gpu, grid, solid):
+    import cuda_voxelizer_amd as V
+    import torch
+    n = 17000 if grid < 100 else (3001 if grid < 500 else 400)
+    if solid:  # below G^2, from where small grids run direct
+        n = min(n, grid * grid - 1)
+    info, tris, d = _case(gpu, n, grid, grid, mu=-2.5)
+    words = V.table_words(grid)
+    if solid:
+        exp, count, _ = oracle.solid(oracle.info_from_bytes(info.as_bytes()), tris, morton=False)
+        call = V.voxelize_solid_table
+    else:
+        exp, call = _expected(oracle, info, tris), V.voxelize_surface
+    rng = np.random.default_rng(grid)
+    fill = rng.integers(0, 2**32, size=words, dtype=np.uint32)
+    guard = torch.full((words + 2,), 0x1234567, dtype=torch.int32, device=gpu)
+    t = guard[1:1 + words]
+    for _ in range(2):
+        call(info, d, table=t)
+        assert (_host(t) == exp).all()
+        t.copy_(torch.from_numpy(fill.view(np.int32)))
+        call(info, d, table=t, accumulate=True)
+        assert (_host(t) == (exp ^ fill if solid else exp | fill)).all()
+    assert int(guard[0]) == int(guard[-1]) == 0x1234567
+    if solid:
+        off = torch.zeros(1, dtype=torch.int64, device=gpu)
+        V.voxelize_solid_table(info, d, table=t, offrow=off)
+        assert int(off.item()) == count
+
+
+def test_ragged_solid_capture(oracle, gpu):
+    import cuda_voxelizer_amd as V
+    import torch
+    info, tris, d = _case(gpu, 500, 100, 3, mu=-2.0)
+    exp = oracle.solid(oracle.info_from_bytes(info.as_bytes()), tris, morton=False)[0]
+    table = torch.zeros(exp.size, dtype=torch.int32, device=gpu)
+    V.voxelize_solid_table(info, d, table=table)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        V.voxelize_solid_table(info, d, table=table)
+    for _ in range(3):
+        table.fill_(-1)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (_host(table) == exp).all()
