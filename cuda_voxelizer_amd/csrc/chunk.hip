@@ -416,7 +416,10 @@ __global__ void __launch_bounds__(256) fill_zero_kernel(ItemDev one, ItemMap M) 
 // 16-byte stores (VEC: rows of whole 16-byte groups, aligned tables), or else
 // one word in x of those 4 rows.  Work unit: 256 threads.
 // accumulate: bits are ORed into the table, only where there are any.
-// FLAGS: groups of 256 bytes whose flag is not set are zero and not read.
+// FLAGS: groups of 256 bytes whose flag is not set are zero and not read.  From
+// kStreamedGrid on the table and the scratch table are beyond the 256 MB of the
+// last cache each, and the rows must not push the scratch words out of it: 81,920
+// at 2048^3 488 -> 300 us, at 1536^3 270 -> 189; at 1152^3 that loses (128, 175).
 template <bool FLAGS>
 __device__ __forceinline__ void unblock_quad(const ItemDev& it, uint32_t t, bool vec) {
     const uint32_t G = it.info.gridsize[0], rw = G >> 5;
@@ -445,7 +448,9 @@ __device__ __forceinline__ void unblock_quad(const ItemDev& it, uint32_t t, bool
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const uint64_t d = (((uint64_t)(4u * bz + zl) * G + 4u * by + (uint32_t)u) * rw >> 2) + wq;
-            if (!it.accumulate) {
+            if (!it.accumulate && FLAGS && G >= kStreamedGrid) {
+                store_streaming(d4 + d, o[u]);
+            } else if (!it.accumulate) {
                 d4[d] = o[u];
             } else if (o[u].x | o[u].y | o[u].z | o[u].w) {
                 const uint4 p = d4[d];
@@ -601,10 +606,9 @@ struct ScratchLease {
 // table as keys -> blocked (us per call): soup of 300,003 at 128^3 160 -> 45,
 // 100,003 at 256^3 88 -> 67; displaced sphere of 81,920 at 256^3 31 -> 21, at
 // 512^3 65 -> 37, 327,680 at 512^3 92 -> 60; torus of 200,000 at 256^3 19 -> 14;
-// with flags: 81,920 at 1024^3 149 -> 86, at 2048^3 728 -> 485; torus of
+// with flags: 81,920 at 1024^3 149 -> 86, at 2048^3 728 -> 300; torus of
 // 1,048,576 at 1024^3 105 -> 76.  The flags save the row pass most of the
-// scratch table at 1024^3 and above (81,920 at 1024^3 103 -> 86, at 2048^3 529 ->
-// 485); at 512^3 and below setting them costs more than that (327,680 at 256^3
+// scratch table at 1024^3 and above (81,920 at 1024^3 103 -> 86); at 512^3 and below setting them costs more than that (327,680 at 256^3
 // 41 without, 46 with).  Grids whose rows are no whole words: torus of 26,866 at
 // 200^3 16.7 -> 14.2, soup of 100,000 at 201^3 89 -> 48, displaced sphere of 81,920
 // at 200^3 32 -> 18.

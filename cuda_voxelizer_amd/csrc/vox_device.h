@@ -31,6 +31,13 @@ __device__ __forceinline__ int iclamp(int f, int lo, int hi) {
     return lo > m ? lo : m;
 }
 
+// A 16-byte store that leaves the caches to what is read again.
+__device__ __forceinline__ void store_streaming(uint4* p, const uint4& v) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 q = {v.x, v.y, v.z, v.w};
+    __builtin_nontemporal_store(q, (u32x4*)p);
+}
+
 // One projection (XY, YZ or ZX) of the Schwarz-Seidel overlap test: three
 // edge half-planes a*u + b*v + d >= 0 in that projection's (u, v) coords.
 struct EdgeTest {

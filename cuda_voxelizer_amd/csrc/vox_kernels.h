@@ -151,6 +151,7 @@ __device__ __forceinline__ void pack_rows(const uint32_t* rows, uint32_t rw, uin
 constexpr int kBlockedSpecs = kSpecBlocked + 1;  // what a batch's classes may be
 constexpr uint32_t kBlockedGrid = 2048;
 constexpr uint32_t kUnflaggedGrid = 512;
+constexpr uint32_t kStreamedGrid = 1312;  // tables above 256 MiB
 bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles);
 uint32_t unblock_units(uint32_t G, const uint32_t* table);
 hipError_t launch_unblock_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, hipStream_t stream);

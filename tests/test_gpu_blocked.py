@@ -26,9 +26,9 @@ def _host(t):
 
 
 # 64: blocked from 16,384 triangles on; 96, 160: rows of 3 and 5 words; 544: 17
-# words, no flags; 640, 1024: flagged
+# words, no flags; 640 up: flagged; 1408: its rows are streamed
 @pytest.mark.parametrize("n,grid", [(16383, 64), (16384, 64), (3000, 96), (5000, 128), (7, 160), (20001, 256),
-                                    (4000, 544), (3000, 640), (900, 1024)])
+                                    (4000, 544), (3000, 640), (900, 1024), (300, 1408)])
 def test_blocked_tables(oracle, gpu, n, grid):
     import cuda_voxelizer_amd as V
     import torch
