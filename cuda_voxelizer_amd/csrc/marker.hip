@@ -93,7 +93,7 @@ __device__ __forceinline__ void marker_xor(MarkerLds<true>& H, uint32_t key, uin
 template <bool REG>
 __device__ __forceinline__ void column_run(uint32_t* __restrict__ table, int64_t xmax, int y, int z, uint32_t G,
                                            uint64_t total_bits, const MarkerWs& ws, unsigned long long& offrow,
-                                           bool spills, unsigned long long jobtag, MarkerLds<REG>& H,
+                                           bool spills, unsigned long long jobtag, bool blocked, MarkerLds<REG>& H,
                                            const RegionArgs& RA) {
     if (xmax < 0 || xmax >= (int64_t)G) offrow++;
     if (xmax < 0) return;
@@ -102,7 +102,9 @@ __device__ __forceinline__ void column_run(uint32_t* __restrict__ table, int64_t
     if constexpr (REG) {
         marker_xor(H, region_row_key(RA.P, xm >> 5, (uint32_t)y, (uint32_t)z), 1u << (31u - (xm & 31u)), RA);
     } else {
-        atomicXor(table + ((uint64_t)z * G + (uint32_t)y) * ((G + 31u) >> 5) + (xm >> 5), 0x80000000u >> (xm & 31u));
+        const uint64_t w = blocked ? (uint64_t)blocked_word(G, xm >> 5, (uint32_t)y, (uint32_t)z)
+                                   : ((uint64_t)z * G + (uint32_t)y) * ((G + 31u) >> 5) + (xm >> 5);
+        atomicXor(table + w, 0x80000000u >> (xm & 31u));
     }
     if (spills && xmax >= (int64_t)G && row + G < total_bits) {
         // bits row+G .. row+xmax, clipped to the table
@@ -163,7 +165,7 @@ __global__ void __launch_bounds__(kMBlock)
     unsigned long long offrow = 0;
     const auto run = [&](const SolidTri& S, int y, int z, float py, float pz) {
         column_run<REG>(table, column_xmax(S, info, py, pz), y, z, (uint32_t)G, total_bits, ws, offrow, spills != 0,
-                        jobtag, H, RA);
+                        jobtag, it.flagged != 0u, H, RA);
     };
     const uint64_t mine = first + (threadIdx.x >> lg);
     const int sub = (int)(threadIdx.x & ((1u << lg) - 1u)), step = 1 << lg;
@@ -335,6 +337,51 @@ __global__ void __launch_bounds__(256) suffix_scratch_rows4_kernel(uint32_t* __r
     suffix_rows4_range<true>(table, G, 0, nrows, wave, nwaves, markers);
 }
 
+// The suffix of the markers of 4 rows in y, word j of each in v, over the lanes
+// (j, consecutive) of the rows: lanes from `seg0` on, rw of them.
+__device__ __forceinline__ uint4 suffix_quad_rows(const uint4& v, bool act, uint32_t seg0, uint32_t j, uint32_t rw) {
+    const auto carry = [&](uint32_t c) -> uint32_t {
+        const unsigned long long par = __ballot(act && (__popc(c) & 1));
+        const unsigned long long above =
+            act && j + 1 < rw ? ((par >> (seg0 + j + 1)) & ((1ull << (rw - 1 - j)) - 1ull)) : 0ull;
+        return prefix_xor_up(c) ^ (0u - (uint32_t)(__popcll(above) & 1));
+    };
+    return make_uint4(carry(v.x), carry(v.y), carry(v.z), carry(v.w));
+}
+
+// Markers in a blocked scratch table (blocked_word) -> the rows of the linear
+// table, the scratch returned to zero; rows of at most 64 words.  A wave takes
+// two steps of 64 / rw row groups (4 rows in y of one z) at once.
+__global__ void __launch_bounds__(256) suffix_blocked_kernel(uint32_t* __restrict__ markers,
+                                                             uint32_t* __restrict__ table, uint32_t G) {
+    const uint32_t rw = G >> 5, per = 64u / rw, nb = G >> 2;
+    const uint32_t lane = (uint32_t)__lane_id(), r_in = lane / rw, j = lane - r_in * rw, seg0 = r_in * rw;
+    const uint32_t groups = nb * G;  // (z >> 2, y >> 2, z & 3)
+    const uint32_t g0 = (blockIdx.x * 4u + (threadIdx.x >> 6)) * 2u * per + r_in;
+    uint4* __restrict__ s4 = (uint4*)markers;
+    uint4 v[2];
+    bool act[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const uint32_t g = g0 + (uint32_t)u * per;
+        act[u] = r_in < per && g < groups;
+        const uint64_t i = ((uint64_t)(g >> 2) * rw + j) * 4u + (g & 3u);
+        v[u] = act[u] ? s4[i] : make_uint4(0u, 0u, 0u, 0u);
+        if (v[u].x | v[u].y | v[u].z | v[u].w) s4[i] = make_uint4(0u, 0u, 0u, 0u);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const uint4 o = suffix_quad_rows(v[u], act[u], seg0, j, rw);
+        if (!act[u]) continue;
+        const uint32_t g = g0 + (uint32_t)u * per, b = g >> 2, bz = b / nb, by = b - bz * nb;
+        uint32_t* d = table + ((uint64_t)(4u * bz + (g & 3u)) * G + 4u * by) * rw + j;
+        __builtin_nontemporal_store(o.x, d);
+        __builtin_nontemporal_store(o.y, d + rw);
+        __builtin_nontemporal_store(o.z, d + 2u * rw);
+        __builtin_nontemporal_store(o.w, d + 3u * rw);
+    }
+}
+
 // Rows that are no whole words (G not a multiple of 32): the markers lie in rows
 // padded to words.  32 rows are G words of the linear table, from a word
 // boundary on, so a workgroup takes 32 rows into LDS, returns them to zero,
@@ -391,7 +438,8 @@ __global__ void __launch_bounds__(256) suffix_jobs_kernel(ItemMap M) {
 // conversion of a finished table).
 // SUFFIX = true: `markers` is the library's scratch marker table, and the block
 // returns its rows to zero once loaded, so the next call needs no zero-fill.
-template <bool SUFFIX>
+// BLK: `markers` is blocked (Morton output, G 128 .. 1024, rz = 8).
+template <bool SUFFIX, bool BLK = false>
 __global__ void __launch_bounds__(256) marker_build_kernel(const uint32_t* markers, uint32_t* __restrict__ table,
                                                            uint32_t G, uint32_t rz, int layout, int accumulate) {
     extern __shared__ uint32_t tile[];  // [rz * 32 rows][rw + 1]: the pad word spreads rows over the banks
@@ -410,7 +458,37 @@ __global__ void __launch_bounds__(256) marker_build_kernel(const uint32_t* marke
     // lanes of one wave, and every wave runs the same number of iterations)
     const bool quads = (rw & 3u) == 0 && (((uintptr_t)markers) & 15u) == 0;
     const bool fused = SUFFIX && !linear && quads && rw <= 256u;
-    if (quads) {
+    if (BLK) {
+        // quads of 4 rows in y, their words in x in consecutive lanes
+        const uint32_t total4 = total >> 2, lane = (uint32_t)__lane_id(), j = lane & (rw - 1u), seg0 = lane - j;
+        uint4* c4 = (uint4*)const_cast<uint32_t*>(markers);
+        for (uint32_t i0 = threadIdx.x; i0 < total4; i0 += 256u * 8u) {
+            uint4 v[8];
+            uint64_t src[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const uint32_t i = i0 + 256u * (uint32_t)u, q = i / rw;  // q: z >> 2, y >> 2 (8), z & 3
+                const uint32_t by = (y0 >> 2) + ((q >> 2) & 7u), bz = (z0 >> 2) + (q >> 5);
+                src[u] = ((uint64_t)(bz * (G >> 2) + by) * rw + j) * 4u + (q & 3u);
+                v[u] = i < total4 ? c4[src[u]] : make_uint4(0u, 0u, 0u, 0u);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (v[u].x | v[u].y | v[u].z | v[u].w) c4[src[u]] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const uint32_t i = i0 + 256u * (uint32_t)u, q = i / rw;
+                const uint4 o = suffix_quad_rows(v[u], i < total4, seg0, j, rw);
+                if (i < total4) {
+                    uint32_t* d = tile + ((((q >> 5) * 4u + (q & 3u)) * 32u) + ((q >> 2) & 7u) * 4u) * ts + j;
+                    d[0] = o.x;
+                    d[ts] = o.y;
+                    d[2u * ts] = o.z;
+                    d[3u * ts] = o.w;
+                }
+            }
+        }
+    } else if (quads) {
         const uint32_t total4 = total >> 2, rq = rw >> 2, zq = 8u * rw;  // quads: all, per row, per z
         const uint32_t lane = (uint32_t)__lane_id(), j = lane % rq, seg0 = lane - j;
         const uint4* __restrict__ m4 = (const uint4*)markers;
@@ -485,7 +563,7 @@ __global__ void __launch_bounds__(256) marker_build_kernel(const uint32_t* marke
         }
     }
     __syncthreads();
-    if (SUFFIX && !fused) {
+    if (SUFFIX && !fused && !BLK) {
         tile_suffix(tile, ts, rw, nrows, [&](uint32_t r, uint32_t j, uint32_t fin) {
             if (linear) {
                 const uint64_t idx = ((uint64_t)(z0 + r / 32u) * G + y0 + (r & 31u)) * rw + j;
@@ -686,20 +764,25 @@ bool marker_supported(uint32_t G, int layout, bool accumulate) {
 // shared by up to 16 lanes each, as long as the job has at most 1280 workgroups
 // by that.  A coarse mesh (fewer than G^2/4 triangles) has triangles of many
 // columns: boxes of more than 8 (kMBigCols) are dealt, and further parts take
-// their share of them, up to about 1024 workgroups.  Measured (us per call;
+// their share of them, up to about 1024 workgroups.  In a batch the other jobs
+// fill the device, so its coarse jobs aim at 256 and its others share nothing.  Measured (us per call;
 // the triangles one after the other over a workgroup of 256 -> this):
 // icosphere 1,280 at 256^3 360 -> 17, 5,120 at 256^3 300 -> 18, 20,480 at
 // 576^3 349 -> 62; displaced sphere 20,480 at 512^3 277 -> 33, 81,920 at
 // 1024^3 346 -> 124 (the row pass takes 58 of it).  From G^2/4 on a limit of 8
 // loses: displaced sphere 20,480 at 256^3 20 with 32 columns, 26 with 8.
-static void marker_shape(ItemDev& it) {
+static void marker_shape(ItemDev& it, bool lone) {
     const uint64_t n = it.info.n_triangles;
     if (n == 0) return;
-    while (it.lg_split < 4u && n << (it.lg_split + 1u) <= 327680u) it.lg_split++;
-    if (!coarse_mesh(n, it.info.gridsize[0])) return;
+    const bool coarse = coarse_mesh(n, it.info.gridsize[0]);
+    if (lone)
+        while (it.lg_split < 4u && n << (it.lg_split + 1u) <= 327680u) it.lg_split++;
+    else
+        it.lg_split = coarse ? 3u : 0u;
+    if (!coarse) return;
     if (!it.big) it.big = kMBigColsCoarse;
     const uint64_t units = ((n << it.lg_split) + kMBlock - 1) / kMBlock;
-    const uint64_t p = 1024u / units;
+    const uint64_t p = (lone ? 1024u : 256u) / units;
     it.parts = p < 1u ? 1u : (p > 256u ? 256u : (uint32_t)p);
 }
 
@@ -785,12 +868,24 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     one.solid = 1;
     ItemDev fin = one;  // spills: into the final table
     fin.table = table;
-    marker_shape(one);
+    marker_shape(one, true);
+    // Blocked markers where a wave holds whole rows of words: a triangle's columns
+    // share lines, so dealt ones share requests, and the row pass returns fewer
+    // lines to zero.  Linear -> blocked (us per call): displaced sphere of 81,920
+    // at 1024^3 120 -> 70, 1,310,720 at 1024^3 124.5 -> 116 (Morton 145 -> 137),
+    // 20,480 at 512^3 31 -> 22 (Morton 34 -> 25), 327,680 at 2048^3 790 -> 475; at
+    // 768^3, whose rows of 24 words leave 16 lanes of a wave idle, 65 -> 70; fine
+    // meshes into Morton tables up to 512^3 gain nothing (33.9, 34.4).
+    const bool pow2 = (G & (G - 1u)) == 0 && G >= 128u;
+    one.flagged = pow2 && ((stream_rows && G <= 2048u) || (!linear && G <= 1024u && (G > 512u || coarse_mesh(info.n_triangles, G)))) ? 1u : 0u;
     if (info.n_triangles)
         solid_marker_kernel<false, false><<<marker_units(one), kMBlock, 0, stream>>>(one, none, ws, linear ? 1 : 0,
                                                                                     RegionArgs{});
     if (ragged) {
         suffix_ragged_kernel<<<(G * G + 31u) / 32u, 256, 0, stream>>>(markers, table, G, accumulate ? 1 : 0);
+    } else if (stream_rows && one.flagged) {
+        const uint32_t groups = (G >> 2) * G, step = 8u * (64u / (G >> 5));  // row groups of a workgroup
+        suffix_blocked_kernel<<<(groups + step - 1u) / step, 256, 0, stream>>>(markers, table, G);
     } else if (stream_rows) {
         const uint64_t nrows = (uint64_t)G * G;
         const uint64_t per = 64 / (G >> 7);
@@ -800,8 +895,13 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     } else {
         const uint32_t rz = linear ? 1u : (G <= 1024u ? 8u : 2u);
         const uint32_t nblocks = (G / 32u) * (G / rz);
-        marker_build_kernel<true><<<nblocks, 256, 4ull * 32u * rz * (G / 32u + 1u), stream>>>(
-            markers, table, G, rz, layout, accumulate ? 1 : 0);
+        const size_t lds = 4ull * 32u * rz * (G / 32u + 1u);
+        if (one.flagged)
+            marker_build_kernel<true, true><<<nblocks, 256, lds, stream>>>(markers, table, G, rz, layout,
+                                                                          accumulate ? 1 : 0);
+        else
+            marker_build_kernel<true><<<nblocks, 256, lds, stream>>>(markers, table, G, rz, layout,
+                                                                    accumulate ? 1 : 0);
     }
     e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -882,7 +982,7 @@ hipError_t launch_marker_in_place(const vox_info& info, const float* tris, uint3
     one.offrow = offrow;
     one.layout = VOX_LAYOUT_LINEAR;
     one.solid = 1;
-    marker_shape(one);
+    marker_shape(one, true);
     if (info.n_triangles)
         solid_marker_kernel<false, false><<<marker_units(one), kMBlock, 0, stream>>>(one, none, ws, 1, RegionArgs{});
     if (rows4_ok(G, table)) {
@@ -957,7 +1057,7 @@ hipError_t launch_solid_marker_static(const vox_info& info, const float* tris, u
 // ---- batched form (linear layout, no accumulation: in place) -------------------
 uint64_t marker_ws_bytes() { return 256 + 16ull * kSpillCap; }
 uint32_t marker_block_units(ItemDev& it) {
-    marker_shape(it);
+    marker_shape(it, false);
     return marker_units(it);
 }
 uint32_t marker_row_units(uint32_t G) { return (uint32_t)(((uint64_t)G * G + kSuffixRows - 1) / kSuffixRows); }

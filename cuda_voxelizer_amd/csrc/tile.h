@@ -48,7 +48,7 @@ struct ItemDev {
     uint32_t big;        // chunk: voxel boxes above this are shared by the workgroup; marker: columns
                          // above this (0: the built-in threshold)
     uint32_t lg_split;   // chunk, marker: 2^lg_split lanes share a triangle, so a workgroup takes 256 >> lg_split
-    uint32_t flagged;    // chunk: the blocked scratch table has flags before it
+    uint32_t flagged;    // chunk: the blocked scratch table has flags before it; marker: the markers' table is blocked
 };
 
 // Work mapping of one launch: a single job passed by value (items == nullptr)
