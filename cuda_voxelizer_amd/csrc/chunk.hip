@@ -627,13 +627,17 @@ uint32_t fill_units(uint32_t G) {
 
 // Chunks per workgroup.  A table of at most kHashCap words is merged densely
 // in LDS, and every workgroup that touches it flushes up to all its words to
-// the same few addresses: such jobs give each workgroup several chunks (while
-// keeping at least 64 workgroups per job) to cut those atomics.
-uint32_t chunk_span(uint32_t G, uint64_t n_triangles) {
+// the same few addresses (16 of them a request): such jobs give each workgroup
+// several chunks to cut those atomics, while keeping at least 512 workgroups of a
+// lone call, or 128 of a batch's job.  With 64 a workgroup's chain of chunks was
+// what the call lasted (us per call, 64 -> this): soup of 269,272 at 32^3 141 ->
+// 28, torus of 100,000 at 32^3 30 -> 15; 13 mixed meshes in a batch 203 -> 157 (161
+// with 512).
+uint32_t chunk_span(uint32_t G, uint64_t n_triangles, bool lone) {
     const uint64_t words = ((uint64_t)G * G * G + 31) / 32;
     if (words > (uint64_t)kHashCap) return 1u;
     const uint64_t chunks = (n_triangles + kChunk - 1) / kChunk;
-    const uint64_t s = chunks / 64;
+    const uint64_t s = chunks / (lone ? 512u : 128u);
     return s < 1 ? 1u : (s > 16 ? 16u : (uint32_t)s);
 }
 
@@ -717,9 +721,19 @@ static ItemDev single_job(const vox_info& info, const float* tris, uint32_t* tab
     one.tris = tris;
     one.table = table;
     one.layout = layout;
-    one.span = chunk_span(info.gridsize[0], info.n_triangles);
+    one.span = chunk_span(info.gridsize[0], info.n_triangles, true);
     one.parts = 1;
     return one;
+}
+
+// Voxel boxes above this are queued (0: the built-in rule): 16 voxels in a coarse
+// mesh of few triangles, whose workgroups would wait for their largest boxes; 64
+// in a coarser one of more (81,920 at 1024^3: 165 us at 256 voxels, 150 at 64; at
+// 512^3 66 and 80).
+uint32_t chunk_big(uint32_t G, uint64_t n) {
+    const uint64_t g2 = (uint64_t)G * G;
+    if (n == 0 || 8ull * n >= 5ull * g2) return 0u;
+    return n <= 32768u ? 16u : (8u * n < g2 ? 64u : 0u);
 }
 
 // The work shape of a lone call.  A mesh of few triangles must still give every
@@ -741,16 +755,15 @@ static void chunk_shape(ItemDev& one) {
     if (one.span > 1u || n == 0) return;
     const uint32_t top = one.layout == VOX_LAYOUT_MORTON ? 3u : 4u;
     one.lg_split = 0;
-    while (one.lg_split < top && n << (one.lg_split + 1u) <= 327680u) one.lg_split++;
+    // (dense tables: fewer workgroups, each of which flushes the whole table)
+    const uint64_t lanes = G * G * G / 32u <= (uint64_t)kHashCap ? 65536u : 327680u;
+    while (one.lg_split < top && n << (one.lg_split + 1u) <= lanes) one.lg_split++;
     if (8ull * n < 5ull * G * G) {
         const uint64_t units = ((n << one.lg_split) + kChunk - 1) / kChunk;
         uint64_t p = 2048u / units;
         if (p > G * G / (2u * n)) p = G * G / (2u * n);
         one.parts = p < 1u ? 1u : (p > 16u ? 16u : (uint32_t)p);
-        if (!one.big && n <= 32768u)
-            one.big = 16u;
-        else if (!one.big && 8u * n < G * G)
-            one.big = 64u;  // 81,920 at 1024^3: 165 us at 256 voxels, 150 at 64; at 512^3 66 and 80
+        if (!one.big) one.big = chunk_big((uint32_t)G, n);
     } else {
         one.parts = one.lg_split <= 1u && n <= 262144u ? 2u : 1u;
     }

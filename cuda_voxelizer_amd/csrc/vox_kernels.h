@@ -107,8 +107,9 @@ inline bool prefer_direct_ragged(uint64_t n_triangles, uint32_t G) {
 }
 hipError_t launch_fill_zero(const vox_info& info, uint32_t* table, hipStream_t stream);
 uint32_t fill_units(uint32_t G);
-uint32_t chunk_span(uint32_t G, uint64_t n_triangles);
+uint32_t chunk_span(uint32_t G, uint64_t n_triangles, bool lone);
 uint32_t chunk_parts(uint32_t G, uint64_t n_triangles);
+uint32_t chunk_big(uint32_t G, uint64_t n_triangles);
 uint32_t chunk_units(uint64_t n_triangles, uint32_t span, uint32_t parts, uint32_t lg_split = 0);
 hipError_t launch_fill_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, hipStream_t stream);
 // What a chunk kernel instantiation knows of its jobs' layout: nothing, linear
