@@ -59,17 +59,23 @@ typedef enum vox_status {
                                     it the call defines every word of the table
                                     (the zero-fill is fused into the kernels). */
 /* Algorithm selection (at most one; default: the library's choice per grid,
-   layout and mode -- chunk for surface; for solid, tile when the mesh has fewer
-   than G^2/4 triangles (large triangles), direct when it has at least 4 G^2 at
-   G <= 64, marker otherwise).  All algorithms give identical tables. */
+   layout and mode -- chunk for surface; for solid, direct when the mesh has at
+   least 4 G^2 triangles at G <= 64, or G^2 at G <= 128 with G % 32 != 0, marker
+   otherwise).  All algorithms give identical tables.  Per device and stream the
+   library keeps scratch tables of up to G^3/8 bytes (rows rounded up to words)
+   for linear surfaces up to 2048^3 and for solids; a linear surface call whose
+   stream is being captured, or that cannot have one, works in the caller's
+   table. */
 #define VOX_FLAG_ALGO_DIRECT 0x2u /* one triangle per lane, global atomics per word */
 #define VOX_FLAG_ALGO_TILE 0x4u   /* triangles binned to output tiles; one workgroup
                                     builds each tile in LDS and writes it once */
 #define VOX_FLAG_ALGO_CHUNK 0x8u  /* surface only: one workgroup per chunk of
                                     consecutive triangles merges words in an LDS
-                                    hash, then one atomicOr per distinct word */
-#define VOX_FLAG_ALGO_MARKER 0x10u /* solid only (G % 32 == 0, G <= 16384; Morton:
-                                    power of two up to 4096; otherwise tile): one
+                                    hash, then one atomicOr per distinct word, into
+                                    the table or a scratch table of its words */
+#define VOX_FLAG_ALGO_MARKER 0x10u /* solid only (G % 32 == 0, G <= 16384, or any G of
+                                    33..1024 not captured; Morton: power of two up
+                                    to 4096; otherwise tile or direct): one
                                     atomicXor marker per hit column at its run end
                                     in a zeroed bit table (the output itself for
                                     the linear layout), then every row becomes the
