@@ -285,7 +285,7 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE || (SPEC != kSpecAny 
     const int lg = SPLIT ? (int)it.lg_split : 0;
     const uint32_t per = (uint32_t)kChunk >> lg;
     uint32_t part = 0, unit = local;
-    if (!LOOP && parts > 1u) {
+    if (parts > 1u) {  // in the looping form too: its launch may hold jobs of either kind
         const uint32_t units = (uint32_t)((n + per - 1) / per);
         part = unit / units;
         unit -= part * units;
