@@ -410,12 +410,17 @@ __global__ void __launch_bounds__(256) fill_zero_kernel(ItemDev one, ItemMap M) 
     }
 }
 
+__device__ __forceinline__ void table_or(uint32_t* p, uint32_t v) {
+    if (v) atomicOr(p, v);
+}
+
 // Blocked scratch table -> rows of the linear table (G a multiple of 32); the
 // scratch words that held bits return to zero.  A thread takes 4 words in x of
 // the 4 rows in y of one z: four 16-byte loads, a transpose in registers, four
 // 16-byte stores (VEC: rows of whole 16-byte groups, aligned tables), or else
 // one word in x of those 4 rows.  Work unit: 256 threads.
-// accumulate: bits are ORed into the table, only where there are any.
+// accumulate: bits are ORed into the table, only where there are any, and
+// atomically: other calls, on other streams, may be adding to the table.
 // FLAGS: groups of 256 bytes whose flag is not set are zero and not read.  From
 // kStreamedGrid on the table and the scratch table are beyond the 256 MB of the
 // last cache each, and the rows must not push the scratch words out of it: 81,920
@@ -452,9 +457,12 @@ __device__ __forceinline__ void unblock_quad(const ItemDev& it, uint32_t t, bool
                 store_streaming(d4 + d, o[u]);
             } else if (!it.accumulate) {
                 d4[d] = o[u];
-            } else if (o[u].x | o[u].y | o[u].z | o[u].w) {
-                const uint4 p = d4[d];
-                d4[d] = make_uint4(p.x | o[u].x, p.y | o[u].y, p.z | o[u].z, p.w | o[u].w);
+            } else {
+                uint32_t* p = (uint32_t*)(d4 + d);
+                table_or(p, o[u].x);
+                table_or(p + 1, o[u].y);
+                table_or(p + 2, o[u].z);
+                table_or(p + 3, o[u].w);
             }
         }
         return;
@@ -472,8 +480,8 @@ __device__ __forceinline__ void unblock_quad(const ItemDev& it, uint32_t t, bool
         const uint64_t d = ((uint64_t)(4u * bz + zl) * G + 4u * by + (uint32_t)u) * rw + w;
         if (!it.accumulate)
             it.table[d] = o[u];
-        else if (o[u])
-            it.table[d] |= o[u];
+        else
+            table_or(it.table + d, o[u]);
     }
 }
 
@@ -497,8 +505,8 @@ __device__ __forceinline__ void unblock_ragged(const ItemDev& it, uint32_t unit,
     pack_rows(rows, rw, G, r0, it.table, [&](uint32_t* d, uint32_t v) {
         if (!it.accumulate)
             *d = v;
-        else if (v)
-            *d |= v;
+        else
+            table_or(d, v);
     });
 }
 

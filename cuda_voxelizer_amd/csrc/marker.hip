@@ -385,7 +385,8 @@ __global__ void __launch_bounds__(256) suffix_blocked_kernel(uint32_t* __restric
 // Rows that are no whole words (G not a multiple of 32): the markers lie in rows
 // padded to words.  32 rows are G words of the linear table, from a word
 // boundary on, so a workgroup takes 32 rows into LDS, returns them to zero,
-// takes their suffixes and packs its G words (or XORs them into the table).
+// takes their suffixes and packs its G words (or XORs them into the table,
+// atomically: other calls, on other streams, may be adding to it).
 __global__ void __launch_bounds__(256) suffix_ragged_kernel(uint32_t* __restrict__ markers,
                                                             uint32_t* __restrict__ table, uint32_t G, int accumulate) {
     __shared__ uint32_t rows[kRaggedWords];
@@ -405,7 +406,7 @@ __global__ void __launch_bounds__(256) suffix_ragged_kernel(uint32_t* __restrict
         if (!accumulate)
             *d = v;
         else if (v)
-            *d ^= v;
+            atomicXor(d, v);
     });
 }
 

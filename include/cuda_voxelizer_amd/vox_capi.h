@@ -57,7 +57,12 @@ typedef enum vox_status {
 #define VOX_FLAG_ACCUMULATE 0x1u /* OR (surface) / XOR (solid) into the table's
                                     current contents, like the reference; without
                                     it the call defines every word of the table
-                                    (the zero-fill is fused into the kernels). */
+                                    (the zero-fill is fused into the kernels).
+                                    Calls that accumulate into one table may overlap
+                                    (streams) for surfaces by the default, chunk and
+                                    direct algorithms and for solids by direct or
+                                    with G % 32 != 0: they add atomically.  The
+                                    others rewrite whole words: order them. */
 /* Algorithm selection (at most one; default: the library's choice per grid,
    layout and mode -- chunk for surface; for solid, direct when the mesh has at
    least 4 G^2 triangles at G <= 64, or G^2 at G <= 128 with G % 32 != 0, marker
