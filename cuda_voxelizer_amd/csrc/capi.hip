@@ -153,15 +153,16 @@ vox_status get_slab_workspace(hipStream_t st, const SlabPlan& P, uint64_t n, voi
     return VOX_OK;
 }
 
-// Grids whose rows are no whole words need marker's scratch table, which a graph
-// must not hold (a later call may replace it): captured calls run direct.
-static bool ragged_marker(hipStream_t st) {
+// Whether calls on a stream are being recorded into a graph.  A graph must not
+// hold a scratch table (a later, larger call replaces it, and eager calls on the
+// stream use it between the replays).
+static bool captured(hipStream_t st) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
         (void)hipGetLastError();
-        return false;
+        return true;  // the null stream beside a capture: nothing shared is touched
     }
-    return cap == hipStreamCaptureStatusNone;
+    return cap != hipStreamCaptureStatusNone;
 }
 
 // One voxelization.  Algorithms: tile (binned, tile-owned writes; needs a
@@ -169,7 +170,8 @@ static bool ragged_marker(hipStream_t st) {
 // atomics after a fill), marker (solid) and direct (one triangle per lane).
 // Without an explicit flag: chunk for surface; direct for a very fine solid
 // mesh on a small grid, marker for the others (tile where a coarse mesh cannot
-// have marker's scratch table); direct when none fits.
+// have marker's scratch table; under capture in the caller's table, or direct where
+// that form does not exist); direct when none fits.
 vox_status run(const vox_info* info, const float* d_tris, uint32_t* d_table, int layout, unsigned flags,
                uint64_t* d_offrow, void* stream, bool solid) {
     vox_status s = validate(info, d_tris, d_table, layout);
@@ -225,7 +227,14 @@ vox_status run(const vox_info* info, const float* d_tris, uint32_t* d_table, int
         if (e != hipSuccess) return hip_fail(e, "slab kernels launch");
         return VOX_OK;
     }
-    if (algo == MARKER && (G & 31u) && !ragged_marker(st)) algo = DIRECT;
+    if (algo == MARKER && captured(st)) {
+        if (marker_batch_supported(G, layout, accumulate)) {
+            e = launch_solid_marker_captured(*info, d_tris, d_table, (unsigned long long*)d_offrow, st, tune_big(flags));
+            if (e != hipSuccess) return hip_fail(e, "marker kernels launch (captured)");
+            return VOX_OK;
+        }
+        algo = DIRECT;
+    }
     if (algo == MARKER) {
         e = launch_solid_marker(*info, d_tris, d_table, layout, accumulate, (unsigned long long*)d_offrow, st,
                                 tune_big(flags));

@@ -1027,6 +1027,45 @@ __global__ void __launch_bounds__(64) clear_counters_kernel(unsigned* misc, int 
 
 size_t static_scratch_bytes() { return kStaticScratchBytes; }
 
+// ---- captured calls ------------------------------------------------------------
+// A call that is recorded into a graph takes the in-place form, whose only
+// workspace is the spill counters and records.  The graph holds their address, so
+// they are not those of the stream's eager calls and are never replaced or freed:
+// one allocation of 1 MB for each stream that captures.  The counters are cleared
+// by a kernel of the graph, as eager calls and replays may have ended anywhere.
+static std::map<std::pair<int, hipStream_t>, void*> g_capture_ws;
+
+hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris, uint32_t* table,
+                                        unsigned long long* offrow, hipStream_t stream, uint32_t big) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    void* p = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(g_mws_mutex);
+        void*& w = g_capture_ws[{dev, stream}];
+        if (!w) {
+            // an allocation is no stream operation; only the default capture mode forbids it
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            e = hipThreadExchangeStreamCaptureMode(&mode);
+            if (e != hipSuccess) return e;
+            e = hipMalloc(&w, kStaticScratchBytes);
+            const hipError_t e2 = hipThreadExchangeStreamCaptureMode(&mode);
+            if (e != hipSuccess) {
+                w = nullptr;
+                return e;
+            }
+            if (e2 != hipSuccess) return e2;
+        }
+        p = w;
+    }
+    const MarkerWs ws{(unsigned*)p, (unsigned long long*)((char*)p + 256)};
+    clear_counters_kernel<<<1, 64, 0, stream>>>(ws.misc, 64);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return launch_marker_in_place(info, tris, table, offrow, ws, stream, big);
+}
+
 hipError_t static_scratch_init(int device, void** out) {
     if (device < 0 || device >= kMaxStaticDevices) return hipErrorInvalidDevice;
     std::lock_guard<std::mutex> lock(g_static_mutex);

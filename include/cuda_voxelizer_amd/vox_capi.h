@@ -70,7 +70,10 @@ typedef enum vox_status {
    library keeps scratch tables of up to G^3/8 bytes (rows rounded up to words)
    for linear surfaces up to 2048^3 and for solids; a linear surface call whose
    stream is being captured, or that cannot have one, works in the caller's
-   table. */
+   table.  A captured marker call holds none either: linear, non-accumulating
+   ones on G % 32 == 0 work in the caller's table (the graph holds 1 MB of
+   counters and records that belong to the capture stream, so graphs captured on
+   one stream must not replay at the same time), the others run direct. */
 #define VOX_FLAG_ALGO_DIRECT 0x2u /* one triangle per lane, global atomics per word */
 #define VOX_FLAG_ALGO_TILE 0x4u   /* triangles binned to output tiles; one workgroup
                                     builds each tile in LDS and writes it once */
@@ -79,8 +82,8 @@ typedef enum vox_status {
                                     hash, then one atomicOr per distinct word, into
                                     the table or a scratch table of its words */
 #define VOX_FLAG_ALGO_MARKER 0x10u /* solid only (G % 32 == 0, G <= 16384, or any G of
-                                    33..1024 not captured; Morton: power of two up
-                                    to 4096; otherwise tile or direct): one
+                                    33..1024; Morton: power of two up to 4096;
+                                    otherwise tile or direct): one
                                     atomicXor marker per hit column at its run end
                                     in a zeroed bit table (the output itself for
                                     the linear layout), then every row becomes the
