@@ -26,11 +26,8 @@
 #include "raster.h"
 #include "region.h"
 #include "rows.h"
+#include "scratch.h"
 #include "vox_kernels.h"
-
-#include <map>
-#include <mutex>
-#include <utility>
 
 #pragma clang fp contract(off)
 
@@ -546,68 +543,6 @@ hipError_t launch_unblock_jobs(const ItemDev& one, const ItemMap& M, uint32_t un
     return hipGetLastError();
 }
 
-// A stream's blocked scratch table of at least `bytes` bytes, all zero between
-// calls: grow-only, at most the table's size
-// and its flags (1 GB + 4 MB, kBlockedGrid).  It is the holder's until the
-// lease ends, so that two threads' calls on one stream do not mix their
-// launches.  words is null when there is none: while the stream is being
-// captured (a later call may replace the buffer that the graph would hold), or
-// without memory.  clean() says that all launches are queued that leave it zero;
-// without it the next holder zero-fills it.
-struct SurfaceScratch {
-    void* ptr = nullptr;
-    uint64_t bytes = 0;
-    bool dirty = true;
-    std::mutex use;
-};
-static std::mutex g_scratch_mutex;
-static std::map<std::pair<int, hipStream_t>, SurfaceScratch> g_scratch;
-
-struct ScratchLease {
-    uint32_t* words = nullptr;
-    SurfaceScratch* b = nullptr;
-
-    ScratchLease(uint64_t bytes, hipStream_t stream) {
-        int dev = 0;
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(stream, &cap) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
-            (void)hipGetLastError();
-            return;
-        }
-        if (cap != hipStreamCaptureStatusNone) return;
-        {
-            std::lock_guard<std::mutex> lock(g_scratch_mutex);
-            b = &g_scratch[{dev, stream}];
-        }
-        b->use.lock();
-        hipError_t e = hipSuccess;
-        if (b->bytes < bytes) {
-            if (b->ptr) {
-                e = hipStreamSynchronize(stream);  // a previous call on this stream may still use it
-                if (e == hipSuccess) e = hipFree(b->ptr);
-            }
-            b->ptr = nullptr;
-            b->bytes = 0;
-            if (e == hipSuccess) e = hipMalloc(&b->ptr, bytes);
-            if (e == hipSuccess) b->bytes = bytes;
-            b->dirty = true;
-        }
-        if (e == hipSuccess && b->dirty) e = hipMemsetAsync(b->ptr, 0, b->bytes, stream);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            return;
-        }
-        words = (uint32_t*)b->ptr;
-        b->dirty = true;
-    }
-    void clean() { b->dirty = false; }
-    ~ScratchLease() {
-        if (b) b->use.unlock();
-    }
-    ScratchLease(const ScratchLease&) = delete;
-    ScratchLease& operator=(const ScratchLease&) = delete;
-};
-
 // Where words go through a blocked scratch table: the linear layout, in tables beyond the dense LDS merge; a call of few triangles at G <= 80 has too
 // few atomics for it (displaced sphere of 1,280 at 64^3 12.3 us, 13.3 blocked; a
 // soup of 100,003 at 64^3 76.6 and 27.9).  Measured with the rows of a linear
@@ -814,9 +749,9 @@ hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_
         const uint64_t bytes = blocked_bytes(G);
         one.flagged = G > kUnflaggedGrid && unblock_vec(G, table) ? 1u : 0u;
         const uint64_t flags = one.flagged ? bytes / 256u : 0u;
-        ScratchLease S(bytes + flags, stream);
-        if (S.words) {
-            one.scratch = S.words + flags / 4u;
+        ScratchLease S(stream);
+        if (uint32_t* words = S.table(bytes + flags)) {
+            one.scratch = words + flags / 4u;
             e = launch_chunk_jobs(one, none, chunk_units(info.n_triangles, one.span, one.parts, one.lg_split), false,
                                   stream, waves);
             if (e == hipSuccess) e = launch_unblock_jobs(one, none, unblock_units(G, table), stream);

@@ -30,6 +30,7 @@
 #include "columns.h"
 #include "jobs.h"
 #include "region.h"
+#include "scratch.h"
 #include "vox_device.h"
 #include "vox_host.h"
 #include "vox_kernels.h"
@@ -744,15 +745,6 @@ hipError_t launch_layout_convert(const uint32_t* src, uint32_t* dst, uint32_t G,
 }
 
 // ---- host ----------------------------------------------------------------------
-struct MarkerBuffers {
-    void* ws = nullptr;       // misc + spill records
-    void* scratch = nullptr;  // linear marker table (Morton output, accumulation)
-    uint64_t scratch_bytes = 0;
-    bool scratch_dirty = true;  // false once zero: the brick pass returns it to zero
-};
-static std::mutex g_mws_mutex;
-static std::map<std::pair<int, hipStream_t>, MarkerBuffers> g_mws;
-
 bool marker_supported(uint32_t G, int layout, bool accumulate) {
     (void)accumulate;
     if (layout == VOX_LAYOUT_LINEAR && (G & 31u)) return G > 32u && G <= kRaggedGrid;
@@ -795,6 +787,13 @@ static uint32_t marker_units(const ItemDev& it) {
 hipError_t launch_marker_in_place(const vox_info& info, const float* tris, uint32_t* table,
                                   unsigned long long* offrow, const MarkerWs& ws, hipStream_t stream, uint32_t big);
 
+static hipError_t marker_ws(ScratchLease& S, MarkerWs& ws) {
+    void* p = nullptr;
+    const hipError_t e = S.spills(&p);
+    ws = MarkerWs{(unsigned*)p, (unsigned long long*)((char*)p + 256)};
+    return e;
+}
+
 hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t* table, int layout,
                                bool accumulate, unsigned long long* offrow, hipStream_t stream, uint32_t big) {
     const uint32_t G = info.gridsize[0];
@@ -802,61 +801,18 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     // pass (suffix into the table, scratch back to zero) where rows are whole
     // 16-byte groups and the scratch table can be had; in place (zero-fill,
     // markers, suffix) otherwise
-    bool stream_rows = layout == VOX_LAYOUT_LINEAR && !accumulate && rows4_ok(G, table);
+    const bool stream_rows = layout == VOX_LAYOUT_LINEAR && !accumulate && rows4_ok(G, table);
     const bool ragged = (G & 31u) != 0;
-    bool in_place = layout == VOX_LAYOUT_LINEAR && !accumulate && !stream_rows && !ragged;
-    // the scratch table of the next multiple of 32, which the zero-fill covers whole (ragged rows use G^2 of its rows)
-    const uint32_t padded_g = (G + 31u) & ~31u;
-    const uint64_t table_bytes = (uint64_t)padded_g * padded_g * padded_g / 8;
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
+    const bool in_place = layout == VOX_LAYOUT_LINEAR && !accumulate && !stream_rows && !ragged;
+    const uint64_t table_bytes = (uint64_t)G * G * ((G + 31u) / 32u) * 4u;  // rows padded to words
+    ScratchLease S(stream);
     MarkerWs ws;
-    uint32_t* markers = table;
-    bool need_fill = in_place;
-    {
-        std::lock_guard<std::mutex> lock(g_mws_mutex);
-        MarkerBuffers& b = g_mws[{dev, stream}];
-        if (!b.ws) {
-            e = hipMalloc(&b.ws, 256 + 16ull * kSpillCap);
-            if (e == hipSuccess) e = hipMemset(b.ws, 0, 256);  // the counters start at zero
-            if (e != hipSuccess) return e;
-        }
-        if (!in_place && b.scratch_bytes < table_bytes) {
-            if (b.scratch) {
-                e = hipStreamSynchronize(stream);  // a previous call on this stream may still read it
-                if (e == hipSuccess) e = hipFree(b.scratch);
-                b.scratch = nullptr;
-                b.scratch_bytes = 0;
-                if (e != hipSuccess) return e;
-            }
-            e = hipMalloc(&b.scratch, table_bytes);
-            if (e == hipErrorOutOfMemory && stream_rows) {
-                (void)hipGetLastError();  // the in-place form needs no scratch table
-                b.scratch = nullptr;
-                stream_rows = false;
-                in_place = true;
-            } else if (e != hipSuccess) {
-                return e;
-            } else {
-                b.scratch_bytes = table_bytes;
-                b.scratch_dirty = true;
-            }
-        }
-        ws = MarkerWs{(unsigned*)b.ws, (unsigned long long*)((char*)b.ws + 256)};
-        if (!in_place) {
-            markers = (uint32_t*)b.scratch;
-            need_fill = b.scratch_dirty;
-            b.scratch_dirty = true;  // until this call's brick pass is queued
-        }
-    }
-    if (in_place) return launch_marker_in_place(info, tris, table, offrow, ws, stream, big);
-    if (need_fill) {
-        vox_info padded = info;
-        padded.gridsize[0] = padded_g;
-        e = launch_fill_zero(padded, markers, stream);
-        if (e != hipSuccess) return e;
-    }
+    hipError_t e = marker_ws(S, ws);
+    if (e != hipSuccess) return e;
+    uint32_t* markers = in_place ? table : S.table(table_bytes);
+    if (!markers && !stream_rows) return hipErrorOutOfMemory;
+    // the in-place form needs no scratch table
+    if (in_place || !markers) return launch_marker_in_place(info, tris, table, offrow, ws, stream, big);
     const bool linear = layout == VOX_LAYOUT_LINEAR;
     const ItemMap none{nullptr, nullptr, 1, 0};
     ItemDev one{};  // markers: into the scratch table
@@ -906,27 +862,9 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     }
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    {
-        std::lock_guard<std::mutex> lock(g_mws_mutex);
-        g_mws[{dev, stream}].scratch_dirty = false;  // every row of the G^3 table was read and cleared
-    }
+    S.clean();  // every row of the scratch table was read and cleared
     if (linear) spill_kernel<<<kSpillBlocks, 256, 0, stream>>>(fin, none, none, ws);
     return hipGetLastError();
-}
-
-static hipError_t marker_ws_for(hipStream_t stream, MarkerWs& ws) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> lock(g_mws_mutex);
-    MarkerBuffers& b = g_mws[{dev, stream}];
-    if (!b.ws) {
-        e = hipMalloc(&b.ws, 256 + 16ull * kSpillCap);
-        if (e == hipSuccess) e = hipMemset(b.ws, 0, 256);  // the counters start at zero
-        if (e != hipSuccess) return e;
-    }
-    ws = MarkerWs{(unsigned*)b.ws, (unsigned long long*)((char*)b.ws + 256)};
-    return hipSuccess;
 }
 
 // Region algorithm, solid: markers staged per region (phase 1), the build
@@ -940,8 +878,9 @@ hipError_t launch_solid_region(const vox_info& info, const float* tris, uint32_t
     RegionWs W;
     hipError_t e = region_workspace(P, (info.n_triangles + kMBlock - 1) / kMBlock, stream, W);
     if (e != hipSuccess) return e;
+    ScratchLease S(stream);
     MarkerWs ws;
-    e = marker_ws_for(stream, ws);
+    e = marker_ws(S, ws);
     if (e != hipSuccess) return e;
     const bool linear = layout == VOX_LAYOUT_LINEAR;
     const ItemMap none{nullptr, nullptr, 1, 0};
@@ -1033,6 +972,7 @@ size_t static_scratch_bytes() { return kStaticScratchBytes; }
 // they are not those of the stream's eager calls and are never replaced or freed:
 // one allocation of 1 MB for each stream that captures.  The counters are cleared
 // by a kernel of the graph, as eager calls and replays may have ended anywhere.
+static std::mutex g_capture_mutex;
 static std::map<std::pair<int, hipStream_t>, void*> g_capture_ws;
 
 hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris, uint32_t* table,
@@ -1042,7 +982,7 @@ hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris,
     if (e != hipSuccess) return e;
     void* p = nullptr;
     {
-        std::lock_guard<std::mutex> lock(g_mws_mutex);
+        std::lock_guard<std::mutex> lock(g_capture_mutex);
         void*& w = g_capture_ws[{dev, stream}];
         if (!w) {
             // an allocation is no stream operation; only the default capture mode forbids it

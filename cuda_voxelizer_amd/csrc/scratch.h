@@ -1,0 +1,40 @@
+// scratch.h -- the scratch memory that calls on one stream share.
+//
+// Per device and stream: a table for blocked surface words, blocked or linear
+// solid markers, all zero between calls, and the counters and records of spilled
+// runs (marker.hip), whose counters are zero between calls.  Both are worked on by
+// several launches of a call in a row, so a call holds the stream's scratch from
+// before its first launch until its last is queued; a second thread's call on the
+// stream waits for that, and the stream's order does the rest.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace voxamd {
+
+struct StreamScratch;
+
+class ScratchLease {
+   public:
+    explicit ScratchLease(hipStream_t stream);
+    ~ScratchLease();
+    ScratchLease(const ScratchLease&) = delete;
+    ScratchLease& operator=(const ScratchLease&) = delete;
+
+    // A zero table of at least `bytes` bytes; null while the stream is being
+    // captured (a later call may replace the table that the graph would hold) and
+    // without memory.
+    uint32_t* table(uint64_t bytes);
+    // All launches are queued that leave the table zero.  Without it the next
+    // holder zero-fills it.
+    void clean();
+    // marker_ws_bytes() bytes: counters and records of spilled runs.
+    hipError_t spills(void** out);
+
+   private:
+    hipStream_t stream_;
+    StreamScratch* s_ = nullptr;
+};
+
+}  // namespace voxamd
