@@ -875,10 +875,10 @@ hipError_t launch_solid_region(const vox_info& info, const float* tris, uint32_t
                                const RegionKnobs& K) {
     RegionPlan P;
     if (!make_region_plan(info.gridsize[0], layout, true, P, K)) return hipErrorInvalidValue;
+    ScratchLease S(stream);
     RegionWs W;
     hipError_t e = region_workspace(P, (info.n_triangles + kMBlock - 1) / kMBlock, stream, W);
     if (e != hipSuccess) return e;
-    ScratchLease S(stream);
     MarkerWs ws;
     e = marker_ws(S, ws);
     if (e != hipSuccess) return e;

@@ -33,6 +33,7 @@
 #include "vox_host.h"
 #include "raster.h"
 #include "scan.h"
+#include "scratch.h"
 #include <map>
 #include <mutex>
 
@@ -179,6 +180,7 @@ static hipError_t sort_triangles(const vox_info& info, const float* tris, float*
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     uint32_t *group_totals, *counts, *cursor, *keys;
+    const ScratchLease lease(stream);  // one call's launches at a time
     {
         std::lock_guard<std::mutex> lock(g_order_mutex);
         OrderBuffers& b = g_order[{dev, stream}];

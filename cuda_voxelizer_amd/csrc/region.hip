@@ -8,6 +8,7 @@
 // nothing are streamed as zeros without touching LDS.
 #include "bricks.h"
 #include "region.h"
+#include "scratch.h"
 #include "vox_kernels.h"
 
 #include <map>
@@ -322,6 +323,7 @@ hipError_t launch_surface_region(const vox_info& info, const float* tris, uint32
                                  bool accumulate, hipStream_t stream, uint32_t big, int waves, const RegionKnobs& K) {
     RegionPlan P;
     if (!make_region_plan(info.gridsize[0], layout, false, P, K)) return hipErrorInvalidValue;
+    const ScratchLease lease(stream);  // one call's launches at a time
     RegionWs W;
     hipError_t e = region_workspace(P, chunk_units(info.n_triangles, 1, 1), stream, W);
     if (e != hipSuccess) return e;
