@@ -15,7 +15,6 @@
 #include <map>
 #include <mutex>
 #include <string>
-#include <utility>
 
 #include "../../include/cuda_voxelizer_amd/vox_capi.h"
 #include "../../include/cuda_voxelizer_amd/voxelize.h"
@@ -76,14 +75,14 @@ struct Workspace {
 };
 
 static std::mutex g_ws_mutex;
-static std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
+static std::map<StreamKey, Workspace> g_ws;
 
 vox_status get_workspace(hipStream_t st, const TilePlan& P, uint64_t n, void** out, WorkspaceLayout* lay) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
+    StreamKey key;
+    hipError_t e = stream_key(st, key);
     if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
     std::lock_guard<std::mutex> lock(g_ws_mutex);
-    Workspace& W = g_ws[std::make_pair(dev, st)];
+    Workspace& W = g_ws[key];
     if (W.ptr == nullptr || (uint64_t)P.ntiles > W.tiles_cap || n > W.n_cap) {
         // counts are read in uint4 groups up to a multiple of 4096 by the scan
         const uint64_t need = ((uint64_t)P.ntiles + 4095) & ~4095ull;
@@ -121,14 +120,14 @@ struct SlabBuffer {
     SlabLayout L{};
 };
 static std::mutex g_slab_mutex;
-static std::map<std::pair<int, hipStream_t>, SlabBuffer> g_slab;
+static std::map<StreamKey, SlabBuffer> g_slab;
 
 vox_status get_slab_workspace(hipStream_t st, const SlabPlan& P, uint64_t n, void** out, SlabLayout* lay) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
+    StreamKey key;
+    hipError_t e = stream_key(st, key);
     if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
     std::lock_guard<std::mutex> lock(g_slab_mutex);
-    SlabBuffer& W = g_slab[std::make_pair(dev, st)];
+    SlabBuffer& W = g_slab[key];
     if (W.ptr == nullptr || !slab_layout_fits(P, n, W.L)) {
         const uint64_t tiles_cap = W.L.tiles_cap > (uint64_t)P.ntiles ? W.L.tiles_cap : (uint64_t)P.ntiles;
         uint64_t n_cap = W.L.n_cap > n ? W.L.n_cap : n;

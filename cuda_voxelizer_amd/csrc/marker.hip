@@ -37,7 +37,6 @@
 
 #include <map>
 #include <mutex>
-#include <utility>
 
 #pragma clang fp contract(off)
 
@@ -973,17 +972,17 @@ size_t static_scratch_bytes() { return kStaticScratchBytes; }
 // one allocation of 1 MB for each stream that captures.  The counters are cleared
 // by a kernel of the graph, as eager calls and replays may have ended anywhere.
 static std::mutex g_capture_mutex;
-static std::map<std::pair<int, hipStream_t>, void*> g_capture_ws;
+static std::map<StreamKey, void*> g_capture_ws;
 
 hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris, uint32_t* table,
                                         unsigned long long* offrow, hipStream_t stream, uint32_t big) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
+    StreamKey key;
+    hipError_t e = stream_key(stream, key);
     if (e != hipSuccess) return e;
     void* p = nullptr;
     {
         std::lock_guard<std::mutex> lock(g_capture_mutex);
-        void*& w = g_capture_ws[{dev, stream}];
+        void*& w = g_capture_ws[key];
         if (!w) {
             // an allocation is no stream operation; only the default capture mode forbids it
             hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;

@@ -170,20 +170,20 @@ struct OrderBuffers {
     bool dirty = true;
 };
 static std::mutex g_order_mutex;
-static std::map<std::pair<int, hipStream_t>, OrderBuffers> g_order;
+static std::map<StreamKey, OrderBuffers> g_order;
 
 static hipError_t sort_triangles(const vox_info& info, const float* tris, float* out, uint32_t* perm,
                                  hipStream_t stream) {
     const uint64_t n = info.n_triangles;
     const OrderGeom g = order_geom(info.gridsize[0]);
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
+    StreamKey key;
+    hipError_t e = stream_key(stream, key);
     if (e != hipSuccess) return e;
     uint32_t *group_totals, *counts, *cursor, *keys;
     const ScratchLease lease(stream);  // one call's launches at a time
     {
         std::lock_guard<std::mutex> lock(g_order_mutex);
-        OrderBuffers& b = g_order[{dev, stream}];
+        OrderBuffers& b = g_order[key];
         if (b.ptr == nullptr || n > b.n_cap || g.buckets > b.buckets_cap) {
             const uint64_t n_cap = n > b.n_cap ? n : b.n_cap;
             const uint32_t buckets_cap = g.buckets > b.buckets_cap ? g.buckets : b.buckets_cap;
@@ -220,7 +220,7 @@ static hipError_t sort_triangles(const vox_info& info, const float* tris, float*
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     std::lock_guard<std::mutex> lock(g_order_mutex);
-    g_order[{dev, stream}].dirty = false;
+    g_order[key].dirty = false;
     return hipSuccess;
 }
 

@@ -14,11 +14,11 @@
 #include <cstring>
 #include <map>
 #include <mutex>
-#include <utility>
 #include <string>
 
 #include "../../include/cuda_voxelizer_amd/vox_capi.h"
 #include "vox_device.h"
+#include "scratch.h"
 #include "vox_host.h"
 #include "vox_kernels.h"
 
@@ -210,7 +210,7 @@ static unsigned grid_for(uint64_t n) {
 
 // pinned staging for vox_upload_async (double buffered, per process)
 static std::mutex g_bbox_mutex;
-static std::map<std::pair<int, hipStream_t>, void*> g_bbox_ws;
+static std::map<StreamKey, void*> g_bbox_ws;
 static std::mutex g_up_mutex;
 static void* g_up_buf[2] = {nullptr, nullptr};
 static hipEvent_t g_up_ev[2] = {nullptr, nullptr};
@@ -230,11 +230,11 @@ vox_status vox_mesh_bbox(const float* d_vertices, uint64_t n_vertices, float* d_
     {
         // per (device, stream): the counter and the partial keys; the counter
         // starts at zero and the kernel's last block returns it there
-        int dev = 0;
-        hipError_t e = hipGetDevice(&dev);
+        StreamKey key;
+        hipError_t e = stream_key(st, key);
         if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
         std::lock_guard<std::mutex> lock(g_bbox_mutex);
-        void*& w = g_bbox_ws[{dev, st}];
+        void*& w = g_bbox_ws[key];
         if (!w) {
             e = hipMalloc(&w, 4u * (64u + 6u * kBboxBlocks));
             if (e == hipSuccess) e = hipMemset(w, 0, 4u * 64u);

@@ -13,7 +13,6 @@
 
 #include <map>
 #include <mutex>
-#include <utility>
 
 namespace voxamd {
 
@@ -246,19 +245,19 @@ struct RegionBuffer {
     uint64_t nreg_cap = 0, desc_cap = 0, scap = 0, scratch_words = 0, bytes = 0;
 };
 static std::mutex g_region_mutex;
-static std::map<std::pair<int, hipStream_t>, RegionBuffer> g_region;
+static std::map<StreamKey, RegionBuffer> g_region;
 
 static uint64_t align256(uint64_t b) { return (b + 255u) & ~255ull; }
 
 hipError_t region_workspace(const RegionPlan& P, uint64_t workgroups, hipStream_t stream, RegionWs& W) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
+    StreamKey key;
+    hipError_t e = stream_key(stream, key);
     if (e != hipSuccess) return e;
     const uint64_t need_nreg = P.nreg, need_desc = (uint64_t)P.nreg * P.dcap;
     const uint64_t need_stage = (workgroups ? workgroups : 1) * (uint64_t)P.slice;
     const uint64_t need_scratch = (uint64_t)P.nreg << P.lg;
     std::lock_guard<std::mutex> lock(g_region_mutex);
-    RegionBuffer& B = g_region[std::make_pair(dev, stream)];
+    RegionBuffer& B = g_region[key];
     if (!B.ptr || B.nreg_cap < need_nreg || B.desc_cap < need_desc || B.scap < need_stage ||
         B.scratch_words < need_scratch) {
         RegionBuffer nb;

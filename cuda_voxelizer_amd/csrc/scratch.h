@@ -12,7 +12,22 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <tuple>
+
 namespace voxamd {
+
+// What a stream's workspaces are kept under.  hipStreamPerThread is one handle for
+// a stream of each thread, so there the thread is part of the key (0 otherwise; a
+// thread's number is never given to another).
+struct StreamKey {
+    int device = 0;
+    hipStream_t stream = nullptr;
+    uint64_t thread = 0;
+    bool operator<(const StreamKey& o) const {
+        return std::tie(device, stream, thread) < std::tie(o.device, o.stream, o.thread);
+    }
+};
+hipError_t stream_key(hipStream_t stream, StreamKey& key);  // on the current device
 
 struct StreamScratch;
 

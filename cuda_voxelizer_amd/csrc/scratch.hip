@@ -1,9 +1,9 @@
 // scratch.hip -- the scratch memory that calls on one stream share (scratch.h).
 #include "scratch.h"
 
+#include <atomic>
 #include <map>
 #include <mutex>
-#include <utility>
 
 #include "vox_kernels.h"
 
@@ -17,18 +17,26 @@ struct StreamScratch {
     std::mutex use;
 };
 
+hipError_t stream_key(hipStream_t stream, StreamKey& key) {
+    static std::atomic<uint64_t> threads{0};
+    static thread_local const uint64_t thread = ++threads;
+    key.stream = stream;
+    key.thread = stream == hipStreamPerThread ? thread : 0;
+    return hipGetDevice(&key.device);
+}
+
 static std::mutex g_scratch_mutex;
-static std::map<std::pair<int, hipStream_t>, StreamScratch> g_scratch;
+static std::map<StreamKey, StreamScratch> g_scratch;
 
 ScratchLease::ScratchLease(hipStream_t stream) : stream_(stream) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) {
+    StreamKey key;
+    if (stream_key(stream, key) != hipSuccess) {
         (void)hipGetLastError();
         return;
     }
     {
         std::lock_guard<std::mutex> lock(g_scratch_mutex);
-        s_ = &g_scratch[{dev, stream}];
+        s_ = &g_scratch[key];
     }
     s_->use.lock();
 }
