@@ -33,7 +33,7 @@ __all__ = [
     "voxinfo_for_mesh", "VoxError", "VOX_LAYOUT_LINEAR", "VOX_LAYOUT_MORTON", "VOX_FLAG_ACCUMULATE",
     "VOX_FLAG_ALGO_DIRECT", "VOX_FLAG_ALGO_TILE", "VOX_FLAG_ALGO_CHUNK", "ALGOS", "BatchJob", "Batch",
     "mesh_bbox_device", "pack_triangles", "upload", "convert_layout", "count_voxels", "check_voxel",
-    "prepare_mesh", "sort_triangles",
+    "prepare_mesh", "sort_triangles", "release_scratch",
 ]
 
 ALGOS = tuple(ALGO_FLAGS)  # "auto", "direct", "tile", "chunk", "marker", "slab", "region"
@@ -410,6 +410,13 @@ def pack_triangles(vertices, faces, stream=None):
     if int(bad.item()):
         raise ValueError(f"{int(bad.item())} face indices out of range")
     return out
+
+
+def release_scratch(device=None) -> None:
+    """Free the scratch tables that the library keeps for the device's streams
+    (up to G^3/8 bytes each); the next call on a stream allocates anew."""
+    with _torch().cuda.device(device):
+        check(_capi.load().vox_release_scratch())
 
 
 def sort_triangles(info: VoxInfo, tris, stream=None, with_perm: bool = False):

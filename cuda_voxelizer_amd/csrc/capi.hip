@@ -243,7 +243,7 @@ vox_status run(const vox_info* info, const float* d_tris, uint32_t* d_table, int
         if (e == hipErrorOutOfMemory && !algo_bits && have_plan && coarse_mesh(info->n_triangles, G)) {
             (void)hipGetLastError();  // tile needs no scratch table
             algo = TILE;
-        } else if (e == hipErrorOutOfMemory && (G & 31u)) {
+        } else if (e == hipErrorOutOfMemory) {
             (void)hipGetLastError();  // nor does direct
             algo = DIRECT;
         } else {

@@ -39,8 +39,8 @@ class ScratchLease {
     ScratchLease& operator=(const ScratchLease&) = delete;
 
     // A zero table of at least `bytes` bytes; null while the stream is being
-    // captured (a later call may replace the table that the graph would hold) and
-    // without memory.
+    // captured (a later call may replace the table that the graph would hold),
+    // without memory, and where the device's tables would grow beyond their limit.
     uint32_t* table(uint64_t bytes);
     // All launches are queued that leave the table zero.  Without it the next
     // holder zero-fills it.
@@ -50,6 +50,7 @@ class ScratchLease {
 
    private:
     hipStream_t stream_;
+    int device_ = 0;
     StreamScratch* s_ = nullptr;
 };
 

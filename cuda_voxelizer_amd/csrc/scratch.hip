@@ -4,7 +4,9 @@
 #include <atomic>
 #include <map>
 #include <mutex>
+#include <vector>
 
+#include "vox_host.h"
 #include "vox_kernels.h"
 
 namespace voxamd {
@@ -14,19 +16,120 @@ struct StreamScratch {
     uint64_t bytes = 0;
     bool dirty = true;
     void* spills = nullptr;
+    bool recorded = false;  // a graph holds the spills: they are never freed
+    int holders = 0;    // leases that hold or await it
+    uint64_t last = 0;  // the device's count of leases at its last one
     std::mutex use;
 };
 
+// All streams' scratch.  A device's tables together stay below an eighth of its
+// memory (36 GB here: 36 streams at 2048^3), or are one stream's table: a call that
+// would go beyond has none, unless a stream of the device that has not had a call
+// for kIdle of the device's leases can give up its table -- a stream that was
+// destroyed, above all.  What a thread's own stream had (hipStreamPerThread) goes
+// once the thread has ended and another table grows.
+constexpr uint64_t kIdle = 64;
+struct ScratchPool {
+    std::mutex m;
+    std::map<StreamKey, StreamScratch> streams;
+    std::map<int, uint64_t> held, leases;  // of a device: bytes in tables, leases so far
+    std::vector<uint64_t> ended;           // threads
+};
+static ScratchPool& pool() {
+    static ScratchPool* p = new ScratchPool;  // threads may end after static objects have gone
+    return *p;
+}
+
+struct ThreadNumber {
+    uint64_t n;
+    ThreadNumber() {
+        static std::atomic<uint64_t> threads{0};
+        n = ++threads;
+    }
+    ~ThreadNumber() {
+        ScratchPool& P = pool();
+        std::lock_guard<std::mutex> lock(P.m);
+        P.ended.push_back(n);
+    }
+};
+
 hipError_t stream_key(hipStream_t stream, StreamKey& key) {
-    static std::atomic<uint64_t> threads{0};
-    static thread_local const uint64_t thread = ++threads;
     key.stream = stream;
-    key.thread = stream == hipStreamPerThread ? thread : 0;
+    key.thread = 0;
+    if (stream == hipStreamPerThread) {
+        static thread_local ThreadNumber thread;
+        key.thread = thread.n;
+    }
     return hipGetDevice(&key.device);
 }
 
-static std::mutex g_scratch_mutex;
-static std::map<StreamKey, StreamScratch> g_scratch;
+// Memory is allocated and freed in the relaxed capture mode: it touches no stream
+// that is being captured, and the default mode refuses it while any thread
+// captures one.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool set;
+    RelaxedCapture() : set(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+    ~RelaxedCapture() {
+        if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
+// Frees what an idle stream of the current device has, whose last call may still
+// run.  False if the device cannot be waited for.
+static bool give_back(ScratchPool& P, int device, StreamScratch& s) {
+    if (!s.table && (!s.spills || s.recorded)) return true;
+    if (hipDeviceSynchronize() != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (s.table) (void)hipFree(s.table);
+    P.held[device] -= s.bytes;
+    s.table = nullptr;
+    s.bytes = 0;
+    if (s.spills && !s.recorded) {
+        (void)hipFree(s.spills);
+        s.spills = nullptr;
+    }
+    s.dirty = true;
+    return true;
+}
+
+// Counts `bytes` instead of s.bytes among the device's tables, if they fit.
+static bool reserve(int device, StreamScratch& s, uint64_t bytes) {
+    size_t total = 0;
+    if (hipDeviceTotalMem(&total, device) != hipSuccess) return false;
+    ScratchPool& P = pool();
+    std::lock_guard<std::mutex> lock(P.m);
+    for (size_t i = 0; i < P.ended.size(); i++) {
+        const uint64_t n = P.ended[i];
+        bool left = false;
+        for (auto it = P.streams.begin(); it != P.streams.end();) {
+            const bool own = it->first.thread == n;
+            if (own && it->first.device == device && it->second.holders == 0 && give_back(P, device, it->second) &&
+                !it->second.spills) {
+                it = P.streams.erase(it);
+                continue;
+            }
+            left = left || own;
+            ++it;
+        }
+        if (!left) P.ended.erase(P.ended.begin() + (long)i--);
+    }
+    const uint64_t limit = total / 8, now = P.leases[device];
+    while (P.held[device] - s.bytes + bytes > limit && P.held[device] > s.bytes) {
+        auto idle = P.streams.end();
+        for (auto it = P.streams.begin(); it != P.streams.end(); ++it)
+            if (it->first.device == device && it->second.holders == 0 && it->second.table &&
+                now - it->second.last >= kIdle &&
+                (idle == P.streams.end() || it->second.last < idle->second.last))
+                idle = it;
+        if (idle == P.streams.end() || !give_back(P, device, idle->second)) return false;
+        if (!idle->second.spills) P.streams.erase(idle);
+    }
+    P.held[device] += bytes - s.bytes;
+    return true;
+}
 
 ScratchLease::ScratchLease(hipStream_t stream) : stream_(stream) {
     StreamKey key;
@@ -34,15 +137,22 @@ ScratchLease::ScratchLease(hipStream_t stream) : stream_(stream) {
         (void)hipGetLastError();
         return;
     }
+    device_ = key.device;
+    ScratchPool& P = pool();
     {
-        std::lock_guard<std::mutex> lock(g_scratch_mutex);
-        s_ = &g_scratch[key];
+        std::lock_guard<std::mutex> lock(P.m);
+        s_ = &P.streams[key];
+        s_->holders++;
+        s_->last = ++P.leases[device_];
     }
     s_->use.lock();
 }
 
 ScratchLease::~ScratchLease() {
-    if (s_) s_->use.unlock();
+    if (!s_) return;
+    s_->use.unlock();
+    std::lock_guard<std::mutex> lock(pool().m);
+    s_->holders--;
 }
 
 uint32_t* ScratchLease::table(uint64_t bytes) {
@@ -51,6 +161,8 @@ uint32_t* ScratchLease::table(uint64_t bytes) {
     hipError_t e = hipStreamIsCapturing(stream_, &cap);
     if (e == hipSuccess && cap != hipStreamCaptureStatusNone) return nullptr;
     if (e == hipSuccess && s_->bytes < bytes) {
+        const RelaxedCapture relaxed;
+        if (!reserve(device_, *s_, bytes)) return nullptr;
         if (s_->table) {
             e = hipStreamSynchronize(stream_);  // a previous call on this stream may still use it
             if (e == hipSuccess) e = hipFree(s_->table);
@@ -59,12 +171,18 @@ uint32_t* ScratchLease::table(uint64_t bytes) {
                 s_->bytes = 0;
             }
         }
-        if (e == hipSuccess) e = hipMalloc(&s_->table, bytes);
         if (e == hipSuccess) {
-            s_->bytes = bytes;
-            s_->dirty = true;
-        } else if (!s_->bytes) {
-            s_->table = nullptr;
+            void* p = nullptr;
+            e = hipMalloc(&p, bytes);
+            if (e == hipSuccess) {
+                s_->table = p;
+                s_->bytes = bytes;
+                s_->dirty = true;
+            }
+        }
+        if (e != hipSuccess) {
+            std::lock_guard<std::mutex> lock(pool().m);
+            pool().held[device_] -= bytes - s_->bytes;
         }
     }
     if (e == hipSuccess && s_->dirty) e = hipMemsetAsync(s_->table, 0, s_->bytes, stream_);
@@ -80,9 +198,17 @@ void ScratchLease::clean() { s_->dirty = false; }
 
 hipError_t ScratchLease::spills(void** out) {
     if (!s_) return hipErrorInvalidDevice;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(stream_, &cap);
+    if (e != hipSuccess) return e;
+    if (cap != hipStreamCaptureStatusNone) {
+        if (!s_->spills) return hipErrorStreamCaptureUnsupported;  // the counters could not be cleared
+        s_->recorded = true;
+    }
     if (!s_->spills) {
+        const RelaxedCapture relaxed;
         void* p = nullptr;
-        hipError_t e = hipMalloc(&p, marker_ws_bytes());
+        e = hipMalloc(&p, marker_ws_bytes());
         if (e != hipSuccess) return e;
         e = hipMemsetAsync(p, 0, 256, stream_);  // the counters start at zero
         if (e != hipSuccess) {
@@ -96,3 +222,27 @@ hipError_t ScratchLease::spills(void** out) {
 }
 
 }  // namespace voxamd
+
+using namespace voxamd;
+
+extern "C" vox_status vox_release_scratch(void) {
+    int device = 0;
+    const hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
+    const RelaxedCapture relaxed;
+    ScratchPool& P = pool();
+    std::lock_guard<std::mutex> lock(P.m);
+    bool all = true;
+    for (auto it = P.streams.begin(); it != P.streams.end();) {
+        if (it->first.device == device && it->second.holders == 0) {
+            if (!give_back(P, device, it->second)) {
+                all = false;
+            } else if (!it->second.spills) {
+                it = P.streams.erase(it);
+                continue;
+            }
+        }
+        ++it;
+    }
+    return all ? VOX_OK : fail(VOX_ERR_HIP, "vox_release_scratch: the device could not be waited for");
+}

@@ -68,7 +68,9 @@ typedef enum vox_status {
    least 4 G^2 triangles at G <= 64, or G^2 at G <= 128 with G % 32 != 0, marker
    otherwise).  All algorithms give identical tables.  Per device and stream the
    library keeps scratch tables of up to G^3/8 bytes (rows rounded up to words)
-   for linear surfaces up to 2048^3 and for solids; a linear surface call whose
+   for linear surfaces up to 2048^3 and for solids: of a device's streams
+   together at most an eighth of its memory (or one stream's table), until
+   vox_release_scratch; a linear surface call whose
    stream is being captured, or that cannot have one, works in the caller's
    table.  A captured marker call holds none either: linear, non-accumulating
    ones on G % 32 == 0 work in the caller's table (the graph holds 1 MB of
@@ -164,6 +166,12 @@ vox_status vox_surface(const vox_info* info, const float* d_tris, uint32_t* d_ta
    (uint64 device memory, stream-ordered; the caller zeroes it). */
 vox_status vox_solid(const vox_info* info, const float* d_tris, uint32_t* d_table, int layout,
                      unsigned flags, uint64_t* d_offrow, void* stream);
+
+/* Frees the scratch tables and spill records that the library keeps for the
+   streams of the current device (after waiting for the device); streams with a
+   call being queued at the moment keep theirs.  The next call on a stream
+   allocates anew. */
+vox_status vox_release_scratch(void);
 
 /* vox_solid without any device allocation.  It has no counterpart in the
    reference: it is for callers that cannot allocate device memory (code under
