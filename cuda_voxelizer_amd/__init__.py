@@ -248,8 +248,9 @@ def voxelize_surface(info: VoxInfo, tris, morton: bool = False, table=None, accu
 
     Without ``accumulate`` the table is fully defined by this call; with it
     bits are OR-ed into the existing contents (reference semantics).
-    ``tune``: VOX_TUNE_* bits (``_capi.tune_*``) and the algorithm's VOX_SLAB_* / VOX_REGION_*
-    bits (``_capi.region_*``); every setting gives the same table."""
+    ``tune``: VOX_TUNE_* bits (``_capi.tune_*``), the algorithm's VOX_SLAB_* / VOX_REGION_*
+    bits (``_capi.region_*``) and VOX_FLAG_NO_SCRATCH (``_capi``: the call allocates no device
+    memory of the library's own); every setting gives the same table."""
     flags = (VOX_FLAG_ACCUMULATE if accumulate else 0) | _algo_flag(algo) | (int(tune) & _capi.KNOB_MASK)
     lib = _capi.load()
     plain = _plain_call(info, tris, table, stream)

@@ -28,6 +28,7 @@ VOX_FLAG_ALGO_CHUNK = 0x8
 VOX_FLAG_ALGO_MARKER = 0x10
 VOX_FLAG_ALGO_SLAB = 0x20
 VOX_FLAG_ALGO_REGION = 0x40
+VOX_FLAG_NO_SCRATCH = 0x80
 ALGO_FLAGS = {"auto": 0, "direct": VOX_FLAG_ALGO_DIRECT, "tile": VOX_FLAG_ALGO_TILE, "chunk": VOX_FLAG_ALGO_CHUNK,
               "marker": VOX_FLAG_ALGO_MARKER, "slab": VOX_FLAG_ALGO_SLAB, "region": VOX_FLAG_ALGO_REGION}
 
@@ -65,7 +66,7 @@ def tune_tile(t: int) -> int:
 
 TUNE_MASK = 0xFF000000
 ALGO_KNOB_MASK = 0x007FFF00  # VOX_SLAB_* / VOX_REGION_* bits (read only with their algorithm flag)
-KNOB_MASK = TUNE_MASK | ALGO_KNOB_MASK
+KNOB_MASK = TUNE_MASK | ALGO_KNOB_MASK | VOX_FLAG_NO_SCRATCH
 
 
 _STATUS_NAMES = {0: "VOX_OK", 1: "VOX_ERR_INVALID", 2: "VOX_ERR_HIP", 3: "VOX_ERR_OOM",

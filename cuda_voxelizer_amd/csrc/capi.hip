@@ -185,7 +185,7 @@ vox_status run(const vox_info* info, const float* d_tris, uint32_t* d_table, int
         return fail(VOX_ERR_INVALID, "the marker algorithm is solid-only");
     hipStream_t st = (hipStream_t)stream;
     const uint32_t G = info->gridsize[0];
-    const bool accumulate = (flags & VOX_FLAG_ACCUMULATE) != 0;
+    const bool accumulate = (flags & VOX_FLAG_ACCUMULATE) != 0, scratch = !(flags & VOX_FLAG_NO_SCRATCH);
     TilePlan P;
     const bool have_plan = make_plan((int)G, layout, solid, P, tune_tile_scale(flags)) || make_plan((int)G, layout, solid, P);
     const bool have_marker = solid && marker_supported(G, layout, accumulate);
@@ -239,8 +239,8 @@ vox_status run(const vox_info* info, const float* d_tris, uint32_t* d_table, int
     }
     if (algo == MARKER) {
         e = launch_solid_marker(*info, d_tris, d_table, layout, accumulate, (unsigned long long*)d_offrow, st,
-                                tune_big(flags));
-        if (e == hipErrorOutOfMemory && !algo_bits && have_plan && coarse_mesh(info->n_triangles, G)) {
+                                tune_big(flags), scratch);
+        if (e == hipErrorOutOfMemory && scratch && !algo_bits && have_plan && coarse_mesh(info->n_triangles, G)) {
             (void)hipGetLastError();  // tile needs no scratch table
             algo = TILE;
         } else if (e == hipErrorOutOfMemory) {
@@ -263,7 +263,8 @@ vox_status run(const vox_info* info, const float* d_tris, uint32_t* d_table, int
         return VOX_OK;
     }
     if (algo == CHUNK) {
-        e = launch_surface_chunk(*info, d_tris, d_table, layout, accumulate, st, tune_big(flags), tune_waves(flags));
+        e = launch_surface_chunk(*info, d_tris, d_table, layout, accumulate, st, tune_big(flags), tune_waves(flags),
+                                 scratch);
         if (e != hipSuccess) return hip_fail(e, "chunk kernels launch");
         return VOX_OK;
     }

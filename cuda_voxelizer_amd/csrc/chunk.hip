@@ -737,14 +737,14 @@ hipError_t launch_surface_region_chunks(const vox_info& info, const float* tris,
 }
 
 hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_t* table, int layout, bool accumulate,
-                                hipStream_t stream, uint32_t big, int waves) {
+                                hipStream_t stream, uint32_t big, int waves, bool scratch) {
     const ItemMap none{nullptr, nullptr, 1, 0};
     ItemDev one = single_job(info, tris, table, layout);
     one.big = big;
     one.accumulate = accumulate ? 1 : 0;
     chunk_shape(one);
     const uint32_t G = info.gridsize[0];
-    if (info.n_triangles && chunk_blocked(layout, G, info.n_triangles)) {
+    if (scratch && info.n_triangles && chunk_blocked(layout, G, info.n_triangles)) {
         hipError_t e = hipSuccess;
         const uint64_t bytes = blocked_bytes(G);
         one.flagged = G > kUnflaggedGrid && unblock_vec(G, table) ? 1u : 0u;

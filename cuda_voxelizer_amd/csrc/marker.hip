@@ -794,7 +794,8 @@ static hipError_t marker_ws(ScratchLease& S, MarkerWs& ws) {
 }
 
 hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t* table, int layout,
-                               bool accumulate, unsigned long long* offrow, hipStream_t stream, uint32_t big) {
+                               bool accumulate, unsigned long long* offrow, hipStream_t stream, uint32_t big,
+                               bool scratch) {
     const uint32_t G = info.gridsize[0];
     // linear, no accumulation: markers into the scratch table and one streaming
     // pass (suffix into the table, scratch back to zero) where rows are whole
@@ -808,7 +809,7 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     MarkerWs ws;
     hipError_t e = marker_ws(S, ws);
     if (e != hipSuccess) return e;
-    uint32_t* markers = in_place ? table : S.table(table_bytes);
+    uint32_t* markers = in_place ? table : (scratch ? S.table(table_bytes) : nullptr);
     if (!markers && !stream_rows) return hipErrorOutOfMemory;
     // the in-place form needs no scratch table
     if (in_place || !markers) return launch_marker_in_place(info, tris, table, offrow, ws, stream, big);

@@ -5,7 +5,9 @@
 // runs (marker.hip), whose counters are zero between calls.  Both are worked on by
 // several launches of a call in a row, so a call holds the stream's scratch from
 // before its first launch until its last is queued; a second thread's call on the
-// stream waits for that, and the stream's order does the rest.  Calls on the
+// stream waits for that, and the stream's order does the rest.  (A new stream may
+// have the handle of one that was destroyed; hipStreamDestroy waits for a stream's
+// work.)  Calls on the
 // stream's other workspaces (tile, slab, region, triangle order) hold it too.
 #pragma once
 

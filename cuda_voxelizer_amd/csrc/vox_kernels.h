@@ -37,7 +37,8 @@ uint32_t marker_row_units(uint32_t G);
 hipError_t launch_marker_jobs(const ItemMap& m_blocks, const ItemMap& m_rows, const ItemMap& m_tris,
                               uint32_t blocks, uint32_t row_units, void* mws, hipStream_t stream);
 hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t* table, int layout,
-                               bool accumulate, unsigned long long* offrow, hipStream_t stream, uint32_t big = 0);
+                               bool accumulate, unsigned long long* offrow, hipStream_t stream, uint32_t big = 0,
+                               bool scratch = true);
 // A call recorded into a graph: in place, marker_batch_supported() forms.
 hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris, uint32_t* table,
                                         unsigned long long* offrow, hipStream_t stream, uint32_t big);
@@ -123,7 +124,7 @@ int chunk_spec(int layout, uint32_t G);
 hipError_t launch_chunk_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, bool loop, hipStream_t stream,
                              int waves = 0, int spec = kSpecAny);
 hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_t* table, int layout, bool accumulate,
-                                hipStream_t stream, uint32_t big = 0, int waves = 0);
+                                hipStream_t stream, uint32_t big = 0, int waves = 0, bool scratch = true);
 // Word w of row (y, z) in a blocked table: the 4 x 4 rows of a block lie together.
 __device__ __forceinline__ uint32_t blocked_word(uint32_t G, uint32_t w, uint32_t y, uint32_t z) {
     return ((((z >> 2) * ((G + 3u) >> 2) + (y >> 2)) * ((G + 31u) >> 5) + w) << 4) | ((z & 3u) << 2) | (y & 3u);

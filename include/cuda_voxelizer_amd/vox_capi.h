@@ -106,6 +106,12 @@ typedef enum vox_status {
                                     and takes the row suffix XOR) and writes every word
                                     of the region once -- no zero-fill pass, and global
                                     atomics only for the staging reservations */
+#define VOX_FLAG_NO_SCRATCH 0x80u /* the call uses no scratch table: a surface by the
+                                    default, chunk or direct algorithm then allocates
+                                    nothing; a marker solid works in the caller's table
+                                    (linear, non-accumulating, G % 32 == 0) or runs
+                                    direct, and keeps 1 MB of run records per stream.
+                                    The table is the same. */
 /* Region capacity bits (with VOX_FLAG_ALGO_REGION; a zero field is the library's
    choice).  Every setting gives the same table: pairs that find no room take a
    scratch-table fallback, so small capacities only cost time. */
