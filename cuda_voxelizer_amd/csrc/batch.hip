@@ -44,6 +44,7 @@ struct vox_batch {
     void* ws = nullptr;
     void* mws = nullptr;  // marker class: spill records and counters
     void* sws = nullptr;  // blocked chunk class: the jobs' scratch tables, all zero between launches
+    uint64_t scratch_bytes = 0;
     voxamd::WorkspaceLayout L{};
     // chunk / chunkw (6 waves per SIMD): one class per layout specialisation (ChunkSpec)
     voxamd::JobClass fill, chunk[voxamd::kBlockedSpecs], chunkw[voxamd::kBlockedSpecs], unblock, marker, dsurf, dsolid,
@@ -203,7 +204,8 @@ struct BatchPlan {
     uint64_t scratch = 0;  // bytes of blocked scratch tables; the jobs hold their offsets until place_scratch
 };
 
-// A batch's scratch tables together; jobs beyond it go to their tables directly.
+// A batch's scratch tables together; jobs beyond it go to their tables directly, as
+// all do where the device has no room for them.
 constexpr uint64_t kBatchScratch = 1ull << 30;
 
 // Every chunk class and the others, in the order of the packed image.
@@ -236,7 +238,8 @@ static void reset_classes(vox_batch* b) {
     b->total_triangles = 0;
 }
 
-static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* b, BatchPlan& plan) {
+static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* b, BatchPlan& plan,
+                             uint64_t scratch_limit) {
     if (count < 0 || (count > 0 && !items)) return fail(VOX_ERR_INVALID, "bad item array");
     reset_classes(b);
     b->count = count;
@@ -280,7 +283,7 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
         const uint64_t table_bytes = blocked_bytes(G);
         // 48 mixed meshes, linear keys -> blocked: 740 -> 405 us a launch
         const bool blocked = a == CHUNK && !(it.flags & VOX_FLAG_NO_SCRATCH) && G <= kUnflaggedGrid && chunk_blocked(it.layout, G, n) &&
-                             plan.scratch + table_bytes <= kBatchScratch;
+                             plan.scratch + table_bytes <= scratch_limit;
         if (a != TILE && !accumulate && !blocked) {
             b->fill.items.push_back(d);
             add_prefix(b->fill.base_a, b->fill.total_a, fill_units(G));
@@ -383,9 +386,8 @@ using namespace voxamd;
 
 extern "C" {
 
-vox_status vox_batch_create(const vox_batch_item* items, int count, unsigned flags, vox_batch** out) {
-    if (!out) return fail(VOX_ERR_INVALID, "out is NULL");
-    *out = nullptr;
+static vox_status create_batch(const vox_batch_item* items, int count, unsigned flags, uint64_t scratch_limit,
+                               uint64_t& scratch, vox_batch** out) {
     vox_batch* b = new (std::nothrow) vox_batch();
     if (!b) return fail(VOX_ERR_OOM, "host allocation");
     b->use_graph = !(flags & VOX_BATCH_NO_GRAPH);
@@ -395,11 +397,12 @@ vox_status vox_batch_create(const vox_batch_item* items, int count, unsigned fla
         return hip_fail(e, "hipGetDevice");
     }
     BatchPlan plan;
-    vox_status s = plan_batch(items, count, b, plan);
+    vox_status s = plan_batch(items, count, b, plan, scratch_limit);
     if (s != VOX_OK) {
         free_batch(b);
         return s;
     }
+    scratch = plan.scratch;
     if (plan.scratch) {
         e = hipMalloc(&b->sws, plan.scratch);
         if (e == hipSuccess) e = hipMemset(b->sws, 0, plan.scratch);
@@ -407,6 +410,7 @@ vox_status vox_batch_create(const vox_batch_item* items, int count, unsigned fla
             free_batch(b);
             return fail(VOX_ERR_OOM, std::string("batch scratch tables: ") + hipGetErrorString(e));
         }
+        b->scratch_bytes = plan.scratch;
         place_scratch(b, plan);
     }
     e = hipMalloc(&b->dev_mem, plan.host.size());
@@ -459,6 +463,18 @@ vox_status vox_batch_create(const vox_batch_item* items, int count, unsigned fla
     return VOX_OK;
 }
 
+vox_status vox_batch_create(const vox_batch_item* items, int count, unsigned flags, vox_batch** out) {
+    if (!out) return fail(VOX_ERR_INVALID, "out is NULL");
+    *out = nullptr;
+    uint64_t scratch = 0;
+    vox_status s = create_batch(items, count, flags, kBatchScratch, scratch, out);
+    if (s == VOX_ERR_OOM && scratch) {  // the scratch tables are optional
+        (void)hipGetLastError();
+        s = create_batch(items, count, flags, 0, scratch, out);
+    }
+    return s;
+}
+
 vox_status vox_batch_launch(vox_batch* b, void* stream) {
     if (!b) return fail(VOX_ERR_INVALID, "batch is NULL");
     hipStream_t st = (hipStream_t)stream;
@@ -477,7 +493,7 @@ vox_status vox_batch_info(const vox_batch* b, int64_t out[8]) {
     out[4] = (int64_t)b->tsolid.items.size();
     out[5] = (int64_t)(b->dsurf.items.size() + b->dsolid.items.size());
     out[6] = b->use_graph ? 1 : 0;
-    out[7] = (int64_t)b->L.total;
+    out[7] = (int64_t)(b->L.total + b->scratch_bytes);
     return VOX_OK;
 }
 
@@ -504,6 +520,7 @@ struct vox_runner {
     int slot = 0;
     uint64_t tiles_cap = 0, n_cap = 0;
     uint64_t scratch_cap = 0;
+    uint64_t scratch_limit = kBatchScratch;  // 0 once the device had no room
     bool scratch_dirty = false;  // a launch failed between the scratch tables' use and their clearing
     uint64_t launches = 0;
 };
@@ -527,10 +544,9 @@ vox_status vox_runner_create(void* stream, vox_runner** out) {
     return VOX_OK;
 }
 
-vox_status vox_runner_launch(vox_runner* r, const vox_batch_item* items, int count) {
-    if (!r) return fail(VOX_ERR_INVALID, "runner is NULL");
-    BatchPlan plan;
-    vox_status s = plan_batch(items, count, &r->b, plan);
+// The launch's plan, and the device buffers that it needs.
+static vox_status prepare_launch(vox_runner* r, const vox_batch_item* items, int count, BatchPlan& plan) {
+    vox_status s = plan_batch(items, count, &r->b, plan, r->scratch_limit);
     if (s != VOX_OK) return s;
     hipError_t e;
     // grow-only device buffers; growing waits for this runner's stream
@@ -597,6 +613,25 @@ vox_status vox_runner_launch(vox_runner* r, const vox_batch_item* items, int cou
             return fail(VOX_ERR_OOM, std::string("runner descriptors: ") + hipGetErrorString(e));
         }
     }
+    return VOX_OK;
+}
+
+vox_status vox_runner_launch(vox_runner* r, const vox_batch_item* items, int count) {
+    if (!r) return fail(VOX_ERR_INVALID, "runner is NULL");
+    BatchPlan plan;
+    vox_status s = prepare_launch(r, items, count, plan);
+    if (s == VOX_ERR_OOM && (plan.scratch || r->b.sws)) {  // the scratch tables are optional
+        (void)hipGetLastError();
+        hipError_t w = hipStreamSynchronize(r->stream);
+        if (w != hipSuccess) return hip_fail(w, "hipStreamSynchronize");
+        if (r->b.sws) (void)hipFree(r->b.sws);
+        r->b.sws = nullptr;
+        r->scratch_cap = r->scratch_limit = 0;
+        plan = BatchPlan{};
+        s = prepare_launch(r, items, count, plan);
+    }
+    if (s != VOX_OK) return s;
+    hipError_t e;
     // stage through a pinned slot whose previous copy has completed
     const int k = r->slot;
     r->slot ^= 1;

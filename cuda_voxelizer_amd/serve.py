@@ -18,8 +18,9 @@ Requests (a mesh, a grid, surface or solid) arrive at any time.  Each call to
 ``serve_plain`` is the comparison path: one plain per-request call
 (``vox_surface`` / ``vox_solid``) per request, in arrival order.
 
-Budget accounting counts table bytes and resident mesh bytes (the runners'
-binning workspaces are outside it); a request larger than the whole budget is
+Budget accounting counts table bytes and resident mesh bytes (outside it are the
+runners' binning workspaces and scratch tables, of the latter at most 1 GB a
+runner, and none where the device has no room); a request larger than the whole budget is
 rejected.
 """
 from __future__ import annotations
