@@ -154,18 +154,6 @@ vox_status get_slab_workspace(hipStream_t st, const SlabPlan& P, uint64_t n, voi
     return VOX_OK;
 }
 
-// Whether calls on a stream are being recorded into a graph.  A graph must not
-// hold a scratch table (a later, larger call replaces it, and eager calls on the
-// stream use it between the replays).
-static bool captured(hipStream_t st) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        return true;  // the null stream beside a capture: nothing shared is touched
-    }
-    return cap != hipStreamCaptureStatusNone;
-}
-
 // One voxelization.  Algorithms: tile (binned, tile-owned writes; needs a
 // plan for this grid/layout), chunk (surface only, LDS word merging + global
 // atomics after a fill), marker (solid) and direct (one triangle per lane).
@@ -229,18 +217,11 @@ vox_status run(const vox_info* info, const float* d_tris, uint32_t* d_table, int
         if (e != hipSuccess) return hip_fail(e, "slab kernels launch");
         return VOX_OK;
     }
-    if (algo == MARKER && captured(st)) {
-        if (marker_batch_supported(G, layout, accumulate)) {
-            e = launch_solid_marker_captured(*info, d_tris, d_table, (unsigned long long*)d_offrow, st, tune_big(flags));
-            if (e != hipSuccess) return hip_fail(e, "marker kernels launch (captured)");
-            return VOX_OK;
-        }
-        algo = DIRECT;
-    }
     if (algo == MARKER) {
         e = launch_solid_marker(*info, d_tris, d_table, layout, accumulate, (unsigned long long*)d_offrow, st,
                                 tune_big(flags), scratch);
-        if (e == hipErrorOutOfMemory && scratch && !algo_bits && have_plan && coarse_mesh(info->n_triangles, G)) {
+        if (e == hipErrorOutOfMemory && scratch && !algo_bits && have_plan && coarse_mesh(info->n_triangles, G) &&
+            !ScratchLease(st).recording()) {
             (void)hipGetLastError();  // tile needs no scratch table
             algo = TILE;
         } else if (e == hipErrorOutOfMemory) {

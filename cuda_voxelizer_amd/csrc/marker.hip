@@ -786,6 +786,9 @@ static uint32_t marker_units(const ItemDev& it) {
 hipError_t launch_marker_in_place(const vox_info& info, const float* tris, uint32_t* table,
                                   unsigned long long* offrow, const MarkerWs& ws, hipStream_t stream, uint32_t big);
 
+static hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris, uint32_t* table,
+                                               unsigned long long* offrow, hipStream_t stream, uint32_t big);
+
 static hipError_t marker_ws(ScratchLease& S, MarkerWs& ws) {
     void* p = nullptr;
     const hipError_t e = S.spills(&p);
@@ -806,6 +809,10 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     const bool in_place = layout == VOX_LAYOUT_LINEAR && !accumulate && !stream_rows && !ragged;
     const uint64_t table_bytes = (uint64_t)G * G * ((G + 31u) / 32u) * 4u;  // rows padded to words
     ScratchLease S(stream);
+    if (S.recording())
+        return marker_batch_supported(G, layout, accumulate)
+                   ? launch_solid_marker_captured(info, tris, table, offrow, stream, big)
+                   : hipErrorOutOfMemory;
     MarkerWs ws;
     hipError_t e = marker_ws(S, ws);
     if (e != hipSuccess) return e;
@@ -975,8 +982,8 @@ size_t static_scratch_bytes() { return kStaticScratchBytes; }
 static std::mutex g_capture_mutex;
 static std::map<StreamKey, void*> g_capture_ws;
 
-hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris, uint32_t* table,
-                                        unsigned long long* offrow, hipStream_t stream, uint32_t big) {
+static hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris, uint32_t* table,
+                                               unsigned long long* offrow, hipStream_t stream, uint32_t big) {
     StreamKey key;
     hipError_t e = stream_key(stream, key);
     if (e != hipSuccess) return e;
@@ -985,17 +992,12 @@ hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris,
         std::lock_guard<std::mutex> lock(g_capture_mutex);
         void*& w = g_capture_ws[key];
         if (!w) {
-            // an allocation is no stream operation; only the default capture mode forbids it
-            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-            e = hipThreadExchangeStreamCaptureMode(&mode);
-            if (e != hipSuccess) return e;
+            const RelaxedCapture relaxed;
             e = hipMalloc(&w, kStaticScratchBytes);
-            const hipError_t e2 = hipThreadExchangeStreamCaptureMode(&mode);
             if (e != hipSuccess) {
                 w = nullptr;
                 return e;
             }
-            if (e2 != hipSuccess) return e2;
         }
         p = w;
     }

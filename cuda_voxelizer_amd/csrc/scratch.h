@@ -28,8 +28,21 @@ struct StreamKey {
     bool operator<(const StreamKey& o) const {
         return std::tie(device, stream, thread) < std::tie(o.device, o.stream, o.thread);
     }
+    bool operator==(const StreamKey& o) const { return !(*this < o) && !(o < *this); }
 };
 hipError_t stream_key(hipStream_t stream, StreamKey& key);  // on the current device
+
+// Memory is allocated and freed, and the device waited for, in the relaxed capture
+// mode: no stream that is being captured is touched, and the default mode refuses
+// it while any thread captures one.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool set;
+    RelaxedCapture() : set(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+    ~RelaxedCapture() {
+        if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
 
 struct StreamScratch;
 
@@ -40,6 +53,9 @@ class ScratchLease {
     ScratchLease(const ScratchLease&) = delete;
     ScratchLease& operator=(const ScratchLease&) = delete;
 
+    // Calls on the stream are being recorded into a graph (or, for the null stream,
+    // another stream's capture keeps it from being used).
+    bool recording() const { return recording_; }
     // A zero table of at least `bytes` bytes; null while the stream is being
     // captured (a later call may replace the table that the graph would hold),
     // without memory, and where the device's tables would grow beyond their limit.
@@ -53,6 +69,7 @@ class ScratchLease {
    private:
     hipStream_t stream_;
     int device_ = 0;
+    bool recording_ = true;
     StreamScratch* s_ = nullptr;
 };
 

@@ -11,7 +11,12 @@
 
 namespace voxamd {
 
+struct DeviceScratch {
+    uint64_t held = 0, leases = 0;  // bytes in tables, leases so far
+};
+
 struct StreamScratch {
+    DeviceScratch* dev = nullptr;
     void* table = nullptr;  // grow-only
     uint64_t bytes = 0;
     bool dirty = true;
@@ -32,7 +37,7 @@ constexpr uint64_t kIdle = 64;
 struct ScratchPool {
     std::mutex m;
     std::map<StreamKey, StreamScratch> streams;
-    std::map<int, uint64_t> held, leases;  // of a device: bytes in tables, leases so far
+    std::map<int, DeviceScratch> devices;
     std::vector<uint64_t> ended;           // threads
 };
 static ScratchPool& pool() {
@@ -63,28 +68,16 @@ hipError_t stream_key(hipStream_t stream, StreamKey& key) {
     return hipGetDevice(&key.device);
 }
 
-// Memory is allocated and freed in the relaxed capture mode: it touches no stream
-// that is being captured, and the default mode refuses it while any thread
-// captures one.
-struct RelaxedCapture {
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    const bool set;
-    RelaxedCapture() : set(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
-    ~RelaxedCapture() {
-        if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
-    }
-};
-
 // Frees what an idle stream of the current device has, whose last call may still
 // run.  False if the device cannot be waited for.
-static bool give_back(ScratchPool& P, int device, StreamScratch& s) {
+static bool give_back(StreamScratch& s) {
     if (!s.table && (!s.spills || s.recorded)) return true;
     if (hipDeviceSynchronize() != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
     if (s.table) (void)hipFree(s.table);
-    P.held[device] -= s.bytes;
+    s.dev->held -= s.bytes;
     s.table = nullptr;
     s.bytes = 0;
     if (s.spills && !s.recorded) {
@@ -106,7 +99,7 @@ static bool reserve(int device, StreamScratch& s, uint64_t bytes) {
         bool left = false;
         for (auto it = P.streams.begin(); it != P.streams.end();) {
             const bool own = it->first.thread == n;
-            if (own && it->first.device == device && it->second.holders == 0 && give_back(P, device, it->second) &&
+            if (own && it->first.device == device && it->second.holders == 0 && give_back(it->second) &&
                 !it->second.spills) {
                 it = P.streams.erase(it);
                 continue;
@@ -116,18 +109,18 @@ static bool reserve(int device, StreamScratch& s, uint64_t bytes) {
         }
         if (!left) P.ended.erase(P.ended.begin() + (long)i--);
     }
-    const uint64_t limit = total / 8, now = P.leases[device];
-    while (P.held[device] - s.bytes + bytes > limit && P.held[device] > s.bytes) {
+    const uint64_t limit = total / 8, now = s.dev->leases;
+    while (s.dev->held - s.bytes + bytes > limit && s.dev->held > s.bytes) {
         auto idle = P.streams.end();
         for (auto it = P.streams.begin(); it != P.streams.end(); ++it)
             if (it->first.device == device && it->second.holders == 0 && it->second.table &&
                 now - it->second.last >= kIdle &&
                 (idle == P.streams.end() || it->second.last < idle->second.last))
                 idle = it;
-        if (idle == P.streams.end() || !give_back(P, device, idle->second)) return false;
+        if (idle == P.streams.end() || !give_back(idle->second)) return false;
         if (!idle->second.spills) P.streams.erase(idle);
     }
-    P.held[device] += bytes - s.bytes;
+    s.dev->held += bytes - s.bytes;
     return true;
 }
 
@@ -138,12 +131,18 @@ ScratchLease::ScratchLease(hipStream_t stream) : stream_(stream) {
         return;
     }
     device_ = key.device;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) == hipSuccess)
+        recording_ = cap != hipStreamCaptureStatusNone;
+    else
+        (void)hipGetLastError();
     ScratchPool& P = pool();
     {
         std::lock_guard<std::mutex> lock(P.m);
         s_ = &P.streams[key];
+        if (!s_->dev) s_->dev = &P.devices[device_];
         s_->holders++;
-        s_->last = ++P.leases[device_];
+        s_->last = ++s_->dev->leases;
     }
     s_->use.lock();
 }
@@ -156,11 +155,9 @@ ScratchLease::~ScratchLease() {
 }
 
 uint32_t* ScratchLease::table(uint64_t bytes) {
-    if (!s_) return nullptr;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    hipError_t e = hipStreamIsCapturing(stream_, &cap);
-    if (e == hipSuccess && cap != hipStreamCaptureStatusNone) return nullptr;
-    if (e == hipSuccess && s_->bytes < bytes) {
+    if (!s_ || recording_) return nullptr;
+    hipError_t e = hipSuccess;
+    if (s_->bytes < bytes) {
         const RelaxedCapture relaxed;
         if (!reserve(device_, *s_, bytes)) return nullptr;
         if (s_->table) {
@@ -182,7 +179,7 @@ uint32_t* ScratchLease::table(uint64_t bytes) {
         }
         if (e != hipSuccess) {
             std::lock_guard<std::mutex> lock(pool().m);
-            pool().held[device_] -= bytes - s_->bytes;
+            s_->dev->held -= bytes - s_->bytes;
         }
     }
     if (e == hipSuccess && s_->dirty) e = hipMemsetAsync(s_->table, 0, s_->bytes, stream_);
@@ -198,17 +195,14 @@ void ScratchLease::clean() { s_->dirty = false; }
 
 hipError_t ScratchLease::spills(void** out) {
     if (!s_) return hipErrorInvalidDevice;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    hipError_t e = hipStreamIsCapturing(stream_, &cap);
-    if (e != hipSuccess) return e;
-    if (cap != hipStreamCaptureStatusNone) {
+    if (recording_) {
         if (!s_->spills) return hipErrorStreamCaptureUnsupported;  // the counters could not be cleared
         s_->recorded = true;
     }
     if (!s_->spills) {
         const RelaxedCapture relaxed;
         void* p = nullptr;
-        e = hipMalloc(&p, marker_ws_bytes());
+        hipError_t e = hipMalloc(&p, marker_ws_bytes());
         if (e != hipSuccess) return e;
         e = hipMemsetAsync(p, 0, 256, stream_);  // the counters start at zero
         if (e != hipSuccess) {
@@ -235,7 +229,7 @@ extern "C" vox_status vox_release_scratch(void) {
     bool all = true;
     for (auto it = P.streams.begin(); it != P.streams.end();) {
         if (it->first.device == device && it->second.holders == 0) {
-            if (!give_back(P, device, it->second)) {
+            if (!give_back(it->second)) {
                 all = false;
             } else if (!it->second.spills) {
                 it = P.streams.erase(it);

@@ -39,9 +39,6 @@ hipError_t launch_marker_jobs(const ItemMap& m_blocks, const ItemMap& m_rows, co
 hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t* table, int layout,
                                bool accumulate, unsigned long long* offrow, hipStream_t stream, uint32_t big = 0,
                                bool scratch = true);
-// A call recorded into a graph: in place, marker_batch_supported() forms.
-hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris, uint32_t* table,
-                                        unsigned long long* offrow, hipStream_t stream, uint32_t big);
 // The allocation-free solid form: its scratch is a static device array of
 // static_scratch_bytes() bytes per GPU (address taken once per device).
 size_t static_scratch_bytes();
