@@ -241,7 +241,8 @@ int vox_check_voxel(const uint32_t* table, uint32_t grid, uint32_t x, uint32_t y
    vox_info and flags are fixed at creation (a plan, as in FFT libraries);
    triangle and table contents may change between launches.  Tables of the
    items must not overlap.  A batch, like a runner, takes up to 1 GB of scratch
-   tables for its linear surfaces if the device has room. */
+   tables for its linear surfaces if the device has room.  Launches of one batch
+   on different streams wait for each other (not when captured). */
 typedef struct vox_batch_item {
     vox_info info;         /* per-job voxinfo (cubic grid) */
     const float* d_tris;   /* device AoS triangles, info.n_triangles of them */
