@@ -418,11 +418,6 @@ __device__ __forceinline__ void table_or(uint32_t* p, uint32_t v) {
 // one word in x of those 4 rows.  Work unit: 256 threads.
 // accumulate: bits are ORed into the table, only where there are any, and
 // atomically: other calls, on other streams, may be adding to the table.
-// FLAGS: groups of 256 bytes whose flag is not set are zero and not read.  From
-// kStreamedGrid on the table and the scratch table are beyond the 256 MB of the
-// last cache each, and the rows must not push the scratch words out of it: 81,920
-// at 2048^3 488 -> 300 us, at 1536^3 270 -> 189; at 1152^3 that loses (128, 175).
-template <bool FLAGS>
 __device__ __forceinline__ void unblock_quad(const ItemDev& it, uint32_t t, bool vec) {
     const uint32_t G = it.info.gridsize[0], rw = G >> 5;
     uint4* __restrict__ s4 = (uint4*)it.scratch;
@@ -435,12 +430,8 @@ __device__ __forceinline__ void unblock_quad(const ItemDev& it, uint32_t t, bool
         if (bz >= G >> 2) return;
         const uint64_t base = ((uint64_t)(bz * (G >> 2) + by) * rw + 4u * wq) * 4u + zl;
         uint4 v[4];
-        // the four lanes of a 256-byte group read its flag in one instruction, before it is cleared
-        uint8_t* flag = (uint8_t*)it.scratch - 1 - (base >> 4);
-        const bool any = !FLAGS || *flag != 0;
-        if (FLAGS && any && zl == 0u) *flag = 0;
 #pragma unroll
-        for (int u = 0; u < 4; u++) v[u] = any ? s4[base + 4u * (uint32_t)u] : make_uint4(0u, 0u, 0u, 0u);
+        for (int u = 0; u < 4; u++) v[u] = s4[base + 4u * (uint32_t)u];
 #pragma unroll
         for (int u = 0; u < 4; u++)
             if (v[u].x | v[u].y | v[u].z | v[u].w) s4[base + 4u * (uint32_t)u] = make_uint4(0u, 0u, 0u, 0u);
@@ -450,9 +441,7 @@ __device__ __forceinline__ void unblock_quad(const ItemDev& it, uint32_t t, bool
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const uint64_t d = (((uint64_t)(4u * bz + zl) * G + 4u * by + (uint32_t)u) * rw >> 2) + wq;
-            if (!it.accumulate && FLAGS && G >= kStreamedGrid) {
-                store_streaming(d4 + d, o[u]);
-            } else if (!it.accumulate) {
+            if (!it.accumulate) {
                 d4[d] = o[u];
             } else {
                 uint32_t* p = (uint32_t*)(d4 + d);
@@ -482,64 +471,218 @@ __device__ __forceinline__ void unblock_quad(const ItemDev& it, uint32_t t, bool
     }
 }
 
+// How rows are written: 16-byte groups, past the caches or not; words (a table at
+// another address); words that are ORed into the table.
+enum RowsForm : int { kRowsStreamed, kRowsCached, kRowsWords, kRowsAdded };
+template <int FORM>
+__device__ __forceinline__ void put_quad(uint4* d, const uint4& v) {
+    if (FORM == kRowsStreamed)
+        store_streaming(d, v);
+    else
+        *d = v;
+}
+
+// The same with flags: groups of 256 bytes whose flag is not set are zero and not
+// read.  A workgroup takes a strip: K blocks in y of one 4-row slab in z, which lie
+// together in the scratch table and are 4 runs of 4 K rows of the table.  One load
+// by every wave has the strip's flags (at most 64).  What they name is turned in
+// LDS, so that both sides are whole 16-byte groups of consecutive lanes whatever
+// the row length (4-byte ones into tables at other addresses).  Lines without bits
+// are written before the others have been read, whole ones: half a line at a time
+// is what the stores must avoid (one at 2048^3 in two parts: 800 us a call, not
+// 312).  Rows written per thread as in unblock_quad, 16 bytes of each of 4, lost up
+// to half the time where rows are no powers of two (us a call, those and strips:
+// 1,280 triangles at 1408^3 247 and 122, at 2016^3 693 and 310, at 992^3 73 and
+// 62; torus of 400,000 at 1312^3 213 and 120; at 1024^3 69 and 68).
+// From kStreamedGrid on the table and the scratch table are beyond the 256 MB of
+// the last cache together, and the rows must not push the scratch words out of it
+// (1,280 at 1152^3 88 -> 74 us, at 1408^3 170 -> 122, at 2048^3 402 -> 310; at
+// 1056^3 69 either way).
+constexpr uint32_t kStripQuads = 1024;
+constexpr uint32_t kStripWords = 4u * kStripQuads + 4u * 80u;
+
+__host__ __device__ inline uint32_t strip_blocks(uint32_t rw) {  // K: a multiple of 4, up to 16 KB a strip
+    const uint32_t k = (kStripQuads / 4u / rw) & ~3u;
+    return k < 4u ? 4u : k;
+}
+
+template <int FORM>
+__global__ void __launch_bounds__(256) unblock_flagged_kernel(uint32_t* __restrict__ scratch,
+                                                              uint32_t* __restrict__ out, uint32_t G) {
+    __shared__ __align__(16) uint32_t lds[kStripWords];
+    const uint32_t rw = G >> 5, nb = G >> 2, K = strip_blocks(rw), unit = blockIdx.x;
+    const uint32_t strips = (nb + K - 1u) / K, bz = unit / strips, by = (unit - bz * strips) * K;
+    const uint32_t kk = nb - by < K ? nb - by : K, run = kk * rw;  // run: 16-byte groups of one z
+    const uint64_t q0 = (uint64_t)(bz * nb + by) * rw * 4u;
+    uint4* __restrict__ s4 = (uint4*)scratch + q0;
+    const uint32_t lane = (uint32_t)__lane_id();
+    uint8_t* flag = (uint8_t*)scratch - 1 - (q0 >> 4) - lane;
+    const bool set = lane < (run >> 2) && *flag != 0;
+    const unsigned long long flags = __ballot(set);
+    uint32_t* __restrict__ table = out + ((uint64_t)(4u * bz) * G + 4u * by) * rw;
+    const uint64_t slab = (uint64_t)G * rw;        // words of one z
+    const uint32_t inv = 65536u / rw + 1u;         // t / rw for t < 1024, rw <= 64
+    const bool whole = (rw & 3u) == 0;             // the 16-byte groups of a row are each of one flag
+    constexpr bool kQuads = FORM == kRowsStreamed || FORM == kRowsCached;
+    // this thread's group of each z, if it has words of a flagged group
+    bool hit = threadIdx.x < run && flags != 0;
+    if (kQuads && hit && whole) {
+        const uint32_t row = (4u * threadIdx.x * inv) >> 16;
+        hit = (flags >> (((row >> 2) * rw + 4u * threadIdx.x - row * rw) >> 2)) & 1ull;
+    }
+    if (kQuads) hit = threadIdx.x < run && ((__ballot(hit) >> (lane & 56u)) & 255ull);  // whole 128-byte lines
+    if (kQuads && threadIdx.x < run && !hit) {
+#pragma unroll
+        for (uint32_t z = 0; z < 4u; z++)
+            put_quad<FORM>((uint4*)(table + z * slab) + threadIdx.x, make_uint4(0u, 0u, 0u, 0u));
+    }
+    if (!flags) {
+        if (FORM == kRowsWords)
+            for (uint32_t z = 0; z < 4u; z++)
+                for (uint32_t i = threadIdx.x; i < 4u * run; i += 256u) table[z * slab + i] = 0u;
+        return;
+    }
+    const uint32_t plane = ((4u * run + 63u) & ~63u) + 16u;  // spreads the 4 planes over the banks
+    uint4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const uint32_t i = threadIdx.x + 256u * (uint32_t)u;
+        v[u] = (flags >> (i >> 4)) & 1ull ? s4[i] : make_uint4(0u, 0u, 0u, 0u);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const uint32_t i = threadIdx.x + 256u * (uint32_t)u, t = i >> 2;
+        if (v[u].x | v[u].y | v[u].z | v[u].w) s4[i] = make_uint4(0u, 0u, 0u, 0u);
+        if (i >= 4u * run) continue;
+        uint32_t* d = lds + (i & 3u) * plane + t + 3u * ((t * inv) >> 16) * rw;
+        d[0] = v[u].x;
+        d[rw] = v[u].y;
+        d[2u * rw] = v[u].z;
+        d[3u * rw] = v[u].w;
+    }
+    __syncthreads();
+    if (set && threadIdx.x < 64u) *flag = 0;  // every wave has read it
+#pragma unroll
+    for (uint32_t z = 0; z < 4u; z++) {
+        uint32_t* d = table + z * slab;
+        if (kQuads) {
+            if (hit) put_quad<FORM>((uint4*)d + threadIdx.x, *(const uint4*)(lds + z * plane + 4u * threadIdx.x));
+        } else {
+            for (uint32_t i = threadIdx.x; i < 4u * run; i += 256u) {
+                const uint32_t o = lds[z * plane + i];
+                if (FORM == kRowsAdded)
+                    table_or(d + i, o);
+                else
+                    d[i] = o;
+            }
+        }
+    }
+}
+
 // Rows that are no whole words (G not a multiple of 32; the scratch table's rows
 // are padded to words): 32 rows are G words of the linear table, from a word
 // boundary on, so a workgroup takes 32 rows into LDS, returns them to zero and
-// packs its G words.
-__device__ __forceinline__ void unblock_ragged(const ItemDev& it, uint32_t unit, uint32_t* rows) {
-    const uint32_t G = it.info.gridsize[0], rw = (G + 31u) >> 5, nrows = G * G, r0 = unit * 32u;
-    for (uint32_t i = threadIdx.x; i < 32u * rw; i += 256u) {
-        const uint32_t r = r0 + (i & 31u), w = i >> 5;  // four rows of a block are neighbours
-        uint32_t v = 0u;
-        if (r < nrows) {
-            uint32_t* p = it.scratch + blocked_word(G, w, r % G, r / G);
-            v = *p;
-            if (v) *p = 0u;
-        }
-        rows[(i & 31u) * rw + w] = v;
+// packs its G words.  The lanes of a load hold 32 rows of one word, which an odd
+// stride in LDS spreads over the banks (a stride of 32 words: torus of 400,000 at
+// 1000^3 127 us a call, with 33 122, with flags and empty rows left out 88).
+// FLAGS: as above, but a group's flag is read by the workgroups of its four z, so
+// the caller clears the flags afterwards.
+template <bool FLAGS>
+__device__ __forceinline__ void unblock_ragged(uint32_t* __restrict__ scratch, uint32_t* __restrict__ table, uint32_t G,
+                                               int accumulate, uint32_t unit, uint32_t* rows) {
+    const uint32_t rw = (G + 31u) >> 5, stride = rw | 1u, r0 = unit * 32u, r = r0 + (threadIdx.x & 31u);
+    const uint32_t y = r % G, z = r / G;  // four rows of a block are neighbours
+    bool any[4];
+    uint32_t v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const uint32_t w = (threadIdx.x >> 5) + 8u * (uint32_t)u;
+        any[u] = w < rw && z < G;
+        if (FLAGS && any[u]) any[u] = *((const uint8_t*)scratch - 1 - (blocked_word(G, w, y, z) >> 6)) != 0;
+    }
+    if (FLAGS && !__syncthreads_or(any[0] || any[1] || any[2] || any[3])) {  // 32 empty rows
+        const uint32_t total = (uint32_t)(((uint64_t)G * G * G + 31u) / 32u), w0 = unit * G;
+        if (!accumulate)
+            for (uint32_t k = threadIdx.x; k < G && w0 + k < total; k += 256u) table[w0 + k] = 0u;
+        return;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        v[u] = any[u] ? scratch[blocked_word(G, (threadIdx.x >> 5) + 8u * (uint32_t)u, y, z)] : 0u;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const uint32_t w = (threadIdx.x >> 5) + 8u * (uint32_t)u;
+        if (v[u]) scratch[blocked_word(G, w, y, z)] = 0u;
+        if (w < rw) rows[(threadIdx.x & 31u) * stride + w] = v[u];
     }
     __syncthreads();
-    pack_rows(rows, rw, G, r0, it.table, [&](uint32_t* d, uint32_t v) {
-        if (!it.accumulate)
-            *d = v;
+    pack_rows(rows, stride, rw, G, r0, table, [&](uint32_t* d, uint32_t p) {
+        if (!accumulate)
+            *d = p;
         else
-            table_or(d, v);
+            table_or(d, p);
     });
+}
+
+__global__ void __launch_bounds__(256) unblock_ragged_kernel(uint32_t* __restrict__ scratch,
+                                                             uint32_t* __restrict__ table, uint32_t G, int accumulate) {
+    __shared__ uint32_t rows[kRaggedWords];
+    unblock_ragged<true>(scratch, table, G, accumulate, blockIdx.x, rows);
+}
+
+__global__ void __launch_bounds__(256) clear_flags_kernel(uint4* __restrict__ flags, uint32_t quads) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < quads) flags[i] = make_uint4(0u, 0u, 0u, 0u);
 }
 
 __host__ __device__ inline bool unblock_vec(uint32_t G, const uint32_t* table) {
     return (G & 127u) == 0 && (((uintptr_t)table) & 15u) == 0;
 }
 
-template <bool FLAGS>
 __global__ void __launch_bounds__(256) unblock_kernel(ItemDev one, ItemMap M) {
     __shared__ BlockJob J;
+    __shared__ uint32_t rows[kRaggedWords];
     if (M.items) {
         resolve_job(one, M, blockIdx.x, J);
         if (J.local == ~0u) return;
     }
     const ItemDev& it = M.items ? J.it : one;
     const uint32_t local = M.items ? J.local : blockIdx.x;
-    if (!FLAGS && (it.info.gridsize[0] & 31u)) {
-        __shared__ uint32_t rows[kRaggedWords];
-        unblock_ragged(it, local, rows);
-        return;
-    }
-    unblock_quad<FLAGS>(it, local * 256u + threadIdx.x, FLAGS || unblock_vec(it.info.gridsize[0], it.table));
+    if (it.info.gridsize[0] & 31u)
+        unblock_ragged<false>(it.scratch, it.table, it.info.gridsize[0], it.accumulate, local, rows);
+    else
+        unblock_quad(it, local * 256u + threadIdx.x, unblock_vec(it.info.gridsize[0], it.table));
 }
 
 uint32_t unblock_units(uint32_t G, const uint32_t* table) {
     const uint64_t words = (uint64_t)G * G * G / 32u;
     if (G & 31u) return (G * G + 31u) / 32u;
-    return (uint32_t)((words / (unblock_vec(G, table) ? 16u : 4u) + 255u) / 256u);
+    if (G <= kUnflaggedGrid) return (uint32_t)((words / (unblock_vec(G, table) ? 16u : 4u) + 255u) / 256u);
+    const uint32_t nb = G >> 2, k = strip_blocks(G >> 5);
+    return nb * ((nb + k - 1u) / k);
+}
+
+static void launch_unblock_flagged(const ItemDev& one, uint32_t units, hipStream_t stream) {
+    const uint32_t G = one.info.gridsize[0];
+    if (G & 31u) {
+        unblock_ragged_kernel<<<units, 256, 0, stream>>>(one.scratch, one.table, G, one.accumulate);
+        const uint32_t quads = (uint32_t)(blocked_flags(G) / 16u);
+        clear_flags_kernel<<<(quads + 255u) / 256u, 256, 0, stream>>>((uint4*)one.scratch - quads, quads);
+        return;
+    }
+    const bool quads = (((uintptr_t)one.table) & 15u) == 0;
+    const auto kernel = one.accumulate ? unblock_flagged_kernel<kRowsAdded>
+                        : !quads       ? unblock_flagged_kernel<kRowsWords>
+                        : G >= kStreamedGrid ? unblock_flagged_kernel<kRowsStreamed> : unblock_flagged_kernel<kRowsCached>;
+    kernel<<<units, 256, 0, stream>>>(one.scratch, one.table, G);
 }
 
 hipError_t launch_unblock_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, hipStream_t stream) {
     if (units == 0) return hipSuccess;
     if (!M.items && one.flagged)
-        unblock_kernel<true><<<units, 256, 0, stream>>>(one, M);
+        launch_unblock_flagged(one, units, stream);
     else
-        unblock_kernel<false><<<units, 256, 0, stream>>>(one, M);
+        unblock_kernel<<<units, 256, 0, stream>>>(one, M);
     return hipGetLastError();
 }
 
@@ -550,11 +693,13 @@ hipError_t launch_unblock_jobs(const ItemDev& one, const ItemMap& M, uint32_t un
 // 100,003 at 256^3 88 -> 67; displaced sphere of 81,920 at 256^3 31 -> 21, at
 // 512^3 65 -> 37, 327,680 at 512^3 92 -> 60; torus of 200,000 at 256^3 19 -> 14;
 // with flags: 81,920 at 1024^3 149 -> 86, at 2048^3 728 -> 300; torus of
-// 1,048,576 at 1024^3 105 -> 76.  The flags save the row pass most of the
-// scratch table at 1024^3 and above (81,920 at 1024^3 103 -> 86); at 512^3 and below setting them costs more than that (327,680 at 256^3
-// 41 without, 46 with).  Grids whose rows are no whole words: torus of 26,866 at
-// 200^3 16.7 -> 14.2, soup of 100,000 at 201^3 89 -> 48, displaced sphere of 81,920
-// at 200^3 32 -> 18.
+// 1,048,576 at 1024^3 105 -> 76.  The flags save the row pass most of the scratch
+// table from about 640^3 on; below, setting them costs more than that (327,680 at
+// 256^3 41 without, 46 with; at 544^3 66 and 71).  Grids whose rows are no whole
+// words: torus of 26,866 at 200^3 16.7 -> 14.2, soup of 100,000 at 201^3 89 -> 48,
+// displaced sphere of 81,920 at 200^3 32 -> 18, torus of 200,000 at 1000^3 105 ->
+// 99.  No mesh of 1,280 to 1,310,720 triangles measured slower than with the rows
+// of the table as keys at any grid of 200 to 2048.
 bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles) {
     const uint64_t words = (uint64_t)G * G * G / 32u;
     return layout == VOX_LAYOUT_LINEAR && G <= ((G & 31u) ? kRaggedGrid : kBlockedGrid) &&
@@ -747,8 +892,8 @@ hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_
     if (scratch && info.n_triangles && chunk_blocked(layout, G, info.n_triangles)) {
         hipError_t e = hipSuccess;
         const uint64_t bytes = blocked_bytes(G);
-        one.flagged = G > kUnflaggedGrid && unblock_vec(G, table) ? 1u : 0u;
-        const uint64_t flags = one.flagged ? bytes / 256u : 0u;
+        one.flagged = G > kUnflaggedGrid ? 1u : 0u;
+        const uint64_t flags = one.flagged ? blocked_flags(G) : 0u;
         ScratchLease S(stream);
         if (uint32_t* words = S.table(bytes + flags)) {
             one.scratch = words + flags / 4u;

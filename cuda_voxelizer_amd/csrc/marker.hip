@@ -402,7 +402,7 @@ __global__ void __launch_bounds__(256) suffix_ragged_kernel(uint32_t* __restrict
     __syncthreads();
     tile_suffix(rows, rw, rw, 32u, [&](uint32_t r, uint32_t j, uint32_t fin) { rows[r * rw + j] = fin; });
     __syncthreads();
-    pack_rows(rows, rw, G, r0, table, [&](uint32_t* d, uint32_t v) {
+    pack_rows(rows, rw, rw, G, r0, table, [&](uint32_t* d, uint32_t v) {
         if (!accumulate)
             *d = v;
         else if (v)

@@ -106,6 +106,17 @@ inline bool prefer_direct_solid(uint64_t n_triangles, uint32_t G) {
 inline bool prefer_direct_ragged(uint64_t n_triangles, uint32_t G) {
     return (G & 31u) != 0 && G <= 128u && n_triangles >= (uint64_t)G * G;
 }
+// Coarse solids whose rows are no whole 16-byte groups work in the caller's table,
+// which marker's row pass then reads and writes: on large grids that loses to the
+// tiles (us, tile and marker: torus of 400,000 at 1312^3 264 and 272, at 1504^3 349
+// and 442, at 2016^3 782 and 921; displaced sphere of 327,680 at 1504^3 477 and
+// 524), but for few triangles of many columns each (81,920 at 1504^3 579 and 518,
+// at 2016^3 1586 and 1085) and on smaller grids (327,680 at 1184^3 265 and 223,
+// torus of 400,000 at 1056^3 167 and 158).
+inline bool prefer_tile_solid(int layout, bool accumulate, uint64_t n_triangles, uint32_t G) {
+    return layout == VOX_LAYOUT_LINEAR && !accumulate && (G & 31u) == 0 && (G & 127u) != 0 && G > 1184u &&
+           24ull * n_triangles >= (uint64_t)G * G && coarse_mesh(n_triangles, G);
+}
 hipError_t launch_fill_zero(const vox_info& info, uint32_t* table, hipStream_t stream);
 uint32_t fill_units(uint32_t G);
 uint32_t chunk_span(uint32_t G, uint64_t n_triangles, bool lone);
@@ -130,30 +141,33 @@ inline uint64_t blocked_bytes(uint32_t G) {
     const uint64_t nb = (G + 3u) >> 2;
     return nb * nb * ((G + 31u) >> 5) * 64u;
 }
+// Bytes of flags before a flagged table: one for each 256 bytes of it.
+inline uint64_t blocked_flags(uint32_t G) { return (blocked_bytes(G) / 256u + 256u) & ~255ull; }
 // Grids whose rows are no whole words are packed from padded rows up to this one.
 constexpr uint32_t kRaggedGrid = 1024;
-constexpr uint32_t kRaggedWords = 32u * (kRaggedGrid / 32u);
-// 32 rows of rw words in LDS, from row r0 on -> their words of the linear table
+constexpr uint32_t kRaggedWords = 32u * (kRaggedGrid / 32u + 1u);
+// 32 rows of rw words in LDS, `stride` words apart, from row r0 on -> their words of the linear table
 // (fewer at its end; bits from G on are zero in every row): put(word, value) for
 // each.  A word has bits of at most two rows (G > 32).
 template <class Put>
-__device__ __forceinline__ void pack_rows(const uint32_t* rows, uint32_t rw, uint32_t G, uint32_t r0,
+__device__ __forceinline__ void pack_rows(const uint32_t* rows, uint32_t stride, uint32_t rw, uint32_t G, uint32_t r0,
                                           uint32_t* __restrict__ table, Put&& put) {
     const uint32_t total = (uint32_t)(((uint64_t)G * G * G + 31u) / 32u), w0 = r0 / 32u * G;
     for (uint32_t k = threadIdx.x; k < G; k += blockDim.x) {
         if (w0 + k >= total) return;
         const uint32_t b = k * 32u, r = b / G, x = b - r * G;
-        const uint32_t* p = rows + r * rw + (x >> 5);
+        const uint32_t* p = rows + r * stride + (x >> 5);
         const uint32_t lo = p[0], hi = (x >> 5) + 1u < rw ? p[1] : 0u, s = x & 31u;
         uint32_t v = s ? (lo << s) | (hi >> (32u - s)) : lo;
-        if (G - x < 32u && r < 31u) v |= rows[(r + 1u) * rw] >> (G - x);
+        if (G - x < 32u && r < 31u) v |= rows[(r + 1u) * stride] >> (G - x);
         put(table + w0 + k, v);
     }
 }
 constexpr int kBlockedSpecs = kSpecBlocked + 1;  // what a batch's classes may be
 constexpr uint32_t kBlockedGrid = 2048;
-constexpr uint32_t kUnflaggedGrid = 512;
-constexpr uint32_t kStreamedGrid = 1312;  // tables above 256 MiB
+constexpr uint32_t kUnflaggedGrid = 608;
+constexpr uint32_t kBatchBlockedGrid = 512;
+constexpr uint32_t kStreamedGrid = 1152;
 bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles);
 uint32_t unblock_units(uint32_t G, const uint32_t* table);
 hipError_t launch_unblock_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, hipStream_t stream);
