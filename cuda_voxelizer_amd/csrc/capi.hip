@@ -193,6 +193,9 @@ vox_status run(const vox_info* info, const float* d_tris, uint32_t* d_table, int
     else if (flags & VOX_FLAG_ALGO_MARKER) algo = have_marker ? MARKER : (have_plan ? TILE : DIRECT);
     else if (solid && prefer_direct_solid(info->n_triangles, G)) algo = DIRECT;
     else if (solid && prefer_direct_ragged(info->n_triangles, G)) algo = DIRECT;
+    else if (solid && have_plan && prefer_tile_solid(layout, accumulate, info->n_triangles, G) &&
+             !ScratchLease(st).recording())
+        algo = TILE;
     else if (solid) algo = have_marker ? MARKER : (have_plan ? TILE : DIRECT);
     else algo = chunk_supported(G) ? CHUNK : (have_plan ? TILE : DIRECT);
     hipError_t e;
