@@ -46,15 +46,14 @@ __device__ __forceinline__ ColBox column_box(const SolidTri& S, int G) {
 // Records of one round: their columns together stay below 2^32.
 __device__ __forceinline__ int column_recs(int G) { return G <= 4096 ? kColRecs : 8; }  // 64 * 2^24, 8 * 2^28
 
-// Columns of the threads with `big`, whose triangle and box are S and B.
+// Columns of the threads with `big`, whose triangle and box setup(S, B) gives.
 // count[w]: the number of them in wave w (written by that wave before a
 // barrier).  Of the windows this workgroup takes every `stride`-th of a wave's
 // from `first` on.  hit(S, y, z, py, pz) is called for every hit column.  All
 // threads of the workgroup call this.
-template <int WAVES, class Hit>
-__device__ __forceinline__ void block_columns(ColRec* rec, const uint32_t* count, const SolidTri& S, const ColBox& B,
-                                              bool big, const vox_info& info, uint32_t first, uint32_t stride,
-                                              Hit&& hit) {
+template <int WAVES, class Setup, class Hit>
+__device__ __forceinline__ void block_columns(ColRec* rec, const uint32_t* count, Setup&& setup, bool big,
+                                              const vox_info& info, uint32_t first, uint32_t stride, Hit&& hit) {
     const int lane = __lane_id(), wave = (int)(threadIdx.x >> 6);
     int rank = 0, nq = 0;
 #pragma unroll
@@ -70,7 +69,8 @@ __device__ __forceinline__ void block_columns(ColRec* rec, const uint32_t* count
         __syncthreads();  // the previous round's records have been read
         if (big && rank >= r0 && rank < r0 + nr) {
             ColRec& R = rec[rank - r0];
-            R.S = S;
+            ColBox B;
+            setup(R.S, B);
             R.ylo = B.ylo;
             R.zlo = B.zlo;
             R.ny = B.ny;

@@ -149,9 +149,14 @@ __global__ void __launch_bounds__(kMBlock)
     const int lg = (int)it.lg_split;
     const uint32_t per = (uint32_t)kMBlock >> lg, parts = it.parts > 1u ? it.parts : 1u;
     // the parts of a unit are a grid's width apart, so part 0, which has the lanes' own columns too, comes first
-    const uint32_t units = (uint32_t)((n + per - 1) / per);
-    const uint32_t part = parts > 1u ? local / units : 0u;
-    const uint64_t first = (uint64_t)(local - part * units) * per;
+    uint32_t part = 0, unit = local;
+    if (parts > 1u) {  // (no division for the others)
+        const uint32_t units = (uint32_t)((n + per - 1) >> (8 - lg));
+        part = local / units;
+        unit -= part * units;
+    }
+    static_assert(kMBlock == 256, "per = 2^(8 - lg)");
+    const uint64_t first = (uint64_t)unit * per;
     if (first >= n || part >= parts) return;
     const int G = (int)info.gridsize[0];
     const uint64_t total_bits = (uint64_t)G * G * G;
@@ -163,9 +168,10 @@ __global__ void __launch_bounds__(kMBlock)
         __syncthreads();  // the LDS hash is set
     }
     unsigned long long offrow = 0;
+    const bool blocked = !MULTI && it.flagged != 0u;  // a batch's markers lie in its jobs' tables
     const auto run = [&](const SolidTri& S, int y, int z, float py, float pz) {
         column_run<REG>(table, column_xmax(S, info, py, pz), y, z, (uint32_t)G, total_bits, ws, offrow, spills != 0,
-                        jobtag, it.flagged != 0u, H, RA);
+                        jobtag, blocked, H, RA);
     };
     const uint64_t mine = first + (threadIdx.x >> lg);
     const int sub = (int)(threadIdx.x & ((1u << lg) - 1u)), step = 1 << lg;
@@ -205,7 +211,20 @@ __global__ void __launch_bounds__(kMBlock)
     const unsigned long long queued = __ballot(big);
     if (__lane_id() == 0) nbig[threadIdx.x >> 6] = (uint32_t)__popcll(queued);
     __syncthreads();
-    block_columns<kMBlock / 64>(recs, nbig, S, B, big, info, part, parts, run);
+    const auto setup = [&](SolidTri& Q, ColBox& C) {
+        if (MULTI) {  // again, from memory: held in registers they cost two waves per SIMD (25 us, 23)
+            float v[3][3];
+            load_tri(tris, mine, info, v);
+            SolidTri T;
+            solid_setup(v, info, T);
+            Q = T;
+            C = column_box(T, G);
+        } else {
+            Q = S;
+            C = B;
+        }
+    };
+    block_columns<kMBlock / 64>(recs, nbig, setup, big, info, part, parts, run);
     if (offrow_out && offrow) atomicAdd(offrow_out, offrow);
     if constexpr (REG) {
         __syncthreads();  // every marker of the workgroup is in the hash
@@ -757,20 +776,23 @@ bool marker_supported(uint32_t G, int layout, bool accumulate) {
 // by that.  A coarse mesh (fewer than G^2/4 triangles) has triangles of many
 // columns: boxes of more than 8 (kMBigCols) are dealt, and further parts take
 // their share of them, up to about 1024 workgroups.  In a batch the other jobs
-// fill the device, so its coarse jobs aim at 256 and its others share nothing.  Measured (us per call;
-// the triangles one after the other over a workgroup of 256 -> this):
-// icosphere 1,280 at 256^3 360 -> 17, 5,120 at 256^3 300 -> 18, 20,480 at
-// 576^3 349 -> 62; displaced sphere 20,480 at 512^3 277 -> 33, 81,920 at
-// 1024^3 346 -> 124 (the row pass takes 58 of it).  From G^2/4 on a limit of 8
+// fill the device, so its coarse jobs aim at 256, and its others share theirs up to
+// 256 (one displaced sphere of 1,280 at 64^3 a batch 30 us shared by none, 23; of
+// 20,480 at 256^3 32 and 25; six of 20,480 at 128^3 25, and 44 with 1280).
+// Measured (us per call; the triangles one after the other over a workgroup of
+// 256 -> this): icosphere 1,280 at 256^3 360 -> 17, 5,120 at 256^3 300 -> 18,
+// 20,480 at 576^3 349 -> 62; displaced sphere 20,480 at 512^3 277 -> 33, 81,920
+// at 1024^3 346 -> 124 (the row pass takes 58 of it).  From G^2/4 on a limit of 8
 // loses: displaced sphere 20,480 at 256^3 20 with 32 columns, 26 with 8.
 static void marker_shape(ItemDev& it, bool lone) {
     const uint64_t n = it.info.n_triangles;
     if (n == 0) return;
     const bool coarse = coarse_mesh(n, it.info.gridsize[0]);
-    if (lone)
-        while (it.lg_split < 4u && n << (it.lg_split + 1u) <= 327680u) it.lg_split++;
+    const uint64_t lanes = lone ? 327680u : 65536u;
+    if (!lone && coarse)
+        it.lg_split = 3u;
     else
-        it.lg_split = coarse ? 3u : 0u;
+        while (it.lg_split < 4u && n << (it.lg_split + 1u) <= lanes) it.lg_split++;
     if (!coarse) return;
     if (!it.big) it.big = kMBigColsCoarse;
     const uint64_t units = ((n << it.lg_split) + kMBlock - 1) / kMBlock;
