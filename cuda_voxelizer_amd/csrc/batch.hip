@@ -29,6 +29,7 @@ struct JobClass {
     uint32_t total_a = 0, total_b = 0, total_c = 0;
     uint32_t max_tile_words = 0;
     bool loop = false;  // chunk class: some job takes several chunks per workgroup
+    bool split = false; // chunk class: some job's triangles are shared by several lanes
     size_t off_items = 0, off_a = 0, off_b = 0, off_c = 0;
 };
 
@@ -56,9 +57,8 @@ struct vox_batch {
     hipEvent_t done = nullptr;
     bool scratch_dirty = false;  // a launch failed between the scratch tables' use and their clearing
     voxamd::WorkspaceLayout L{};
-    // chunk / chunkw (6 waves per SIMD): one class per layout specialisation (ChunkSpec)
-    voxamd::JobClass fill, chunk[voxamd::kBlockedSpecs], chunkw[voxamd::kBlockedSpecs], unblock, marker, dsurf, dsolid,
-        tsurf, tsolid;
+    // chunk: one class per layout specialisation (ChunkSpec); chunkw: layout-generic jobs at 6 waves per SIMD
+    voxamd::JobClass fill, chunk[voxamd::kBlockedSpecs], chunkw, unblock, marker, dsurf, dsolid, tsurf, tsolid;
     int count = 0;
     uint64_t total_triangles = 0;
 };
@@ -90,13 +90,14 @@ static hipError_t launch_chunk_classes(vox_batch* b, hipStream_t s, ChunkClassSe
     hipError_t e = hipSuccess;
     for (int sp = 0; sp < kBlockedSpecs; sp++) {
         if ((which == kBlockedChunkClass) != (sp == kSpecBlocked)) continue;
-        const JobClass& c5 = b->chunk[sp];
-        const JobClass& c6 = b->chunkw[sp];
-        if (c5.total_a && (e = launch_chunk_jobs(dummy, c5.m_a, c5.total_a, c5.loop, s, 5, sp)) != hipSuccess)
-            return e;
-        if (c6.total_a && (e = launch_chunk_jobs(dummy, c6.m_a, c6.total_a, c6.loop, s, 6, sp)) != hipSuccess)
+        const JobClass& c = b->chunk[sp];
+        if (c.total_a && (e = launch_chunk_jobs(dummy, c.m_a, c.total_a, c.loop, s, 5, sp, c.split)) != hipSuccess)
             return e;
     }
+    const JobClass& w = b->chunkw;
+    if (which == kFilledChunkClasses && w.total_a &&
+        (e = launch_chunk_jobs(dummy, w.m_a, w.total_a, w.loop, s, 6, kSpecAny, w.split)) != hipSuccess)
+        return e;
     if (which == kBlockedChunkClass) return launch_unblock_jobs(dummy, b->unblock.m_a, b->unblock.total_a, s);
     return hipSuccess;
 }
@@ -161,8 +162,8 @@ static hipError_t launch_forked(vox_batch* b, hipStream_t m) {
     hipError_t e = hipSuccess;
     uint64_t filled = 0, blocked = 0;  // triangles of the two chunk chains
     for (int sp = 0; sp < kBlockedSpecs; sp++)
-        for (const JobClass* c : {&b->chunk[sp], &b->chunkw[sp]})
-            for (const ItemDev& it : c->items) (sp == kSpecBlocked ? blocked : filled) += it.info.n_triangles;
+        for (const ItemDev& it : b->chunk[sp].items) (sp == kSpecBlocked ? blocked : filled) += it.info.n_triangles;
+    for (const ItemDev& it : b->chunkw.items) filled += it.info.n_triangles;
     const bool filled_first = 2 * filled >= blocked;
     hipStream_t fs = filled_first ? m : b->side[3], bs = filled_first ? b->side[3] : m;
 #define VOX_TRY(x) \
@@ -220,15 +221,14 @@ struct BatchPlan {
 constexpr uint64_t kBatchScratch = 1ull << 30;
 
 // Every chunk class and the others, in the order of the packed image.
-constexpr int kClasses = 2 * kBlockedSpecs + 7;
+constexpr int kClasses = kBlockedSpecs + 8;
 struct ClassList {
     JobClass* c[kClasses];
     explicit ClassList(vox_batch* b) {
         int k = 0;
         c[k++] = &b->fill;
         for (JobClass& j : b->chunk) c[k++] = &j;
-        for (JobClass& j : b->chunkw) c[k++] = &j;
-        for (JobClass* j : {&b->unblock, &b->marker, &b->dsurf, &b->dsolid, &b->tsurf, &b->tsolid}) c[k++] = j;
+        for (JobClass* j : {&b->chunkw, &b->unblock, &b->marker, &b->dsurf, &b->dsolid, &b->tsurf, &b->tsolid}) c[k++] = j;
     }
     JobClass** begin() { return c; }
     JobClass** end() { return c + kClasses; }
@@ -254,7 +254,8 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
     if (count < 0 || (count > 0 && !items)) return fail(VOX_ERR_INVALID, "bad item array");
     reset_classes(b);
     b->count = count;
-    uint64_t tri_sum_surf = 0, tri_sum_solid = 0;
+    uint64_t tri_sum_surf = 0, tri_sum_solid = 0, surface_triangles = 0;
+    for (int i = 0; i < count; i++) surface_triangles += items[i].solid ? 0u : items[i].info.n_triangles;
     for (int i = 0; i < count; i++) {
         const vox_batch_item& it = items[i];
         vox_status s = validate(&it.info, it.d_tris, it.d_table, it.layout);
@@ -277,6 +278,7 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
         else if (algo & VOX_FLAG_ALGO_CHUNK) a = chunk_supported(G) ? CHUNK : DIRECT;
         else if (algo & VOX_FLAG_ALGO_MARKER) a = have_marker ? MARKER : (have_plan ? TILE : DIRECT);
         else if (solid && prefer_direct_solid(it.info.n_triangles, G)) a = DIRECT;
+        else if (solid && have_plan && prefer_tile_solid(it.layout, accumulate, it.info.n_triangles, G)) a = TILE;
         else if (solid && have_marker) a = MARKER;
         else if (solid) a = have_plan ? TILE : DIRECT;
         else a = chunk_supported(G) ? CHUNK : (have_plan ? TILE : DIRECT);
@@ -309,8 +311,7 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
             add_prefix(b->marker.base_c, b->marker.total_c, n);  // triangles (spill overflow pass)
         } else if (a == CHUNK) {
             d.span = chunk_span(G, n, false);
-            d.parts = chunk_parts(G, n);
-            if (!d.big) d.big = chunk_big(G, n);
+            if (d.span <= 1u) chunk_batch_shape(d, surface_triangles <= kSharedBatch);
             // jobs that loop over chunks run in the 4-wave form (any layout): they stay in the 5-wave class;
             // a layout-specialised kernel runs at six waves per SIMD under either bound, so only
             // layout-generic jobs are split by the waves knob (each class is one more kernel)
@@ -323,10 +324,11 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
                 add_prefix(b->unblock.base_a, b->unblock.total_a, unblock_units(G, it.d_table));
             }
             const bool wide = tune_waves(it.flags) == 6 && !loop && sp == kSpecAny;
-            JobClass& c = wide ? b->chunkw[sp] : b->chunk[sp];
+            JobClass& c = wide ? b->chunkw : b->chunk[sp];
             if (loop) c.loop = true;
+            if (d.lg_split) c.split = true;
             c.items.push_back(d);
-            add_prefix(c.base_a, c.total_a, chunk_units(n, d.span, d.parts));
+            add_prefix(c.base_a, c.total_a, chunk_units(n, d.span, d.parts, d.lg_split));
         } else if (a == DIRECT) {
             JobClass& c = solid ? b->dsolid : b->dsurf;
             c.items.push_back(d);
@@ -525,7 +527,8 @@ vox_status vox_batch_info(const vox_batch* b, int64_t out[8]) {
     out[0] = b->count;
     out[1] = (int64_t)b->total_triangles;
     out[2] = 0;
-    for (int sp = 0; sp < kBlockedSpecs; sp++) out[2] += (int64_t)(b->chunk[sp].items.size() + b->chunkw[sp].items.size());
+    for (const JobClass& c : b->chunk) out[2] += (int64_t)c.items.size();
+    out[2] += (int64_t)b->chunkw.items.size();
     out[3] = (int64_t)b->tsurf.items.size();
     out[4] = (int64_t)b->tsolid.items.size();
     out[5] = (int64_t)(b->dsurf.items.size() + b->dsolid.items.size());

@@ -283,7 +283,7 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE || (SPEC != kSpecAny 
     const uint32_t per = (uint32_t)kChunk >> lg;
     uint32_t part = 0, unit = local;
     if (parts > 1u) {  // in the looping form too: its launch may hold jobs of either kind
-        const uint32_t units = (uint32_t)((n + per - 1) / per);
+        const uint32_t units = (uint32_t)((n + per - 1) >> (8 - lg));
         part = unit / units;
         unit -= part * units;
     }
@@ -729,17 +729,6 @@ uint32_t chunk_span(uint32_t G, uint64_t n_triangles, bool lone) {
     return s < 1 ? 1u : (s > 16 ? 16u : (uint32_t)s);
 }
 
-// Parts per chunk of a batch's job, whose other jobs fill the device as well
-// (a lone call: chunk_shape).  A coarse mesh (fewer than G^2/4 triangles) has few
-// chunks of large triangles: their row windows are shared by up to 32 parts,
-// aiming at 256 workgroups per job.
-uint32_t chunk_parts(uint32_t G, uint64_t n_triangles) {
-    if (!coarse_mesh(n_triangles, G)) return 1u;
-    const uint64_t chunks = (n_triangles + kChunk - 1) / kChunk;
-    const uint64_t p = chunks ? 256 / chunks : 1;
-    return p < 1 ? 1u : (p > 32 ? 32u : (uint32_t)p);
-}
-
 uint32_t chunk_units(uint64_t n_triangles, uint32_t span, uint32_t parts, uint32_t lg_split) {
     const uint64_t per = (uint32_t)kChunk >> lg_split;
     const uint64_t chunks = (n_triangles + per - 1) / per;
@@ -760,46 +749,64 @@ int chunk_spec(int layout, uint32_t G) {
     return kSpecAny;
 }
 
-template <bool MULTI, bool WIDE, bool SPLIT = false>
+template <bool MULTI, bool SPLIT>
 static void launch_chunk_spec(int spec, uint32_t units, hipStream_t stream, const ItemDev& one, const ItemMap& M) {
     const RegionArgs none{};
     if (spec == kSpecLinear)
-        surface_chunk_kernel<MULTI, false, WIDE, false, kSpecLinear, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
+        surface_chunk_kernel<MULTI, false, false, false, kSpecLinear, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
     else if (spec == kSpecBlocked)
-        surface_chunk_kernel<MULTI, false, WIDE, false, kSpecBlocked, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
+        surface_chunk_kernel<MULTI, false, false, false, kSpecBlocked, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
     else if (!MULTI && spec == kSpecFlagged)
-        surface_chunk_kernel<false, false, WIDE, false, kSpecFlagged, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
-    else if (spec == kSpecMorton)
-        surface_chunk_kernel<MULTI, false, WIDE, false, kSpecMorton, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
+        surface_chunk_kernel<false, false, false, false, kSpecFlagged, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
     else
-        surface_chunk_kernel<MULTI, false, WIDE, false, kSpecAny, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
+        surface_chunk_kernel<MULTI, false, false, false, kSpecMorton, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
 }
 
-// waves: 5 or 6 waves per SIMD for the one-chunk form (0: 6 for the linear
-// layout, 5 for Morton -- the measured better choice for each; a layout-
-// specialised form needs few enough registers to run at six either way); the
-// chunk loop always runs at 4.  spec: the layout every job of M shares
-// (chunk_spec of each, or kSpecAny); a single job's comes from `one`.
-hipError_t launch_chunk_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, bool loop, hipStream_t stream,
-                             int waves, int spec) {
-    if (units == 0) return hipSuccess;
-    const bool wide = waves == 6 || (waves == 0 && !M.items && one.layout == VOX_LAYOUT_LINEAR);
-    if (!M.items) spec = one.scratch ? (int)(one.flagged ? kSpecFlagged : kSpecBlocked) : chunk_spec(one.layout, one.info.gridsize[0]);
+template <bool MULTI, bool SPLIT>
+static void launch_chunk_any(bool wide, uint32_t units, hipStream_t stream, const ItemDev& one, const ItemMap& M) {
     const RegionArgs none{};
-    if (loop && M.items)
-        surface_chunk_kernel<true, true, false, false><<<units, kChunk, 0, stream>>>(one, M, none);
-    else if (loop)
-        surface_chunk_kernel<false, true, false, false><<<units, kChunk, 0, stream>>>(one, M, none);
-    else if (M.items && wide)
-        launch_chunk_spec<true, true>(spec, units, stream, one, M);
-    else if (M.items)
-        launch_chunk_spec<true, false>(spec, units, stream, one, M);
-    else if (one.lg_split)
-        launch_chunk_spec<false, false, true>(spec, units, stream, one, M);
-    else if (wide)
-        launch_chunk_spec<false, true>(spec, units, stream, one, M);
+    if (wide)
+        surface_chunk_kernel<MULTI, false, true, false, kSpecAny, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
     else
-        launch_chunk_spec<false, false>(spec, units, stream, one, M);
+        surface_chunk_kernel<MULTI, false, false, false, kSpecAny, SPLIT><<<units, kChunk, 0, stream>>>(one, M, none);
+}
+
+template <bool MULTI>
+static void launch_chunk_form(int spec, bool split, bool wide, uint32_t units, hipStream_t stream, const ItemDev& one,
+                              const ItemMap& M) {
+    if (spec == kSpecAny && split)
+        launch_chunk_any<MULTI, true>(wide, units, stream, one, M);
+    else if (spec == kSpecAny)
+        launch_chunk_any<MULTI, false>(wide, units, stream, one, M);
+    else if (split)
+        launch_chunk_spec<MULTI, true>(spec, units, stream, one, M);
+    else
+        launch_chunk_spec<MULTI, false>(spec, units, stream, one, M);
+}
+
+// waves: 5 or 6 waves per SIMD for the layout-generic one-chunk form (0: 6 for a
+// lone linear job without shared triangles, 5 otherwise); the layout-specialised
+// ones need few enough registers to run at six (lone) or five whatever it is, and
+// the chunk loop always runs at 4.  spec: the layout every job of M shares
+// (chunk_spec of each, or kSpecAny); a single job's comes from `one`.  split: some
+// job of M has lg_split.
+hipError_t launch_chunk_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, bool loop, hipStream_t stream,
+                             int waves, int spec, bool split) {
+    if (units == 0) return hipSuccess;
+    const RegionArgs none{};
+    if (loop && M.items) {
+        // its other jobs may be split
+        surface_chunk_kernel<true, true, false, false, kSpecAny, true><<<units, kChunk, 0, stream>>>(one, M, none);
+    } else if (loop) {
+        surface_chunk_kernel<false, true, false, false><<<units, kChunk, 0, stream>>>(one, M, none);
+    } else if (M.items) {
+        launch_chunk_form<true>(spec, split, waves == 6, units, stream, one, M);
+    } else {
+        spec = one.scratch ? (int)(one.flagged ? kSpecFlagged : kSpecBlocked)
+                           : chunk_spec(one.layout, one.info.gridsize[0]);
+        const bool wide = waves == 6 || (waves == 0 && !one.lg_split && one.layout == VOX_LAYOUT_LINEAR);
+        launch_chunk_form<false>(spec, one.lg_split != 0u, wide, units, stream, one, M);
+    }
     return hipGetLastError();
 }
 
@@ -818,7 +825,7 @@ static ItemDev single_job(const vox_info& info, const float* tris, uint32_t* tab
 // mesh of few triangles, whose workgroups would wait for their largest boxes; 64
 // in a coarser one of more (81,920 at 1024^3: 165 us at 256 voxels, 150 at 64; at
 // 512^3 66 and 80).
-uint32_t chunk_big(uint32_t G, uint64_t n) {
+static uint32_t chunk_big(uint32_t G, uint64_t n) {
     const uint64_t g2 = (uint64_t)G * G;
     if (n == 0 || 8ull * n >= 5ull * g2) return 0u;
     return n <= 32768u ? 16u : (8u * n < g2 ? 64u : 0u);
@@ -855,6 +862,29 @@ static void chunk_shape(ItemDev& one) {
     } else {
         one.parts = one.lg_split <= 1u && n <= 262144u ? 2u : 1u;
     }
+}
+
+// The work shape of a batch's job.  A mesh of large triangles is a long chain of
+// rounds to each of its few workgroups.  In a batch of few triangles (share) it is
+// shared as a lone call's is, up to 16 lanes a triangle and 16 parts, but by about
+// 512 workgroups only; in one of more, whose other jobs fill the device meanwhile,
+// a coarse one (fewer than G^2/4 triangles) has up to 32 parts, for 256 workgroups:
+// there the form of the kernel that shares triangles costs the others more than it
+// gains.  Measured (us a launch, parts only and shared): displaced sphere of 1,280
+// at 64^3 93 and 20, of 20,480 at 256^3 94 and 37, six of them 104 and 78; mixed
+// meshes, 13 of 0.9 million triangles 151 and 125, 24 of 1.7 million 152 and 149,
+// 48 of 3.5 million 443 and 459.
+void chunk_batch_shape(ItemDev& it, bool share) {
+    const uint64_t n = it.info.n_triangles, G = it.info.gridsize[0];
+    it.parts = 1;
+    if (!it.big) it.big = chunk_big((uint32_t)G, n);
+    if (n == 0 || (share ? 8u * n >= 5u * G * G : !coarse_mesh(n, (uint32_t)G))) return;
+    while (share && it.lg_split < 4u && n << (it.lg_split + 1u) <= 131072u) it.lg_split++;
+    const uint64_t units = ((n << it.lg_split) + kChunk - 1) / kChunk;
+    uint64_t p = (share ? 512u : 256u) / units;
+    if (share && p > G * G / (2u * n)) p = G * G / (2u * n);
+    const uint64_t most = share ? 16u : 32u;
+    it.parts = p < 1u ? 1u : (p > most ? (uint32_t)most : (uint32_t)p);
 }
 
 hipError_t launch_fill_zero(const vox_info& info, uint32_t* table, hipStream_t stream) {

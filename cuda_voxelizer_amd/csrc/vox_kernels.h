@@ -120,8 +120,8 @@ inline bool prefer_tile_solid(int layout, bool accumulate, uint64_t n_triangles,
 hipError_t launch_fill_zero(const vox_info& info, uint32_t* table, hipStream_t stream);
 uint32_t fill_units(uint32_t G);
 uint32_t chunk_span(uint32_t G, uint64_t n_triangles, bool lone);
-uint32_t chunk_parts(uint32_t G, uint64_t n_triangles);
-uint32_t chunk_big(uint32_t G, uint64_t n_triangles);
+void chunk_batch_shape(ItemDev& it, bool share);
+constexpr uint64_t kSharedBatch = 1500000;  // triangles of a batch's surfaces
 uint32_t chunk_units(uint64_t n_triangles, uint32_t span, uint32_t parts, uint32_t lg_split = 0);
 hipError_t launch_fill_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, hipStream_t stream);
 // What a chunk kernel instantiation knows of its jobs' layout: nothing, linear
@@ -130,7 +130,7 @@ hipError_t launch_fill_jobs(const ItemDev& one, const ItemMap& M, uint32_t units
 enum ChunkSpec : int { kSpecAny = 0, kSpecLinear = 1, kSpecMorton = 2, kSpecBlocked = 3, kSpecFlagged = 4 };
 int chunk_spec(int layout, uint32_t G);
 hipError_t launch_chunk_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, bool loop, hipStream_t stream,
-                             int waves = 0, int spec = kSpecAny);
+                             int waves = 0, int spec = kSpecAny, bool split = false);
 hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_t* table, int layout, bool accumulate,
                                 hipStream_t stream, uint32_t big = 0, int waves = 0, bool scratch = true);
 // Word w of row (y, z) in a blocked table: the 4 x 4 rows of a block lie together.
