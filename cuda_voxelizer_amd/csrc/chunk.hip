@@ -592,10 +592,12 @@ __device__ __forceinline__ void unblock_ragged(uint32_t* __restrict__ scratch, u
                                                int accumulate, uint32_t unit, uint32_t* rows) {
     const uint32_t rw = (G + 31u) >> 5, stride = rw | 1u, r0 = unit * 32u, r = r0 + (threadIdx.x & 31u);
     const uint32_t y = r % G, z = r / G;  // four rows of a block are neighbours
-    bool any[4];
+    const int passes = (int)((rw + 7u) >> 3);
+    bool any[4] = {false, false, false, false};
     uint32_t v[4];
 #pragma unroll
     for (int u = 0; u < 4; u++) {
+        if (u >= passes) break;
         const uint32_t w = (threadIdx.x >> 5) + 8u * (uint32_t)u;
         any[u] = w < rw && z < G;
         if (FLAGS && any[u]) any[u] = *((const uint8_t*)scratch - 1 - (blocked_word(G, w, y, z) >> 6)) != 0;
@@ -607,10 +609,13 @@ __device__ __forceinline__ void unblock_ragged(uint32_t* __restrict__ scratch, u
         return;
     }
 #pragma unroll
-    for (int u = 0; u < 4; u++)
+    for (int u = 0; u < 4; u++) {
+        if (u >= passes) break;
         v[u] = any[u] ? scratch[blocked_word(G, (threadIdx.x >> 5) + 8u * (uint32_t)u, y, z)] : 0u;
+    }
 #pragma unroll
     for (int u = 0; u < 4; u++) {
+        if (u >= passes) break;
         const uint32_t w = (threadIdx.x >> 5) + 8u * (uint32_t)u;
         if (v[u]) scratch[blocked_word(G, w, y, z)] = 0u;
         if (w < rw) rows[(threadIdx.x & 31u) * stride + w] = v[u];
@@ -838,7 +843,10 @@ static uint32_t chunk_big(uint32_t G, uint64_t n) {
 // of their words.  A coarse mesh (about 2.5 voxels a triangle's edge and more)
 // queues smaller boxes and shares its few workgroups' queued rows with further
 // parts, the more the coarser it is.  A finer one of up to 262,144 triangles
-// takes two parts, for the large triangles that it may have among them.
+// takes two parts, for the large triangles that it may have among them.  Where
+// triangles are a voxel or less (16 G^2 and more) sharing them only repeats their
+// setup: 81,920 at 64^3 Morton 16.6 us a call with four lanes a triangle, 15.5
+// with two (14.4 with one, but a soup of as many 37 and 30).
 // Measured (us per call, 256 triangles a workgroup and one part -> this rule; a
 // loop of calls does not go below about 15): icosphere 5,120 at 64^3 21.7 ->
 // 15, 1,280 at 256^3 277 -> 18; torus 26,896 at 200^3 32.7 -> 17, 5,000 at
@@ -848,7 +856,8 @@ static uint32_t chunk_big(uint32_t G, uint64_t n) {
 static void chunk_shape(ItemDev& one) {
     const uint64_t n = one.info.n_triangles, G = one.info.gridsize[0];
     if (one.span > 1u || n == 0) return;
-    const uint32_t top = one.layout == VOX_LAYOUT_MORTON ? 3u : 4u;
+    const bool fine = n >= 16u * G * G;  // triangles of a voxel or less
+    const uint32_t top = fine ? 1u : (one.layout == VOX_LAYOUT_MORTON ? 3u : 4u);
     one.lg_split = 0;
     // (dense tables: fewer workgroups, each of which flushes the whole table)
     const uint64_t lanes = G * G * G / 32u <= (uint64_t)kHashCap ? 65536u : 327680u;
@@ -860,7 +869,7 @@ static void chunk_shape(ItemDev& one) {
         one.parts = p < 1u ? 1u : (p > 16u ? 16u : (uint32_t)p);
         if (!one.big) one.big = chunk_big((uint32_t)G, n);
     } else {
-        one.parts = one.lg_split <= 1u && n <= 262144u ? 2u : 1u;
+        one.parts = one.lg_split <= 1u && n <= 262144u && !fine ? 2u : 1u;
     }
 }
 

@@ -121,10 +121,13 @@ __device__ __forceinline__ void column_run(uint32_t* __restrict__ table, int64_t
 
 // Work unit: kMBlock >> it.lg_split consecutive triangles of one job, each
 // shared by 2^it.lg_split lanes, or with it.parts > 1 one part of their dealt
-// columns; the markers go to the job's table.  MULTI: the job comes from the launch's job map (block prefix);
-// otherwise it is `one`.  REG: the markers are staged as region pairs (RA)
-// instead (phase 1 of the region algorithm).
-template <bool MULTI, bool REG>
+// columns; the markers go to the job's table.  MULTI: the job comes from the
+// launch's job map (block prefix); otherwise it is `one`.  REG: the markers are
+// staged as region pairs (RA) instead (phase 1 of the region algorithm).  KEEP: a
+// triangle that is dealt is published from registers, as coarse meshes want it;
+// otherwise it is set up again, which leaves the others ten registers or more (six
+// spheres of 327,680 at 128^3 in a batch: 25 us in six waves per SIMD, 23 in eight).
+template <bool MULTI, bool REG, bool KEEP = false>
 __global__ void __launch_bounds__(kMBlock)
     solid_marker_kernel(ItemDev one, ItemMap M, MarkerWs ws, int spills, RegionArgs RA) {
     __shared__ ColRec recs[kColRecs];
@@ -212,7 +215,7 @@ __global__ void __launch_bounds__(kMBlock)
     if (__lane_id() == 0) nbig[threadIdx.x >> 6] = (uint32_t)__popcll(queued);
     __syncthreads();
     const auto setup = [&](SolidTri& Q, ColBox& C) {
-        if (MULTI) {  // again, from memory: held in registers they cost two waves per SIMD (25 us, 23)
+        if (!KEEP) {
             float v[3][3];
             load_tri(tris, mine, info, v);
             SolidTri T;
@@ -808,6 +811,13 @@ static uint32_t marker_units(const ItemDev& it) {
 hipError_t launch_marker_in_place(const vox_info& info, const float* tris, uint32_t* table,
                                   unsigned long long* offrow, const MarkerWs& ws, hipStream_t stream, uint32_t big);
 
+static void launch_markers(const ItemDev& one, const MarkerWs& ws, bool spills, hipStream_t stream) {
+    const ItemMap none{nullptr, nullptr, 1, 0};
+    const auto kernel = coarse_mesh(one.info.n_triangles, one.info.gridsize[0])
+                            ? solid_marker_kernel<false, false, true> : solid_marker_kernel<false, false, false>;
+    kernel<<<marker_units(one), kMBlock, 0, stream>>>(one, none, ws, spills ? 1 : 0, RegionArgs{});
+}
+
 static hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris, uint32_t* table,
                                                unsigned long long* offrow, hipStream_t stream, uint32_t big);
 
@@ -860,13 +870,17 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     // lines to zero.  Linear -> blocked (us per call): displaced sphere of 81,920
     // at 1024^3 120 -> 70, 1,310,720 at 1024^3 124.5 -> 116 (Morton 145 -> 137),
     // 20,480 at 512^3 31 -> 22 (Morton 34 -> 25), 327,680 at 2048^3 790 -> 475; at
-    // 768^3, whose rows of 24 words leave 16 lanes of a wave idle, 65 -> 70; fine
-    // meshes into Morton tables up to 512^3 gain nothing (33.9, 34.4).
+    // 768^3, whose rows of 24 words leave 16 lanes of a wave idle, 65 -> 70.  Fine
+    // meshes gain nothing into Morton tables up to 512^3 (33.9, 34.4), and lose into
+    // linear ones up to 256^3 (327,680 at 128^3 10.4 -> 11.3, 1,310,720 at 256^3 19.5
+    // either way, torus 18.4 -> 19.4), whose row pass then has few workgroups.
+    const bool coarse = coarse_mesh(info.n_triangles, G);
     const bool pow2 = (G & (G - 1u)) == 0 && G >= 128u;
-    one.flagged = pow2 && ((stream_rows && G <= 2048u) || (!linear && G <= 1024u && (G > 512u || coarse_mesh(info.n_triangles, G)))) ? 1u : 0u;
+    const bool blocked = pow2 && ((stream_rows && G <= 2048u && (G > 256u || coarse)) ||
+                                  (!linear && G <= 1024u && (G > 512u || coarse)));
+    one.flagged = blocked ? 1u : 0u;
     if (info.n_triangles)
-        solid_marker_kernel<false, false><<<marker_units(one), kMBlock, 0, stream>>>(one, none, ws, linear ? 1 : 0,
-                                                                                    RegionArgs{});
+        launch_markers(one, ws, linear, stream);
     if (ragged) {
         suffix_ragged_kernel<<<(G * G + 31u) / 32u, 256, 0, stream>>>(markers, table, G, accumulate ? 1 : 0);
     } else if (stream_rows && one.flagged) {
@@ -953,7 +967,7 @@ hipError_t launch_marker_in_place(const vox_info& info, const float* tris, uint3
     one.solid = 1;
     marker_shape(one, true);
     if (info.n_triangles)
-        solid_marker_kernel<false, false><<<marker_units(one), kMBlock, 0, stream>>>(one, none, ws, 1, RegionArgs{});
+        launch_markers(one, ws, true, stream);
     if (rows4_ok(G, table)) {
         const uint64_t nrows = (uint64_t)G * G;
         const uint64_t per = 64 / (G >> 7);
