@@ -249,13 +249,27 @@ static void reset_classes(vox_batch* b) {
     b->total_triangles = 0;
 }
 
+// Workgroups for which a job of large triangles shares them (0: not shared); see
+// chunk_batch_shape.
+static uint32_t shared_groups(const vox_batch_item* items, int count) {
+    uint64_t triangles = 0, jobs = 0;
+    for (int i = 0; i < count; i++) {
+        if (items[i].solid) continue;
+        triangles += items[i].info.n_triangles;
+        jobs += chunk_large(items[i].info.gridsize[0], items[i].info.n_triangles) ? 1u : 0u;
+    }
+    if (triangles > kSharedBatch || jobs == 0) return 0u;
+    const uint64_t groups = 1024u / jobs;
+    return groups > 512u ? 512u : (groups < 64u ? 64u : (uint32_t)groups);
+}
+
 static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* b, BatchPlan& plan,
                              uint64_t scratch_limit) {
     if (count < 0 || (count > 0 && !items)) return fail(VOX_ERR_INVALID, "bad item array");
     reset_classes(b);
     b->count = count;
-    uint64_t tri_sum_surf = 0, tri_sum_solid = 0, surface_triangles = 0;
-    for (int i = 0; i < count; i++) surface_triangles += items[i].solid ? 0u : items[i].info.n_triangles;
+    uint64_t tri_sum_surf = 0, tri_sum_solid = 0;
+    const uint32_t share = shared_groups(items, count);
     for (int i = 0; i < count; i++) {
         const vox_batch_item& it = items[i];
         vox_status s = validate(&it.info, it.d_tris, it.d_table, it.layout);
@@ -311,7 +325,7 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
             add_prefix(b->marker.base_c, b->marker.total_c, n);  // triangles (spill overflow pass)
         } else if (a == CHUNK) {
             d.span = chunk_span(G, n, false);
-            if (d.span <= 1u) chunk_batch_shape(d, surface_triangles <= kSharedBatch);
+            if (d.span <= 1u) chunk_batch_shape(d, share);
             // jobs that loop over chunks run in the 4-wave form (any layout): they stay in the 5-wave class;
             // a layout-specialised kernel runs at six waves per SIMD under either bound, so only
             // layout-generic jobs are split by the waves knob (each class is one more kernel)

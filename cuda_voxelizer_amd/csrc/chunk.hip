@@ -346,7 +346,10 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE || (SPEC != kSpecAny 
         __syncthreads();  // every slot is set before any lane inserts into the table; the counts are there
         if (part == 0 && live && !big) {
             surface_setup_tests(v, info, T);  // the box is T's already
-            lane_raster<REG, SPEC, SPLIT>(S, table, ident, T, info, layout, RA, sub, lg);  // nx <= 32 here
+            if (SPLIT && lg)  // nx <= 32 here
+                lane_raster<REG, SPEC, SPLIT>(S, table, ident, T, info, layout, RA, sub, lg);
+            else
+                lane_raster<REG, SPEC, false>(S, table, ident, T, info, layout, RA, 0, 0);
         }
         const auto setup = [&](uint32_t thread, SurfTri& Q) {
             float p[3][3];
@@ -832,7 +835,7 @@ static ItemDev single_job(const vox_info& info, const float* tris, uint32_t* tab
 // 512^3 66 and 80).
 static uint32_t chunk_big(uint32_t G, uint64_t n) {
     const uint64_t g2 = (uint64_t)G * G;
-    if (n == 0 || 8ull * n >= 5ull * g2) return 0u;
+    if (n == 0 || !chunk_large(G, n)) return 0u;
     return n <= 32768u ? 16u : (8u * n < g2 ? 64u : 0u);
 }
 
@@ -862,7 +865,7 @@ static void chunk_shape(ItemDev& one) {
     // (dense tables: fewer workgroups, each of which flushes the whole table)
     const uint64_t lanes = G * G * G / 32u <= (uint64_t)kHashCap ? 65536u : 327680u;
     while (one.lg_split < top && n << (one.lg_split + 1u) <= lanes) one.lg_split++;
-    if (8ull * n < 5ull * G * G) {
+    if (chunk_large((uint32_t)G, n)) {
         const uint64_t units = ((n << one.lg_split) + kChunk - 1) / kChunk;
         uint64_t p = 2048u / units;
         if (p > G * G / (2u * n)) p = G * G / (2u * n);
@@ -874,23 +877,23 @@ static void chunk_shape(ItemDev& one) {
 }
 
 // The work shape of a batch's job.  A mesh of large triangles is a long chain of
-// rounds to each of its few workgroups.  In a batch of few triangles (share) it is
-// shared as a lone call's is, up to 16 lanes a triangle and 16 parts, but by about
-// 512 workgroups only; in one of more, whose other jobs fill the device meanwhile,
-// a coarse one (fewer than G^2/4 triangles) has up to 32 parts, for 256 workgroups:
-// there the form of the kernel that shares triangles costs the others more than it
-// gains.  Measured (us a launch, parts only and shared): displaced sphere of 1,280
-// at 64^3 93 and 20, of 20,480 at 256^3 94 and 37, six of them 104 and 78; mixed
-// meshes, 13 of 0.9 million triangles 151 and 125, 24 of 1.7 million 152 and 149,
-// 48 of 3.5 million 443 and 459.
-void chunk_batch_shape(ItemDev& it, bool share) {
+// rounds to each of its few workgroups.  In a batch of few triangles they are shared
+// as in a lone call, up to 16 lanes a triangle and 16 parts, for `share` workgroups:
+// 1024 over all such jobs, 64 to 512 each.  In one of more, whose other jobs fill
+// the device meanwhile (share 0), a coarse mesh (fewer than G^2/4 triangles) has up
+// to 32 parts, for 256 workgroups.  Measured (us a launch, parts only and shared):
+// displaced sphere of 1,280 at 64^3 93 and 20, of 20,480 at 256^3 94 and 37, six of
+// them 104 and 78; mixed meshes, 13 of 0.3 million surface triangles 159 and 127,
+// 38 of 0.7 million 182 and 150, 26 of 1.2 million 291 and 286, 17 of 0.1 million
+// 118 and 121; 44 of 1.8 million 377 and 383.
+void chunk_batch_shape(ItemDev& it, uint32_t share) {
     const uint64_t n = it.info.n_triangles, G = it.info.gridsize[0];
     it.parts = 1;
     if (!it.big) it.big = chunk_big((uint32_t)G, n);
-    if (n == 0 || (share ? 8u * n >= 5u * G * G : !coarse_mesh(n, (uint32_t)G))) return;
-    while (share && it.lg_split < 4u && n << (it.lg_split + 1u) <= 131072u) it.lg_split++;
+    if (n == 0 || !(share ? chunk_large((uint32_t)G, n) : coarse_mesh(n, (uint32_t)G))) return;
+    while (share && it.lg_split < 4u && n << (it.lg_split + 1u) <= 256u * share) it.lg_split++;
     const uint64_t units = ((n << it.lg_split) + kChunk - 1) / kChunk;
-    uint64_t p = (share ? 512u : 256u) / units;
+    uint64_t p = (share ? share : 256u) / units;
     if (share && p > G * G / (2u * n)) p = G * G / (2u * n);
     const uint64_t most = share ? 16u : 32u;
     it.parts = p < 1u ? 1u : (p > most ? (uint32_t)most : (uint32_t)p);

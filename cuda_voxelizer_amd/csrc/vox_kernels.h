@@ -120,8 +120,10 @@ inline bool prefer_tile_solid(int layout, bool accumulate, uint64_t n_triangles,
 hipError_t launch_fill_zero(const vox_info& info, uint32_t* table, hipStream_t stream);
 uint32_t fill_units(uint32_t G);
 uint32_t chunk_span(uint32_t G, uint64_t n_triangles, bool lone);
-void chunk_batch_shape(ItemDev& it, bool share);
-constexpr uint64_t kSharedBatch = 1500000;  // triangles of a batch's surfaces
+void chunk_batch_shape(ItemDev& it, uint32_t share);
+constexpr uint64_t kSharedBatch = 1600000;  // triangles of a batch's surfaces
+// Triangles of about 2.5 voxels an edge and more.
+inline bool chunk_large(uint32_t G, uint64_t n_triangles) { return 8u * n_triangles < 5ull * G * G; }
 uint32_t chunk_units(uint64_t n_triangles, uint32_t span, uint32_t parts, uint32_t lg_split = 0);
 hipError_t launch_fill_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, hipStream_t stream);
 // What a chunk kernel instantiation knows of its jobs' layout: nothing, linear
