@@ -152,12 +152,12 @@ static hipError_t launch_all(vox_batch* b, hipStream_t s) {
 // order the critical path wants them dispatched: the fill, then the longer of
 // the two chunk chains on `m` (the classes that need the fill, or the blocked one
 // and its unblock pass, which does not), the other on a branch, and the tile
-// chain (no fill), the marker chain and the direct classes.  Of 13 mixed meshes
-// whose longest job was a soup of 269,272 at 32^3 the filled chain first took 203
-// us, the blocked one 228; of 48 mixed meshes 407 and 387.  `m` joins every branch
-// at the end.  Tables of
-// different jobs do not overlap, so the branches share no data (the out-of-row
-// counters they add to are atomic).
+// chain (no fill), the marker chain and the direct classes.  A launch of 13 mixed
+// meshes whose longest job is a soup of 269,272 at 32^3 takes 125 us with the
+// filled chain first, 157 with the blocked one; of 31 171 and 202; of 36 208 and
+// 191, of 48 442 and 423.  `m` joins every branch at the end.  Tables of different
+// jobs do not overlap, so the branches share no data (the out-of-row counters they
+// add to are atomic).
 static hipError_t launch_forked(vox_batch* b, hipStream_t m) {
     hipError_t e = hipSuccess;
     uint64_t filled = 0, blocked = 0;  // triangles of the two chunk chains
@@ -309,7 +309,8 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
         b->total_triangles += n;
         const uint64_t table_bytes = blocked_bytes(G);
         // 48 mixed meshes, linear keys -> blocked: 740 -> 405 us a launch
-        const bool blocked = a == CHUNK && !(it.flags & VOX_FLAG_NO_SCRATCH) && G <= kBatchBlockedGrid && chunk_blocked(it.layout, G, n) &&
+        const bool blocked = a == CHUNK && !(it.flags & VOX_FLAG_NO_SCRATCH) && G <= kBatchBlockedGrid &&
+                             chunk_blocked(it.layout, G, n) &&
                              plan.scratch + table_bytes <= scratch_limit;
         if (a != TILE && !accumulate && !blocked) {
             b->fill.items.push_back(d);

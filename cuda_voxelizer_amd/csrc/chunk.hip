@@ -246,7 +246,7 @@ __device__ __forceinline__ void lane_raster(ChunkShared& S, uint32_t* __restrict
 
 // Work unit: `span` consecutive chunks of kChunk triangles of one job, merged
 // in one LDS table and flushed once -- or one chunk of it.per triangles, each
-// shared by 2^it.lg_split lanes (SPLIT).  With `parts` > 1 the row windows of
+// shared by 2^it.lg_split lanes (SPLIT; a job of a batch may have none).  With `parts` > 1 the row windows of
 // a chunk's queued triangles are shared: the first units (part 0) take every
 // parts-th window and the lane rasters, further units one part's windows each.
 // MULTI: the job comes from the launch's job map; otherwise it is `one` (kernel
@@ -256,9 +256,9 @@ __device__ __forceinline__ void lane_raster(ChunkShared& S, uint32_t* __restrict
 // words are staged as region pairs (RA) instead of ORed into the table.
 // Workgroups per CU: the LDS allows six.  The bound holds the registers at
 // five waves per SIMD, or six with WIDE and in a single job's specialised form
-// (no spills there), or four for the chunk loop.  SPEC:
-// the layout when it is known at compile time, so the other layout's word
-// paths are compiled out (at six waves this removes the spills).
+// (no spills there), or four for the chunk loop.  SPEC: the layout when it is
+// known at compile time, so the other layout's word paths are compiled out (at
+// six waves this removes the spills).
 template <bool MULTI, bool LOOP, bool WIDE, bool REG, int SPEC = kSpecAny, bool SPLIT = false>
 __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE || (SPEC != kSpecAny && !MULTI) ? 6 : 5))
     surface_chunk_kernel(ItemDev one, ItemMap M, RegionArgs RA) {
@@ -694,20 +694,21 @@ hipError_t launch_unblock_jobs(const ItemDev& one, const ItemMap& M, uint32_t un
     return hipGetLastError();
 }
 
-// Where words go through a blocked scratch table: the linear layout, in tables beyond the dense LDS merge; a call of few triangles at G <= 80 has too
-// few atomics for it (displaced sphere of 1,280 at 64^3 12.3 us, 13.3 blocked; a
-// soup of 100,003 at 64^3 76.6 and 27.9).  Measured with the rows of a linear
-// table as keys -> blocked (us per call): soup of 300,003 at 128^3 160 -> 45,
-// 100,003 at 256^3 88 -> 67; displaced sphere of 81,920 at 256^3 31 -> 21, at
-// 512^3 65 -> 37, 327,680 at 512^3 92 -> 60; torus of 200,000 at 256^3 19 -> 14;
-// with flags: 81,920 at 1024^3 149 -> 86, at 2048^3 728 -> 300; torus of
-// 1,048,576 at 1024^3 105 -> 76.  The flags save the row pass most of the scratch
-// table from about 640^3 on; below, setting them costs more than that (327,680 at
-// 256^3 41 without, 46 with; at 544^3 66 and 71).  Grids whose rows are no whole
-// words: torus of 26,866 at 200^3 16.7 -> 14.2, soup of 100,000 at 201^3 89 -> 48,
-// displaced sphere of 81,920 at 200^3 32 -> 18, torus of 200,000 at 1000^3 105 ->
-// 99.  No mesh of 1,280 to 1,310,720 triangles measured slower than with the rows
-// of the table as keys at any grid of 200 to 2048.
+// Where words go through a blocked scratch table: the linear layout, in tables
+// beyond the dense LDS merge.  A call of few triangles at G <= 80 has too few
+// atomics for it (displaced sphere of 1,280 at 64^3 12.3 us, 13.3 blocked; a soup
+// of 100,003 at 64^3 76.6 and 27.9).  Measured with the rows of a linear table as
+// keys -> blocked (us per call): soup of 300,003 at 128^3 160 -> 45, 100,003 at
+// 256^3 88 -> 67; displaced sphere of 81,920 at 256^3 31 -> 21, at 512^3 65 -> 37,
+// 327,680 at 512^3 92 -> 60; torus of 200,000 at 256^3 19 -> 14; with flags, 81,920
+// at 1024^3 149 -> 86, at 2048^3 728 -> 300, torus of 1,048,576 at 1024^3 105 ->
+// 76.  The flags save the row pass most of the scratch table from about 640^3 on;
+// below, setting them costs more than that (327,680 at 256^3 41 without, 46 with;
+// at 544^3 66 and 71).  Grids whose rows are no whole words: torus of 26,866 at
+// 200^3 16.7 -> 14.2, soup of 100,000 at 201^3 89 -> 48, displaced sphere of 81,920
+// at 200^3 32 -> 18, torus of 200,000 at 1000^3 105 -> 99.  No mesh of 1,280 to
+// 1,310,720 triangles measured slower than with the rows of the table as keys at
+// any grid of 200 to 2048.
 bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles) {
     const uint64_t words = (uint64_t)G * G * G / 32u;
     return layout == VOX_LAYOUT_LINEAR && G <= ((G & 31u) ? kRaggedGrid : kBlockedGrid) &&
@@ -726,9 +727,9 @@ uint32_t fill_units(uint32_t G) {
 // the same few addresses (16 of them a request): such jobs give each workgroup
 // several chunks to cut those atomics, while keeping at least 512 workgroups of a
 // lone call, or 128 of a batch's job.  With 64 a workgroup's chain of chunks was
-// what the call lasted (us per call, 64 -> this): soup of 269,272 at 32^3 141 ->
-// 28, torus of 100,000 at 32^3 30 -> 15; 13 mixed meshes in a batch 203 -> 157 (161
-// with 512).
+// what the call lasted (us per call, 64 -> this): soup of 269,272 at 32^3 137 ->
+// 28, torus of 100,000 at 32^3 29 -> 11; batches of 13 mixed meshes 190 -> 125
+// (116 with 512), of 11 195 -> 163 (181 with 512), of 48 423 with any.
 uint32_t chunk_span(uint32_t G, uint64_t n_triangles, bool lone) {
     const uint64_t words = ((uint64_t)G * G * G + 31) / 32;
     if (words > (uint64_t)kHashCap) return 1u;

@@ -6,18 +6,20 @@
 // of its column with xmax >= x, so it is enough to toggle ONE marker bit at
 // (xmax, y, z) per run and then replace every row by its suffix XOR along x:
 //
-//   1. fill      zero the marker table: the output table itself (linear
-//                layout, no accumulate) or a linear scratch table
+//   1. fill      the marker table is the stream's scratch table, which every
+//                call leaves zero, with its words in rows or, on power-of-two
+//                grids from 128, blocked (4 x 4 rows of a word together); or
+//                the output table itself (linear, no accumulate), zeroed
 //   2. markers   per triangle (one lane each; triangles with many columns
 //                have them dealt over the workgroup, columns.h): solid setup,
 //                column tests, xmax, one non-returning atomicXor per hit column
 //   3. suffix    per row (G/32 words, lanes = words): in-word prefix XOR from
 //                bit 0 up (larger x = lower bit) plus the parity of the words
-//                of larger x (a ballot).  In place for the linear layout;
-//                from the scratch table, one workgroup per block of 32 x rz
-//                rows staged in LDS, for the Morton layout (4x4x2 brick words
-//                assembled from 8 rows at a time) and for accumulation
-//                (XOR into the caller's table)
+//                of larger x (a ballot).  Linear: from the scratch table into
+//                the output, or in place; Morton (4x4x2 brick words assembled
+//                from 8 rows at a time) and accumulation (XOR into the
+//                caller's table): from the scratch table, one workgroup per
+//                block of 32 x rz rows staged in LDS
 //   4. spills    runs with xmax >= G continue along the linear index into the
 //                following rows (as the reference indexes them): their
 //                in-row part is a marker at G-1, the rest is recorded and

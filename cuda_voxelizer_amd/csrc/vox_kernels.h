@@ -148,9 +148,9 @@ inline uint64_t blocked_flags(uint32_t G) { return (blocked_bytes(G) / 256u + 25
 // Grids whose rows are no whole words are packed from padded rows up to this one.
 constexpr uint32_t kRaggedGrid = 1024;
 constexpr uint32_t kRaggedWords = 32u * (kRaggedGrid / 32u + 1u);
-// 32 rows of rw words in LDS, `stride` words apart, from row r0 on -> their words of the linear table
-// (fewer at its end; bits from G on are zero in every row): put(word, value) for
-// each.  A word has bits of at most two rows (G > 32).
+// 32 rows of rw words in LDS, `stride` words apart, from row r0 on -> their words of
+// the linear table (fewer at its end; bits from G on are zero in every row):
+// put(word, value) for each.  A word has bits of at most two rows (G > 32).
 template <class Put>
 __device__ __forceinline__ void pack_rows(const uint32_t* rows, uint32_t stride, uint32_t rw, uint32_t G, uint32_t r0,
                                           uint32_t* __restrict__ table, Put&& put) {
@@ -167,9 +167,9 @@ __device__ __forceinline__ void pack_rows(const uint32_t* rows, uint32_t stride,
 }
 constexpr int kBlockedSpecs = kSpecBlocked + 1;  // what a batch's classes may be
 constexpr uint32_t kBlockedGrid = 2048;
-constexpr uint32_t kUnflaggedGrid = 608;
+constexpr uint32_t kUnflaggedGrid = 608;  // (chunk.hip: chunk_blocked)
 constexpr uint32_t kBatchBlockedGrid = 512;
-constexpr uint32_t kStreamedGrid = 1152;
+constexpr uint32_t kStreamedGrid = 1152;  // (chunk.hip: unblock_flagged_kernel)
 bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles);
 uint32_t unblock_units(uint32_t G, const uint32_t* table);
 hipError_t launch_unblock_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, hipStream_t stream);
