@@ -310,7 +310,7 @@ static vox_status plan_batch(const vox_batch_item* items, int count, vox_batch* 
         const uint64_t table_bytes = blocked_bytes(G);
         // 48 mixed meshes, linear keys -> blocked: 740 -> 405 us a launch
         const bool blocked = a == CHUNK && !(it.flags & VOX_FLAG_NO_SCRATCH) && G <= kBatchBlockedGrid &&
-                             chunk_blocked(it.layout, G, n) &&
+                             chunk_blocked(it.layout, G, n, accumulate) &&
                              plan.scratch + table_bytes <= scratch_limit;
         if (a != TILE && !accumulate && !blocked) {
             b->fill.items.push_back(d);

@@ -346,7 +346,7 @@ __global__ void __launch_bounds__(kChunk, LOOP ? 4 : (WIDE || (SPEC != kSpecAny 
         __syncthreads();  // every slot is set before any lane inserts into the table; the counts are there
         if (part == 0 && live && !big) {
             surface_setup_tests(v, info, T);  // the box is T's already
-            if (SPLIT && lg)  // nx <= 32 here
+            if (SPLIT && (!MULTI || lg))  // nx <= 32 here
                 lane_raster<REG, SPEC, SPLIT>(S, table, ident, T, info, layout, RA, sub, lg);
             else
                 lane_raster<REG, SPEC, false>(S, table, ident, T, info, layout, RA, 0, 0);
@@ -410,7 +410,8 @@ __global__ void __launch_bounds__(256) fill_zero_kernel(ItemDev one, ItemMap M) 
     }
 }
 
-__device__ __forceinline__ void table_or(uint32_t* p, uint32_t v) {
+template <class Word>
+__device__ __forceinline__ void table_or(Word* p, Word v) {
     if (v) atomicOr(p, v);
 }
 
@@ -447,11 +448,9 @@ __device__ __forceinline__ void unblock_quad(const ItemDev& it, uint32_t t, bool
             if (!it.accumulate) {
                 d4[d] = o[u];
             } else {
-                uint32_t* p = (uint32_t*)(d4 + d);
-                table_or(p, o[u].x);
-                table_or(p + 1, o[u].y);
-                table_or(p + 2, o[u].z);
-                table_or(p + 3, o[u].w);
+                unsigned long long* p = (unsigned long long*)(d4 + d);
+                table_or(p, (unsigned long long)o[u].y << 32 | o[u].x);
+                table_or(p + 1, (unsigned long long)o[u].w << 32 | o[u].z);
             }
         }
         return;
@@ -709,8 +708,15 @@ hipError_t launch_unblock_jobs(const ItemDev& one, const ItemMap& M, uint32_t un
 // at 200^3 32 -> 18, torus of 200,000 at 1000^3 105 -> 99.  No mesh of 1,280 to
 // 1,310,720 triangles measured slower than with the rows of the table as keys at
 // any grid of 200 to 2048.
-bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles) {
+//
+// An accumulating call has no zero-fill to save, and its row pass adds to the table
+// by atomics itself: few triangles go to the table directly (us, blocked and
+// direct: 1,280 at 256^3 17.6 and 13.3, at 1024^3 97 and 82; soup of 3,000 at 128^3
+// 16.0 and 12.7; displaced sphere of 20,480 at 128^3 15.9 and 12.7, at 200^3 18.2 and
+// 21.6, of 81,920 at 128^3 16.2 and 20.0, at 512^3 46 and 60, at 1024^3 123 and 128).
+bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles, bool accumulate) {
     const uint64_t words = (uint64_t)G * G * G / 32u;
+    if (accumulate && n_triangles <= (G <= 160u ? 32768u : 4096u)) return false;
     return layout == VOX_LAYOUT_LINEAR && G <= ((G & 31u) ? kRaggedGrid : kBlockedGrid) &&
            words > (n_triangles < 16384u ? 16384u : (uint64_t)kHashCap);
 }
@@ -932,7 +938,7 @@ hipError_t launch_surface_chunk(const vox_info& info, const float* tris, uint32_
     one.accumulate = accumulate ? 1 : 0;
     chunk_shape(one);
     const uint32_t G = info.gridsize[0];
-    if (scratch && info.n_triangles && chunk_blocked(layout, G, info.n_triangles)) {
+    if (scratch && info.n_triangles && chunk_blocked(layout, G, info.n_triangles, accumulate)) {
         hipError_t e = hipSuccess;
         const uint64_t bytes = blocked_bytes(G);
         one.flagged = G > kUnflaggedGrid ? 1u : 0u;

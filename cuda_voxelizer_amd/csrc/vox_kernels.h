@@ -170,7 +170,7 @@ constexpr uint32_t kBlockedGrid = 2048;
 constexpr uint32_t kUnflaggedGrid = 608;  // (chunk.hip: chunk_blocked)
 constexpr uint32_t kBatchBlockedGrid = 512;
 constexpr uint32_t kStreamedGrid = 1152;  // (chunk.hip: unblock_flagged_kernel)
-bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles);
+bool chunk_blocked(int layout, uint32_t G, uint64_t n_triangles, bool accumulate);
 uint32_t unblock_units(uint32_t G, const uint32_t* table);
 hipError_t launch_unblock_jobs(const ItemDev& one, const ItemMap& M, uint32_t units, hipStream_t stream);
 // Tuning bits of the flags (VOX_TUNE_*): queue threshold, chunk waves per SIMD, tile size.

@@ -17,7 +17,7 @@ def test_launches_on_several_streams(oracle, gpu, use_graph, threads):
     from cuda_voxelizer_amd import meshgen
     jobs, exp = [], []
     # (triangles, grid, solid, accumulate, algorithm)
-    for k, (n, grid, solid, acc, algo) in enumerate([(9000, 256, False, False, "auto"), (3000, 128, False, True, "auto"),
+    for k, (n, grid, solid, acc, algo) in enumerate([(9000, 256, False, False, "auto"), (33000, 128, False, True, "auto"),
                                                      (2000, 100, False, False, "auto"), (3000, 128, True, False, "auto"),
                                                      (3000, 128, True, False, "tile"), (3000, 128, False, False, "tile")]):
         tris = np.ascontiguousarray(meshgen.triangle_soup(n, seed=60 + k, mu=-2.5, sigma=0.6), np.float32)
