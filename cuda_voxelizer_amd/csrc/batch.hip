@@ -519,8 +519,7 @@ vox_status vox_batch_launch(vox_batch* b, void* stream) {
         if (b->done) {
             e = hipStreamWaitEvent(st, b->done, 0);
         } else {
-            const RelaxedCapture relaxed;
-            e = hipDeviceSynchronize();
+            e = wait_for_device();
             if (e == hipSuccess) e = hipEventCreateWithFlags(&b->done, hipEventDisableTiming);
         }
     }
@@ -531,7 +530,7 @@ vox_status vox_batch_launch(vox_batch* b, void* stream) {
         b->scratch_dirty = b->sws && e != hipSuccess;
         b->last = key;
         b->launched = true;
-        if (b->done && hipEventRecord(b->done, st) != hipSuccess) (void)hipDeviceSynchronize();
+        if (b->done && hipEventRecord(b->done, st) != hipSuccess) (void)wait_for_device();
     }
     if (e != hipSuccess) return hip_fail(e, "batch launch");
     return VOX_OK;

@@ -32,9 +32,8 @@ struct StreamKey {
 };
 hipError_t stream_key(hipStream_t stream, StreamKey& key);  // on the current device
 
-// Memory is allocated and freed, and the device waited for, in the relaxed capture
-// mode: no stream that is being captured is touched, and the default mode refuses
-// it while any thread captures one.
+// Memory is allocated and freed in the relaxed capture mode: no stream that is being
+// captured is touched, and the default mode refuses it while any thread captures one.
 struct RelaxedCapture {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     const bool set;
@@ -43,6 +42,10 @@ struct RelaxedCapture {
         if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
     }
 };
+
+// Waits for all work of the device that has been queued, as hipFree does; unlike
+// hipDeviceSynchronize it leaves other threads' captures valid.
+hipError_t wait_for_device();
 
 struct StreamScratch;
 

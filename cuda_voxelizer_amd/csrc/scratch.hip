@@ -68,24 +68,25 @@ hipError_t stream_key(hipStream_t stream, StreamKey& key) {
     return hipGetDevice(&key.device);
 }
 
-// Frees what an idle stream of the current device has, whose last call may still
-// run.  False if the device cannot be waited for.
-static bool give_back(StreamScratch& s) {
-    if (!s.table && (!s.spills || s.recorded)) return true;
-    if (hipDeviceSynchronize() != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
+hipError_t wait_for_device() {
+    const RelaxedCapture relaxed;
+    void* p = nullptr;
+    const hipError_t e = hipMalloc(&p, 256);
+    return e == hipSuccess ? hipFree(p) : e;
+}
+
+// Frees what an idle stream of the current device has; its last call may still run,
+// and hipFree waits for the device.
+static void give_back(StreamScratch& s) {
     if (s.table) (void)hipFree(s.table);
     s.dev->held -= s.bytes;
     s.table = nullptr;
     s.bytes = 0;
+    s.dirty = true;
     if (s.spills && !s.recorded) {
         (void)hipFree(s.spills);
         s.spills = nullptr;
     }
-    s.dirty = true;
-    return true;
 }
 
 // Counts `bytes` instead of s.bytes among the device's tables, if they fit.
@@ -99,10 +100,12 @@ static bool reserve(int device, StreamScratch& s, uint64_t bytes) {
         bool left = false;
         for (auto it = P.streams.begin(); it != P.streams.end();) {
             const bool own = it->first.thread == n;
-            if (own && it->first.device == device && it->second.holders == 0 && give_back(it->second) &&
-                !it->second.spills) {
-                it = P.streams.erase(it);
-                continue;
+            if (own && it->first.device == device && it->second.holders == 0) {
+                give_back(it->second);
+                if (!it->second.spills) {
+                    it = P.streams.erase(it);
+                    continue;
+                }
             }
             left = left || own;
             ++it;
@@ -117,7 +120,8 @@ static bool reserve(int device, StreamScratch& s, uint64_t bytes) {
                 now - it->second.last >= kIdle &&
                 (idle == P.streams.end() || it->second.last < idle->second.last))
                 idle = it;
-        if (idle == P.streams.end() || !give_back(idle->second)) return false;
+        if (idle == P.streams.end()) return false;
+        give_back(idle->second);
         if (!idle->second.spills) P.streams.erase(idle);
     }
     s.dev->held += bytes - s.bytes;
@@ -226,17 +230,15 @@ extern "C" vox_status vox_release_scratch(void) {
     const RelaxedCapture relaxed;
     ScratchPool& P = pool();
     std::lock_guard<std::mutex> lock(P.m);
-    bool all = true;
     for (auto it = P.streams.begin(); it != P.streams.end();) {
         if (it->first.device == device && it->second.holders == 0) {
-            if (!give_back(it->second)) {
-                all = false;
-            } else if (!it->second.spills) {
+            give_back(it->second);
+            if (!it->second.spills) {
                 it = P.streams.erase(it);
                 continue;
             }
         }
         ++it;
     }
-    return all ? VOX_OK : fail(VOX_ERR_HIP, "vox_release_scratch: the device could not be waited for");
+    return VOX_OK;
 }

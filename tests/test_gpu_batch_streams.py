@@ -46,3 +46,44 @@ def test_launches_on_several_streams(oracle, gpu, use_graph, threads):
         for k, (j, e) in enumerate(zip(jobs, exp)):
             assert (j.table.cpu().numpy().view(np.uint32) == e).all(), k
     batch.close()
+
+
+@pytest.mark.parametrize("other_thread", [False, True])
+def test_beside_a_capture(oracle, gpu, other_thread):
+    """Waits and frees of the library leave a capture under way valid."""
+    import cuda_voxelizer_amd as V
+    import torch
+    from cuda_voxelizer_amd import meshgen
+    tris = np.ascontiguousarray(meshgen.triangle_soup(3000, seed=9, mu=-2.5, sigma=0.6), np.float32)
+    info = V.voxinfo_for_mesh(tris.reshape(-1, 3), 128, len(tris))
+    oinfo = oracle.info_from_bytes(info.as_bytes())
+    surface, solid = (f(oinfo, tris, morton=False)[0] for f in (oracle.surface, oracle.solid))
+    d = torch.from_numpy(tris.reshape(-1)).to(gpu)
+    tables = [torch.zeros(surface.size, dtype=torch.int32, device=gpu) for _ in range(4)]
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    batch = V.Batch([V.BatchJob(info, d, tables[0]), V.BatchJob(info, d, tables[1], solid=True)])
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+
+    def beside():
+        for k in range(4):
+            batch.launch(stream=streams[k % 2])
+        V.release_scratch()
+
+    with torch.cuda.graph(graph, stream=streams[2]):
+        V.voxelize_surface(info, d, table=tables[2])
+        if other_thread:
+            t = threading.Thread(target=beside)
+            t.start()
+            t.join()
+        else:
+            beside()
+        V.voxelize_solid_table(info, d, table=tables[3])
+    for _ in range(3):
+        for k in (2, 3):
+            tables[k].fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        for table, exp in zip(tables, (surface, solid, surface, solid)):
+            assert (table.cpu().numpy().view(np.uint32) == exp).all()
+    batch.close()
