@@ -37,7 +37,6 @@
 #include "vox_host.h"
 #include "vox_kernels.h"
 
-#include <map>
 #include <mutex>
 
 #pragma clang fp contract(off)
@@ -820,8 +819,17 @@ static void launch_markers(const ItemDev& one, const MarkerWs& ws, bool spills, 
     kernel<<<marker_units(one), kMBlock, 0, stream>>>(one, none, ws, spills ? 1 : 0, RegionArgs{});
 }
 
-static hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris, uint32_t* table,
-                                               unsigned long long* offrow, hipStream_t stream, uint32_t big);
+// Zero the counter words (a kernel, so the sequence has no memset node when a
+// caller captures it into a graph).
+__global__ void __launch_bounds__(64) clear_counters_kernel(unsigned* misc, int words) {
+    for (int i = threadIdx.x; i < words; i += 64) misc[i] = 0u;
+}
+
+// Zero a graph's own table.
+__global__ void __launch_bounds__(256) clear_table_kernel(uint4* __restrict__ t, uint64_t quads) {
+    for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < quads; i += (uint64_t)gridDim.x * 256u)
+        t[i] = make_uint4(0u, 0u, 0u, 0u);
+}
 
 static hipError_t marker_ws(ScratchLease& S, MarkerWs& ws) {
     void* p = nullptr;
@@ -841,19 +849,40 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     const bool stream_rows = layout == VOX_LAYOUT_LINEAR && !accumulate && rows4_ok(G, table);
     const bool ragged = (G & 31u) != 0;
     const bool in_place = layout == VOX_LAYOUT_LINEAR && !accumulate && !stream_rows && !ragged;
-    const uint64_t table_bytes = (uint64_t)G * G * ((G + 31u) / 32u) * 4u;  // rows padded to words
+    // rows padded to words, and the table to 16-byte groups
+    const uint64_t table_bytes = ((uint64_t)G * G * ((G + 31u) / 32u) * 4u + 15u) & ~15ull;
     ScratchLease S(stream);
-    if (S.recording())
-        return marker_batch_supported(G, layout, accumulate)
-                   ? launch_solid_marker_captured(info, tris, table, offrow, stream, big)
-                   : hipErrorOutOfMemory;
     MarkerWs ws;
-    hipError_t e = marker_ws(S, ws);
-    if (e != hipSuccess) return e;
-    uint32_t* markers = in_place ? table : (scratch ? S.table(table_bytes) : nullptr);
-    if (!markers && !stream_rows) return hipErrorOutOfMemory;
-    // the in-place form needs no scratch table
-    if (in_place || !markers) return launch_marker_in_place(info, tris, table, offrow, ws, stream, big);
+    uint32_t* markers = nullptr;
+    hipError_t e;
+    if (S.recording()) {
+        // A graph holds memory of its own, which a kernel of the graph clears, so that
+        // graphs replay beside each other and beside the stream's calls.  In place
+        // wherever that is possible: the 1 MB of run records is all it needs then.
+        const bool own = !marker_batch_supported(G, layout, accumulate);
+        void* p = nullptr;
+        if (own && !scratch) return hipErrorOutOfMemory;
+        e = graph_memory(stream, marker_ws_bytes() + (own ? table_bytes : 0u), &p);
+        if (e != hipSuccess) return hipErrorOutOfMemory;
+        ws = MarkerWs{(unsigned*)p, (unsigned long long*)((char*)p + 256)};
+        if (own) markers = (uint32_t*)((char*)p + marker_ws_bytes());
+        clear_counters_kernel<<<1, 64, 0, stream>>>(ws.misc, 64);
+        if (own) {
+            const uint64_t quads = (table_bytes + 15u) / 16u;
+            const uint64_t blocks = (quads + 1023u) / 1024u;
+            clear_table_kernel<<<(unsigned)(blocks < 65536u ? blocks : 65536u), 256, 0, stream>>>((uint4*)markers, quads);
+        }
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        if (!own) return launch_marker_in_place(info, tris, table, offrow, ws, stream, big);
+    } else {
+        e = marker_ws(S, ws);
+        if (e != hipSuccess) return e;
+        if (scratch && !in_place) markers = S.table(table_bytes);
+        if (!markers && !in_place && !stream_rows) return hipErrorOutOfMemory;
+        // the in-place form needs no scratch table
+        if (!markers) return launch_marker_in_place(info, tris, table, offrow, ws, stream, big);
+    }
     const bool linear = layout == VOX_LAYOUT_LINEAR;
     const ItemMap none{nullptr, nullptr, 1, 0};
     ItemDev one{};  // markers: into the scratch table
@@ -881,8 +910,7 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     const bool blocked = pow2 && ((stream_rows && G <= 2048u && (G > 256u || coarse)) ||
                                   (!linear && G <= 1024u && (G > 512u || coarse)));
     one.flagged = blocked ? 1u : 0u;
-    if (info.n_triangles)
-        launch_markers(one, ws, linear, stream);
+    if (info.n_triangles) launch_markers(one, ws, linear, stream);
     if (ragged) {
         suffix_ragged_kernel<<<(G * G + 31u) / 32u, 256, 0, stream>>>(markers, table, G, accumulate ? 1 : 0);
     } else if (stream_rows && one.flagged) {
@@ -907,7 +935,7 @@ hipError_t launch_solid_marker(const vox_info& info, const float* tris, uint32_t
     }
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    S.clean();  // every row of the scratch table was read and cleared
+    if (!S.recording()) S.clean();  // every row of the scratch table was read and cleared
     if (linear) spill_kernel<<<kSpillBlocks, 256, 0, stream>>>(fin, none, none, ws);
     return hipGetLastError();
 }
@@ -1003,48 +1031,7 @@ constexpr int kMaxStaticDevices = 64;
 static std::mutex g_static_mutex;
 static void* g_static_ptr[kMaxStaticDevices];  // device address of `scratch`, per device
 
-// Zero the counter words (a kernel, so the sequence has no memset node when a
-// caller captures it into a graph).
-__global__ void __launch_bounds__(64) clear_counters_kernel(unsigned* misc, int words) {
-    for (int i = threadIdx.x; i < words; i += 64) misc[i] = 0u;
-}
-
 size_t static_scratch_bytes() { return kStaticScratchBytes; }
-
-// ---- captured calls ------------------------------------------------------------
-// A call that is recorded into a graph takes the in-place form, whose only
-// workspace is the spill counters and records.  The graph holds their address, so
-// they are not those of the stream's eager calls and are never replaced or freed:
-// one allocation of 1 MB for each stream that captures.  The counters are cleared
-// by a kernel of the graph, as eager calls and replays may have ended anywhere.
-static std::mutex g_capture_mutex;
-static std::map<StreamKey, void*> g_capture_ws;
-
-static hipError_t launch_solid_marker_captured(const vox_info& info, const float* tris, uint32_t* table,
-                                               unsigned long long* offrow, hipStream_t stream, uint32_t big) {
-    StreamKey key;
-    hipError_t e = stream_key(stream, key);
-    if (e != hipSuccess) return e;
-    void* p = nullptr;
-    {
-        std::lock_guard<std::mutex> lock(g_capture_mutex);
-        void*& w = g_capture_ws[key];
-        if (!w) {
-            const RelaxedCapture relaxed;
-            e = hipMalloc(&w, kStaticScratchBytes);
-            if (e != hipSuccess) {
-                w = nullptr;
-                return e;
-            }
-        }
-        p = w;
-    }
-    const MarkerWs ws{(unsigned*)p, (unsigned long long*)((char*)p + 256)};
-    clear_counters_kernel<<<1, 64, 0, stream>>>(ws.misc, 64);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return launch_marker_in_place(info, tris, table, offrow, ws, stream, big);
-}
 
 hipError_t static_scratch_init(int device, void** out) {
     if (device < 0 || device >= kMaxStaticDevices) return hipErrorInvalidDevice;

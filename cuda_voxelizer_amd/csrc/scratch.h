@@ -7,8 +7,9 @@
 // before its first launch until its last is queued; a second thread's call on the
 // stream waits for that, and the stream's order does the rest.  (A new stream may
 // have the handle of one that was destroyed; hipStreamDestroy waits for a stream's
-// work.)  Calls on the
-// stream's other workspaces (tile, slab, region, triangle order) hold it too.
+// work.)  Calls on the stream's other workspaces (tile, slab, region, triangle
+// order) hold it too.  A call that is recorded into a graph uses none of it but
+// memory of the graph's (graph_memory), the region algorithm's records apart.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -46,6 +47,11 @@ struct RelaxedCapture {
 // Waits for all work of the device that has been queued, as hipFree does; unlike
 // hipDeviceSynchronize it leaves other threads' captures valid.
 hipError_t wait_for_device();
+
+// Device memory for the graph into which calls on `stream` are being recorded, its
+// own until it and all that was cloned or instantiated from it are gone.  The contents
+// are undefined.  An error where the device's limit does not allow it.
+hipError_t graph_memory(hipStream_t stream, uint64_t bytes, void** out);
 
 struct StreamScratch;
 

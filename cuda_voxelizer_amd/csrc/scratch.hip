@@ -1,9 +1,11 @@
 // scratch.hip -- the scratch memory that calls on one stream share (scratch.h).
 #include "scratch.h"
 
+#include <algorithm>
 #include <atomic>
 #include <map>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 #include "vox_host.h"
@@ -13,6 +15,7 @@ namespace voxamd {
 
 struct DeviceScratch {
     uint64_t held = 0, leases = 0;  // bytes in tables, leases so far
+    uint64_t graphs = 0;            // bytes that graphs have, or had
 };
 
 struct StreamScratch {
@@ -27,18 +30,29 @@ struct StreamScratch {
     std::mutex use;
 };
 
+struct GraphMemory {
+    void* ptr;
+    uint64_t bytes;
+    int device;
+};
+
 // All streams' scratch.  A device's tables together stay below an eighth of its
 // memory (36 GB here: 36 streams at 2048^3), or are one stream's table: a call that
 // would go beyond has none, unless a stream of the device that has not had a call
 // for kIdle of the device's leases can give up its table -- a stream that was
 // destroyed, above all.  What a thread's own stream had (hipStreamPerThread) goes
-// once the thread has ended and another table grows.
+// once the thread has ended and another table grows.  What a graph had is kept for
+// the next one, and freed by vox_release_scratch only: an executable that was updated
+// from a graph does not hold what that graph had.  All graphs of a device have an
+// eighth of its memory at most.
 constexpr uint64_t kIdle = 64;
 struct ScratchPool {
     std::mutex m;
     std::map<StreamKey, StreamScratch> streams;
     std::map<int, DeviceScratch> devices;
     std::vector<uint64_t> ended;           // threads
+    std::mutex mr;                       // of returned; never held around a call of the runtime
+    std::vector<GraphMemory*> returned;  // of graphs that are gone
 };
 static ScratchPool& pool() {
     static ScratchPool* p = new ScratchPool;  // threads may end after static objects have gone
@@ -87,6 +101,78 @@ static void give_back(StreamScratch& s) {
         (void)hipFree(s.spills);
         s.spills = nullptr;
     }
+}
+
+// The runtime lets a graph's memory go: on any thread, where it must not be called.
+static void graph_gone(void* memory) {
+    ScratchPool& P = pool();
+    std::lock_guard<std::mutex> lock(P.mr);
+    P.returned.push_back((GraphMemory*)memory);
+}
+
+// Memory of at least `bytes` bytes, not above twice that, whose graph is gone; null if there is none.
+static GraphMemory* take_returned(int device, uint64_t bytes) {
+    ScratchPool& P = pool();
+    std::lock_guard<std::mutex> lock(P.mr);
+    auto best = P.returned.end();
+    for (auto it = P.returned.begin(); it != P.returned.end(); ++it)
+        if ((*it)->device == device && (*it)->bytes >= bytes && (*it)->bytes / 2 <= bytes &&
+            (best == P.returned.end() || (*it)->bytes < (*best)->bytes))
+            best = it;
+    if (best == P.returned.end()) return nullptr;
+    GraphMemory* g = *best;
+    P.returned.erase(best);
+    return g;
+}
+
+static hipError_t new_graph_memory(int device, uint64_t bytes, GraphMemory** out) {
+    size_t total = 0;
+    hipError_t e = hipDeviceTotalMem(&total, device);
+    if (e != hipSuccess) return e;
+    ScratchPool& P = pool();
+    {
+        std::lock_guard<std::mutex> lock(P.m);
+        uint64_t& held = P.devices[device].graphs;
+        if (held + bytes > total / 8) return hipErrorOutOfMemory;
+        held += bytes;
+    }
+    void* p = nullptr;
+    e = hipMalloc(&p, bytes);
+    if (e != hipSuccess) {
+        std::lock_guard<std::mutex> lock(P.m);
+        P.devices[device].graphs -= bytes;
+        return e;
+    }
+    *out = new GraphMemory{p, bytes, device};
+    return hipSuccess;
+}
+
+hipError_t graph_memory(hipStream_t stream, uint64_t bytes, void** out) {
+    int device = 0;
+    hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return e;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    hipGraph_t graph = nullptr;
+    const hipGraphNode_t* deps = nullptr;
+    size_t ndeps = 0;
+    e = hipStreamGetCaptureInfo_v2(stream, &status, &id, &graph, &deps, &ndeps);
+    if (e != hipSuccess) return e;
+    if (status != hipStreamCaptureStatusActive || !graph) return hipErrorIllegalState;
+    const RelaxedCapture relaxed;
+    GraphMemory* g = take_returned(device, bytes);
+    // a graph that is gone may still run
+    e = g ? wait_for_device() : new_graph_memory(device, bytes, &g);
+    hipUserObject_t owner = nullptr;
+    if (e == hipSuccess) e = hipUserObjectCreate(&owner, g, graph_gone, 1, hipUserObjectNoDestructorSync);
+    if (e != hipSuccess) {
+        if (g) graph_gone(g);
+        return e;
+    }
+    *out = g->ptr;
+    e = hipGraphRetainUserObject(graph, owner, 1, hipGraphUserObjectMove);
+    if (e != hipSuccess) (void)hipUserObjectRelease(owner, 1);
+    return e;
 }
 
 // Counts `bytes` instead of s.bytes among the device's tables, if they fit.
@@ -229,7 +315,19 @@ extern "C" vox_status vox_release_scratch(void) {
     if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
     const RelaxedCapture relaxed;
     ScratchPool& P = pool();
+    std::vector<GraphMemory*> gone;
+    {
+        std::lock_guard<std::mutex> lock(P.mr);
+        for (GraphMemory*& g : P.returned)
+            if (g->device == device) gone.push_back(std::exchange(g, nullptr));
+        P.returned.erase(std::remove(P.returned.begin(), P.returned.end(), nullptr), P.returned.end());
+    }
     std::lock_guard<std::mutex> lock(P.m);
+    for (GraphMemory* g : gone) {
+        (void)hipFree(g->ptr);
+        P.devices[device].graphs -= g->bytes;
+        delete g;
+    }
     for (auto it = P.streams.begin(); it != P.streams.end();) {
         if (it->first.device == device && it->second.holders == 0) {
             give_back(it->second);

@@ -71,11 +71,17 @@ typedef enum vox_status {
    for linear surfaces up to 2048^3 and for solids: of a device's streams
    together at most an eighth of its memory (or one stream's table), until
    vox_release_scratch; a linear surface call whose
-   stream is being captured, or that cannot have one, works in the caller's
-   table.  A captured marker call holds none either: linear, non-accumulating
-   ones on G % 32 == 0 work in the caller's table (the graph holds 1 MB of
-   counters and records that belong to the capture stream, so graphs captured on
-   one stream must not replay at the same time), the others run direct. */
+   stream is being captured, that accumulates few triangles, or that cannot have
+   one, works in the caller's table.  A captured marker call holds none either:
+   linear, non-accumulating ones on G % 32 == 0 work in the caller's table with
+   1 MB of the graph's own, the others have a table of the graph's own besides
+   (while a device's graphs have an eighth of its memory at most; they run direct
+   beyond, which is much slower for coarse meshes).  What a graph had goes to a
+   later one, or is freed by vox_release_scratch; so keep a graph that an
+   executable was updated from (hipGraphExecUpdate) while that is used.  The
+   region, slab and tile algorithms' captured calls hold their stream's
+   workspaces: graphs of theirs that were captured on one stream must not replay
+   at the same time. */
 #define VOX_FLAG_ALGO_DIRECT 0x2u /* one triangle per lane, global atomics per word */
 #define VOX_FLAG_ALGO_TILE 0x4u   /* triangles binned to output tiles; one workgroup
                                     builds each tile in LDS and writes it once */
@@ -174,9 +180,9 @@ vox_status vox_solid(const vox_info* info, const float* d_tris, uint32_t* d_tabl
                      unsigned flags, uint64_t* d_offrow, void* stream);
 
 /* Frees the scratch tables and spill records that the library keeps for the
-   streams of the current device (after waiting for the device); streams with a
-   call being queued at the moment keep theirs.  The next call on a stream
-   allocates anew. */
+   streams of the current device and what graphs that are gone had (after waiting
+   for the device); streams with a call being queued at the moment keep theirs.
+   The next call on a stream allocates anew. */
 vox_status vox_release_scratch(void);
 
 /* vox_solid without any device allocation.  It has no counterpart in the
