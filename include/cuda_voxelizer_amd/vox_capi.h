@@ -65,8 +65,9 @@ typedef enum vox_status {
                                     others rewrite whole words: order them. */
 /* Algorithm selection (at most one; default: the library's choice per grid,
    layout and mode -- chunk for surface; for solid, direct when the mesh has at
-   least 4 G^2 triangles at G <= 64, or G^2 at G <= 128 with G % 32 != 0, marker
-   otherwise).  All algorithms give identical tables.  Per device and stream the
+   least 4 G^2 triangles at G <= 64, or G^2 at G <= 128 with G % 32 != 0, tile
+   when it has G^2/24 to G^2/4 and the layout is linear, without accumulation, at
+   G > 1184 with G % 32 == 0 and G % 128 != 0, marker otherwise).  All algorithms give identical tables.  Per device and stream the
    library keeps scratch tables of up to G^3/8 bytes (rows rounded up to words)
    for linear surfaces up to 2048^3 and for solids: of a device's streams
    together at most an eighth of its memory (or one stream's table), until
@@ -220,12 +221,12 @@ vox_status vox_pack_triangles(const float* d_vertices, uint64_t n_vertices, cons
    d_tris of each output triangle.  Every voxelization of d_out, at any grid,
    layout and algorithm, gives the same table as of d_tris; the chunk
    algorithm merges more of its words in LDS and issues fewer atomics (1024^3
-   torus of 1 M triangles 0.083 vs 0.107 ms per call, an icosphere whose faces
-   interleave 0.126 vs 0.323 ms; the sort of the torus takes 0.036 ms).  It
+   torus of 1 M triangles 0.072 vs 0.076 ms per call, an icosphere whose faces
+   interleave 0.088 vs 0.198 ms; the sort of the torus takes 0.036 ms).  It
    pays for surfaces of small triangles stored out of spatial order; it does
    not for soups of large overlapping triangles, whose sorted chunks pile
-   their bits onto the same words (random soups: 1.9x to 3.4x slower).  Out of place: d_out and d_perm must not
-   overlap d_tris or each other.  The order within a brick is unspecified.
+   their bits onto the same words (random soups: 1.5x to 1.7x the time on
+   average).  Out of place: d_out and d_perm must not overlap d_tris or each other.  The order within a brick is unspecified.
    The library keeps per-stream counts and keys (4 bytes per triangle and up
    to 2 MiB), allocated at the first call or when a larger one comes. */
 vox_status vox_sort_triangles(const vox_info* info, const float* d_tris, float* d_out, uint32_t* d_perm,
