@@ -520,6 +520,10 @@ vox_status vox_batch_launch(vox_batch* b, void* stream) {
             e = hipStreamWaitEvent(st, b->done, 0);
         } else {
             e = wait_for_device();
+            if (e == hipErrorOutOfMemory) {  // it has none to free
+                (void)hipGetLastError();
+                e = hipDeviceSynchronize();
+            }
             if (e == hipSuccess) e = hipEventCreateWithFlags(&b->done, hipEventDisableTiming);
         }
     }
@@ -530,7 +534,7 @@ vox_status vox_batch_launch(vox_batch* b, void* stream) {
         b->scratch_dirty = b->sws && e != hipSuccess;
         b->last = key;
         b->launched = true;
-        if (b->done && hipEventRecord(b->done, st) != hipSuccess) (void)wait_for_device();
+        if (b->done && hipEventRecord(b->done, st) != hipSuccess) (void)hipDeviceSynchronize();
     }
     if (e != hipSuccess) return hip_fail(e, "batch launch");
     return VOX_OK;

@@ -45,7 +45,7 @@ struct RelaxedCapture {
 };
 
 // Waits for all work of the device that has been queued, as hipFree does; unlike
-// hipDeviceSynchronize it leaves other threads' captures valid.
+// hipDeviceSynchronize it leaves other threads' captures valid.  It needs 256 bytes.
 hipError_t wait_for_device();
 
 // Device memory for the graph into which calls on `stream` are being recorded, its
